@@ -9,7 +9,7 @@ all cells), replayed from a hipGraph.  value = interior zones x steps / time.
 
 Prints one JSON line.  Extra objects:
   roofline      dominant kernel (largest measured time per step; the three
-                direction instantiations of the face flux kernel k_flux count
+                directions of the face flux kernel k_flux, timed apart, count
                 as one kernel, averaged per launch, HIP events on its launch
                 stream).  Its bound follows from its algorithmic intensity
                 (operation count of the oracle per face over the algorithmic
@@ -53,7 +53,8 @@ FP64_PEAK_TFLOPS = 78.6
 #  c2p    : reads 7 cons + 3 face B + C2P_ERR, writes 12 prims + BDIV,
 #           C2P_DENS_ERR, C2P_ERR and rewrites <= 7 cons                -> 264 B
 ALG_BYTES = {"flux": 168, "emf": 216, "update": 456, "c2p": 264, "ghost": 0, "ghost_faces": 0}
-# timer families of one kernel function (k_flux<EOS, REC, FLAT, D>, one launch per direction)
+# timer families of one kernel function (k_flux<EOS, REC, FLAT>; while the families are timed, one launch per
+# direction, otherwise the three in one)
 KERNEL_FAMILIES = {"flux": ("flux_x", "flux_y", "flux_z")}
 # Whole-step algorithmic bytes per zone-update (flat metric; RHS 3x(38..48
 # reads + 10 writes) + c2p 3x) -- 1552 B.

@@ -41,6 +41,8 @@ struct FForest {
     int n[3], ng, N[3];    // interior cells, ghosts, padded extents per block
     int64_t ncell;         // padded cells per block
     int64_t nface[3];      // faces per block per direction
+    int sp, so;            // layout of the context's face and edge arrays (DevGrid)
+    int64_t ns;
     int64_t nq;            // blocks
     const int32_t* cmap;   // per coarse block: q >= 0 leaf, or -(1 + q of child 0)
     const int4* blk;       // per block: level, coordinates at that level
@@ -507,13 +509,12 @@ __global__ __launch_bounds__(256) void k_amr_faces_mid(const int2* __restrict__ 
 // (entry, var); blockIdx.y is the var.
 struct RefluxFace { int64_t dst, src; int32_t s0, s1, d, pad; };
 __global__ __launch_bounds__(256) void k_reflux_flux(const RefluxFace* __restrict__ ent, int n, double* f0, double* f1,
-                                                     double* f2, int64_t n0, int64_t n1, int64_t n2) {
+                                                     double* f2, int64_t nf) {
     const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= n) return;
     const RefluxFace r = ent[e];
     const int v = (int)blockIdx.y;
     double* f = r.d == 0 ? f0 : (r.d == 1 ? f1 : f2);
-    const int64_t nf = r.d == 0 ? n0 : (r.d == 1 ? n1 : n2);
     const double* s = f + r.src + v * nf;
     const double sum = ((s[0] + s[r.s1]) + s[r.s0]) + s[r.s0 + r.s1];
     f[r.dst + v * nf] = 0.25 * sum;
@@ -559,18 +560,18 @@ inline void forest_source(const FForest& F, int q, int fd, const int loc[3], int
 // leaf's surface that a fine cell touches.
 inline void forest_reflux(const FForest& F, std::vector<RefluxFace>& rf, std::vector<RefluxEdge>& re) {
     const int ng = F.ng;
-    struct { int n[3], N[3]; int64_t nface[3], nedge; } G;
-    for (int d = 0; d < 3; ++d) { G.n[d] = F.n[d]; G.N[d] = F.N[d]; G.nface[d] = F.nface[d]; }
-    G.nedge = (int64_t)(F.N[0] + 1) * (F.N[1] + 1) * (F.N[2] + 1);
+    struct { int n[3]; } G;
+    for (int d = 0; d < 3; ++d) G.n[d] = F.n[d];
     const int64_t nq = F.nq;
-    auto eix = [&](int i, int j, int k) { return i + (int64_t)(G.N[0] + 1) * (j + (int64_t)(G.N[1] + 1) * k); };
+    // element (i, j, k) of the context's face and edge arrays, and their strides
+    auto six = [&](int i, int j, int k) { return F.so + i + (int64_t)F.sp * (j + (int64_t)(F.N[1] + 1) * k); };
+    const int64_t st[3] = {1, F.sp, (int64_t)F.sp * (F.N[1] + 1)};
     for (int64_t q = 0; q < nq; ++q) {
         const int4 b = F.blk[q];
         if (b.x != 0) continue;
         const int cr[3] = {b.y, b.z, b.w};
         for (int d = 0; d < 3; ++d) {
             const int t0 = d == 0 ? 1 : 0, t1 = d == 2 ? 1 : 2;
-            const int64_t sf[3] = {1, G.N[0] + (d == 0), (int64_t)(G.N[0] + (d == 0)) * (G.N[1] + (d == 1))};
             for (int side = 0; side < 2; ++side) {
                 int cb[3] = {cr[0], cr[1], cr[2]};
                 cb[d] += side ? 1 : -1;
@@ -588,14 +589,13 @@ inline void forest_reflux(const FForest& F, std::vector<RefluxFace>& rf, std::ve
                         lc[d] = side ? G.n[d] + ng : ng; lc[t0] = ng + aa; lc[t1] = ng + bb;
                         lf[d] = side ? ng : G.n[d] + ng; lf[t0] = ng + (2 * aa) % G.n[t0]; lf[t1] = ng + (2 * bb) % G.n[t1];
                         RefluxFace r;
-                        r.dst = q * gm::NHRSC * G.nface[d] + ff_fidx(F, d, lc[0], lc[1], lc[2]);
-                        r.src = (int64_t)(c0 + ch) * gm::NHRSC * G.nface[d] + ff_fidx(F, d, lf[0], lf[1], lf[2]);
-                        r.s0 = (int32_t)sf[t0]; r.s1 = (int32_t)sf[t1]; r.d = d; r.pad = 0;
+                        r.dst = q * gm::NHRSC * F.ns + six(lc[0], lc[1], lc[2]);
+                        r.src = (int64_t)(c0 + ch) * gm::NHRSC * F.ns + six(lf[0], lf[1], lf[2]);
+                        r.s0 = (int32_t)st[t0]; r.s1 = (int32_t)st[t1]; r.d = d; r.pad = 0;
                         rf.push_back(r);
                     }
             }
             // edges along d on the block surface
-            const int64_t se[3] = {1, G.N[0] + 1, (int64_t)(G.N[0] + 1) * (G.N[1] + 1)};
             for (int bb = ng; bb <= G.n[t1] + ng; ++bb)
                 for (int aa = ng; aa <= G.n[t0] + ng; ++aa) {
                     if (!(aa == ng || aa == G.n[t0] + ng || bb == ng || bb == G.n[t1] + ng)) continue;
@@ -621,9 +621,9 @@ inline void forest_reflux(const FForest& F, std::vector<RefluxFace>& rf, std::ve
                         if (qf < 0) continue;
                         int lc[3]; lc[d] = ic; lc[t0] = aa; lc[t1] = bb;
                         RefluxEdge r;
-                        r.dst = (q * 3 + d) * G.nedge + eix(lc[0], lc[1], lc[2]);
-                        r.src = ((int64_t)qf * 3 + d) * G.nedge + eix(lf[0], lf[1], lf[2]);
-                        r.stride = (int32_t)se[d]; r.pad = 0;
+                        r.dst = (q * 3 + d) * F.ns + six(lc[0], lc[1], lc[2]);
+                        r.src = ((int64_t)qf * 3 + d) * F.ns + six(lf[0], lf[1], lf[2]);
+                        r.stride = (int32_t)st[d]; r.pad = 0;
                         re.push_back(r);
                     }
                 }

@@ -1,9 +1,10 @@
 // grmhd.hip -- gfx950 kernels and C ABI for the Cowling GRMHD RHS + con2prim.
 //
 // Kernel families (all FP64):
-//   k_flux<D>      one thread per face of direction D: 10-variable
-//                  reconstruction, face metric, EOS, HLLE/LLF fluxes, vbar/Eface
-//                  (reference: evolve.cpp:813-1068, grmhd.hh:551-970)
+//   k_flux         (flux.hh) one thread per face, the three directions in one
+//                  launch: reconstruction, face metric, EOS, HLLE/LLF fluxes,
+//                  vbar/Eface (reference: evolve.cpp:813-1068,
+//                  grmhd.hh:551-970)
 //   k_emf_uct      one thread per edge triple: UCT edge EMFs (evolve.cpp:1130-1340)
 //   k_emf_gs       Gardiner-Stone edge EMFs (grmhd_helpers.hh:492-627)
 //   k_update       fused RK linear combination + geometric sources + flux
@@ -64,6 +65,17 @@ struct DevGrid {
     int64_t nface[3];  // faces per block per direction
     int64_t nedge;     // edges per block per component
     int64_t nq;
+    // Layout of the context's own face and edge arrays (fluxes, UCT/GS face
+    // values, edge EMFs), the same for every direction: rows of pitch sp
+    // doubles, N[1] + 1 rows to a plane, element i of a row at so + i.  sp
+    // and so put the first interior element of every row on a 128-byte
+    // boundary: a row of 16 faces is then one whole line, written and read
+    // with one request.  (With the rows of the boundary's arrays, 22 doubles
+    // from byte 24 on, each row shares both its lines with the next rows, and
+    // a kernel that walks along y writes every line twice, in parts: y faces
+    // 314 us against 258 us, z 277 against 224, 512 blocks of 16^3.)
+    int sp, so;
+    int64_t ns;        // doubles per block per component
 };
 struct DevInst { int nb[3]; int64_t q0; int bc[6]; double idx[3]; double x0[3]; };
 
@@ -107,6 +119,11 @@ GHD int64_t eidx(const DevGrid& G, int i, int j, int k) {
     return i + (int64_t)(G.N[0] + 1) * (j + (int64_t)(G.N[1] + 1) * k);
 }
 
+// Element (i, j, k) of a component of the context's face and edge arrays.
+GHD int64_t sidx(const DevGrid& G, int i, int j, int k) {
+    return G.so + i + (int64_t)G.sp * (j + (int64_t)(G.N[1] + 1) * k);
+}
+
 // Position of this workgroup in a 1-D grid of wpb workgroups per block times
 // the number of blocks.  The hardware deals workgroups to the 8 XCDs round
 // robin; the remap hands each XCD a contiguous range of logical workgroups,
@@ -115,13 +132,13 @@ GHD int64_t eidx(const DevGrid& G, int i, int j, int k) {
 // (A 1-D grid has fewer than 2^32 workgroups, so 32-bit unsigned
 // arithmetic: one short scalar division instead of a 64-bit one.)
 struct WgPos { int tile; int64_t q; };
-__device__ __forceinline__ WgPos wg_pos(int wpb) {
-    const uint32_t p = blockIdx.x, n = gridDim.x;
+__device__ __forceinline__ WgPos wg_pos_in(uint32_t p, uint32_t n, int wpb) {
     const uint32_t x = p & 7u, i = p >> 3, base = n >> 3, rem = n & 7u;
     const uint32_t L = x * base + (x < rem ? x : rem) + i;
     const uint32_t w = (uint32_t)wpb, q = L / w;
     return WgPos{(int)(L - q * w), (int64_t)q};
 }
+__device__ __forceinline__ WgPos wg_pos(int wpb) { return wg_pos_in(blockIdx.x, gridDim.x, wpb); }
 // x = q d + r for x >= 0, d > 0 (unsigned: no sign fix-ups)
 GHD void udivmod(int x, int d, int& q, int& r) {
     const uint32_t uq = (uint32_t)x / (uint32_t)d;
@@ -167,347 +184,7 @@ GHD void face_metric(const double* __restrict__ M, int64_t nc, int64_t c0, int64
 // nface[D] per block.
 constexpr int FMC = 13;
 
-// ---------------------------------------------------------------------------
-// Face flux kernel
-// ---------------------------------------------------------------------------
-// Minimum waves per SIMD the compiler must fit (VGPR budget); unset: its own choice.
-#ifdef GRMHD_FLUX_MINW
-#define GRMHD_FLUX_BOUNDS __launch_bounds__(256, GRMHD_FLUX_MINW)
-#else
-#define GRMHD_FLUX_BOUNDS __launch_bounds__(256)
-#endif
-// PF: every stencil value of the face is loaded before the first
-// reconstruction (54 loads in flight per lane instead of 6; about 150 VGPRs,
-// 3 waves per SIMD instead of 4): a tuning choice per direction
-// (grmhd_tuning.flux_prefetch), results bit-identical.
-template <typename EOS, int REC, bool FLAT, int D, bool PF = false>
-__global__ GRMHD_FLUX_BOUNDS void k_flux(DevGrid G, EOS eos, Opts o, const double* __restrict__ aux,
-                                              const double* __restrict__ mstate, int mnv,
-                                              const double* __restrict__ Bd, double* __restrict__ flux,
-                                              double* __restrict__ vbar, int wpb,
-                                              const uint8_t* __restrict__ only,
-                                              const uint8_t* __restrict__ ring_own,
-                                              const int32_t* __restrict__ push_nbr,
-                                              const double* __restrict__ fmc) {
-    // wpb workgroups per block (see wg_pos).  UCT: the first
-    // (n_D+1) n_T0 n_T1 threads take the faces whose transverse indices are
-    // both interior (full fluxes), the next ones the faces with exactly one
-    // transverse index in the ghost layers ("ring": they feed only the
-    // transverse reconstructions of the edge EMFs: vbar and wave speeds);
-    // faces with both transverse indices in the ghost layers are never read
-    // and get no thread.  GS reads fluxes and face EMFs one layer into the
-    // transverse ghosts, so it takes every face (normal [ng, n+ng],
-    // transverse [0, N)).  ring_own (per block, bit 2 d + side for the six
-    // block faces): when given, a ring face is computed only if its ghost
-    // side lies beyond an outflow face of the instance; the others are
-    // interior faces of the neighbouring block, whose face threads write
-    // them through push_nbr (the neighbour across each of the six block
-    // faces; with periodicity per dimension the relation is symmetric).
-    const WgPos wp = wg_pos(wpb);
-    const int64_t q = wp.q;
-    const int e = wp.tile * (int)blockDim.x + (int)threadIdx.x;
-    int i, j, k;
-    bool ring = false;
-    {
-        const int ng = G.ng, Rn = G.n[D] + 1;
-        constexpr int T0 = D == 0 ? 1 : 0, T1 = D == 2 ? 1 : 2;
-        const int n0 = G.n[T0], n1 = G.n[T1];
-        int a = 0, b = 0, c = 0;   // (normal, t0, t1)
-        if (o.emf != 0) {
-            // GS: every face; FOFC widens the normal range by one face on each side
-            const int N0 = G.N[T0], N1 = G.N[T1];
-            const int Rg = Rn + 2 * o.fofc;
-            if (e >= Rg * N0 * N1) return;
-            int r;
-            if (D == 0) { udivmod(e, Rg, r, a); udivmod(r, N0, c, b); }
-            else if (D == 1) { udivmod(e, N0, r, b); udivmod(r, Rg, c, a); }
-            else { udivmod(e, N0, r, b); udivmod(r, N1, a, c); }
-            a -= o.fofc;
-        } else {
-            const int nint = Rn * n0 * n1, g2 = 2 * ng;
-            const int nA = Rn * g2 * n1, nB = Rn * n0 * g2;
-            auto ghost = [&](int g, int nn) { return g < ng ? g : nn + g; };
-            int r;
-            if (e < nint) {
-                if (D == 0) { udivmod(e, Rn, r, a); udivmod(r, n0, c, b); }
-                else if (D == 1) { udivmod(e, n0, r, b); udivmod(r, Rn, c, a); }
-                else { udivmod(e, n0, r, b); udivmod(r, n1, a, c); }
-                b += ng; c += ng;
-            } else if (e < nint + nA) {          // t0 ghost, t1 interior
-                const int x = e - nint;
-                ring = true;
-                int gl;
-                if (D == 0) { udivmod(x, Rn, r, a); udivmod(r, g2, c, gl); }
-                else if (D == 1) { udivmod(x, g2, r, gl); udivmod(r, Rn, c, a); }
-                else { udivmod(x, g2, r, gl); udivmod(r, n1, a, c); }
-                c += ng;
-                if (ring_own && !((ring_own[q] >> (2 * T0 + (gl >= ng))) & 1)) return;
-                b = ghost(gl, n0);
-            } else if (e < nint + nA + nB) {     // t0 interior, t1 ghost
-                const int x = e - nint - nA;
-                ring = true;
-                int gl;
-                if (D == 0) { udivmod(x, Rn, r, a); udivmod(r, n0, gl, b); }
-                else if (D == 1) { udivmod(x, n0, r, b); udivmod(r, Rn, gl, a); }
-                else { udivmod(x, n0, r, b); udivmod(r, g2, a, gl); }
-                b += ng;
-                if (ring_own && !((ring_own[q] >> (2 * T1 + (gl >= ng))) & 1)) return;
-                c = ghost(gl, n1);
-            } else {
-                return;
-            }
-        }
-        a += ng;
-        if (D == 0) { i = a; j = b; k = c; }
-        else if (D == 1) { i = b; j = a; k = c; }
-        else { i = b; j = c; k = a; }
-        // FOFC correction pass: only the tagged faces of the normal range
-        // [ng, n+ng] (evolve.cpp:646-702)
-        if (only && (a < ng || a > ng + G.n[D] || !only[q * G.nface[D] + fidx<D>(G, i, j, k)])) return;
-    }
-    const int64_t nc = G.ncell;
-    const int64_t c0 = cidx(G, i, j, k);
-    const int64_t st = D == 0 ? 1 : (D == 1 ? G.N[0] : (int64_t)G.N[0] * G.N[1]);
-    const double* A = aux + q * NAUX * nc;
-    // flat metric: the six stencil cells along D (var 0).  With push_nbr (the
-    // second and third RK stages, whose gathers leave the face slabs alone)
-    // a full face takes a cell beyond a block face from the neighbouring
-    // block's interior (normal index shifted by one block extent); beyond an
-    // outflow face (no neighbour) and on ring faces, from its own ghosts,
-    // which run their own c2p or copy one that does.  (The curved kernels,
-    // which never get push_nbr, keep one row pointer per variable: six
-    // pointers cost them 7% on x faces.)
-    const double* Pt[6];
-    if constexpr (FLAT) {
-        const int an = D == 0 ? i : (D == 1 ? j : k), nD = G.n[D];
-        int32_t nl = -1, nh = -1;
-        if (push_nbr && !ring) { nl = push_nbr[q * 6 + 2 * D]; nh = push_nbr[q * 6 + 2 * D + 1]; }
-#pragma unroll
-        for (int t = 0; t < 6; ++t) {
-            const int ap = an + t - 3;
-            int64_t qb = q;
-            int sh = 0;
-            if (ap < G.ng && nl >= 0) { qb = nl; sh = nD; }
-            else if (ap >= nD + G.ng && nh >= 0) { qb = nh; sh = -nD; }
-            Pt[t] = aux + qb * NAUX * nc + c0 + (int64_t)(t - 3 + sh) * st;
-        }
-    }
-
-    Met mf;
-    bool excise_override = false;
-    if constexpr (FLAT) {
-        mf.flat();
-    } else if (fmc) {
-        // the face-metric cache: only the inverse component this direction
-        // uses (cmcp, the LLF speed limit) is kept
-        const int64_t nfd = G.nface[D];
-        const double* FM = fmc + q * FMC * nfd + fidx<D>(G, i, j, k);
-        for (int a = 0; a < 6; ++a) { mf.g[a] = FM[a * nfd]; mf.gi[a] = 0.0; }
-        mf.gi[D == 0 ? 0 : (D == 1 ? 3 : 5)] = FM[6 * nfd];
-        for (int a = 0; a < 3; ++a) mf.beta[a] = FM[(7 + a) * nfd];
-        mf.alp = FM[10 * nfd];
-        mf.sqrtg = FM[11 * nfd];
-        excise_override = FM[12 * nfd] != 0.0;
-    } else {
-        face_metric(mstate + q * (int64_t)mnv * nc, nc, c0, st, o.ex.alp_ex, mf, excise_override);
-    }
-    // reconstruction of RHO Z(3) YE THERMO ENT B(3)
-    const int th_aux = o.thermo ? PRESS_ : TEMP_;
-    const int ridx[10] = {RHO_, ZVECX_, ZVECY_, ZVECZ_, YE_, th_aux, ENTROPY_, BX_, BY_, BZ_};
-    const int rloc[10] = {RHOL, ZXL, ZYL, ZZL, YEL, o.thermo ? PRESSL : TEMPL, ENTL, BXL, BYL, BZL};
-    double pL[NPRIM], pR[NPRIM];
-    if constexpr (PF) {
-        double us[10][6];
-#pragma unroll
-        for (int v = 0; v < 10; ++v) {
-            if (v == 7 + D) continue;
-            if constexpr (FLAT) {
-                const int64_t ov = ridx[v] * nc;
-#pragma unroll
-                for (int t = 0; t < 6; ++t) us[v][t] = Pt[t][ov];
-            } else {
-                const double* P = A + ridx[v] * nc + c0;
-#pragma unroll
-                for (int t = 0; t < 6; ++t) us[v][t] = P[(t - 3) * st];
-            }
-        }
-#pragma unroll
-        for (int v = 0; v < 10; ++v) {
-            if (v == 7 + D || (ring && (v == 4 || v == 6))) { pL[rloc[v]] = 0.0; pR[rloc[v]] = 0.0; continue; }
-            double uL, uR;
-            if (excise_override) { uL = us[v][2]; uR = us[v][3]; }
-            else recon<REC>(us[v][0], us[v][1], us[v][2], us[v][3], us[v][4], us[v][5], uL, uR);
-            pL[rloc[v]] = uL; pR[rloc[v]] = uR;
-        }
-    } else {
-#pragma unroll
-        for (int v = 0; v < 10; ++v) {
-            // Work whose result is never read: the normal B component is replaced
-            // by the face value below, and a ring face (UCT velocities and wave
-            // speeds only) reads neither Ye nor the entropy.
-            if (v == 7 + D || (ring && (v == 4 || v == 6))) { pL[rloc[v]] = 0.0; pR[rloc[v]] = 0.0; continue; }
-            double uL, uR;
-            if constexpr (FLAT) {
-                const int64_t ov = ridx[v] * nc;
-                recon<REC>(Pt[0][ov], Pt[1][ov], Pt[2][ov], Pt[3][ov], Pt[4][ov], Pt[5][ov], uL, uR);
-            } else {
-                const double* P = A + ridx[v] * nc + c0;
-                if (excise_override) { uL = P[-st]; uR = P[0]; }
-                else recon<REC>(P[-3 * st], P[-2 * st], P[-st], P[0], P[st], P[2 * st], uL, uR);
-            }
-            pL[rloc[v]] = uL; pR[rloc[v]] = uR;
-        }
-    }
-    double Bn = Bd[q * G.nface[D] + fidx<D>(G, i, j, k)] / mf.sqrtg;
-    pL[BXL + D] = Bn; pR[BXL + D] = Bn;
-    unsigned ee = 0;
-    if (o.thermo) {
-        double h, s;
-        pL[EPSL] = eos.eps_from_press(h, pL[CS2L], pL[TEMPL], s, pL[PRESSL], pL[RHOL], ee);
-        pR[EPSL] = eos.eps_from_press(h, pR[CS2L], pR[TEMPL], s, pR[PRESSL], pR[RHOL], ee);
-    } else {
-        pL[PRESSL] = eos.press_from_temp(pL[EPSL], pL[CS2L], pL[TEMPL], pL[RHOL], ee);
-        pR[PRESSL] = eos.press_from_temp(pR[EPSL], pR[CS2L], pR[TEMPL], pR[RHOL], ee);
-    }
-    // compute_mhd_fluxes (grmhd.hh:774-970)
-    const double *zl = &pL[ZXL], *zr = &pR[ZXL], *Bl = &pL[BXL], *Br = &pR[BXL];
-    double wl = lorentz<FLAT>(mf.g, zl), wr = lorentz<FLAT>(mf.g, zr);
-    double bl[4], br[4], b2l, b2r;
-    smallb<FLAT>(mf, Bl, zl, wl, bl, b2l);
-    smallb<FLAT>(mf, Br, zr, wr, br, b2r);
-    double vtl[3], vtr[3];
-    vtilde(mf, zl, wl, vtl);
-    vtilde(mf, zr, wr, vtr);
-    double cml, cpl, cmr, cpr, cmin, cmax;
-    cmcp<FLAT>(mf, pL[RHOL], pL[PRESSL], pL[EPSL], pL[CS2L], wl, b2l, vtl, D, cml, cpl);
-    cmcp<FLAT>(mf, pR[RHOL], pR[PRESSL], pR[EPSL], pR[CS2L], wr, b2r, vtr, D, cmr, cpr);
-    if (o.riemann == 1) {
-        cmax = fmax(fmax(fabs(cml), fabs(cmr)), fmax(fabs(cpl), fabs(cpr)));
-        if (fmin(pL[RHOL], pR[RHOL]) < o.c_limit) {
-            double gdd = D == 0 ? mf.gi[0] : (D == 1 ? mf.gi[3] : mf.gi[5]);
-            cmax = fmax(cmax, mf.alp * sqrt(gdd) + fabs(mf.beta[D]));
-        }
-        cmin = cmax;
-    } else {
-        cmin = -fmin(0., fmin(cml, cmr));
-        cmax = fmax(0., fmax(cpl, cpr));
-    }
-    if (cmin < 1e-12 && cmax < 1e-12) { cmin = 1; cmax = 1; }
-    const double ihll = 1.0 / (cmax + cmin);   // shared by the HLL fluxes of this face
-    const int64_t fo = fidx<D>(G, i, j, k);
-    const int64_t nf = G.nface[D];
-    double* V = vbar + q * 4 * nf + fo;
-    constexpr int J0 = D == 0 ? 1 : 0, J1 = D == 2 ? 1 : 2;
-    double vb0 = 0.0, vb1 = 0.0;
-    if (o.emf == 0) {  // UCT: HLL-averaged transverse vtilde + wave speeds, slots strided by nf
-        vb0 = hll_r(vtl[J0], vtr[J0], 0, 0, cmin, cmax, ihll);
-        vb1 = hll_r(vtl[J1], vtr[J1], 0, 0, cmin, cmax, ihll);
-        V[0] = vb0; V[nf] = vb1;
-        V[2 * nf] = cmin; V[3 * nf] = cmax;
-        if (ring) return;
-    }
-    double Dl, taul, Sl[3], Esl, Dr, taur, Sr[3], Esr;
-    conserved<FLAT>(mf, pL[RHOL], pL[PRESSL], pL[EPSL], zl, pL[ENTL], wl, b2l, bl, Dl, taul, Sl, Esl);
-    conserved<FLAT>(mf, pR[RHOL], pR[PRESSL], pR[EPSL], zr, pR[ENTL], wr, b2r, br, Dr, taur, Sr, Esr);
-    // fluxes along D (grmhd_subexpressions.hh:97-156)
-    double bsh[3]; lower3(mf.g, mf.beta[0], mf.beta[1], mf.beta[2], bsh);
-    double ia2 = 1. / (mf.alp * mf.alp);
-    double Fl[7], Fr[7];
-    {
-        double rhoh = b2l + pL[EPSL] * pL[RHOL] + pL[PRESSL] + pL[RHOL];
-        double ps = 0.5 * b2l + pL[PRESSL];
-        double W2rh = wl * wl * rhoh;
-        double fD = vtl[D] * Dl;
-        Fl[0] = fD;
-        double blo[3]; lower3<FLAT>(mf.g, bl[1], bl[2], bl[3], blo);
-        double vlo[3]; lower3<FLAT>(mf.g, vtl[0], vtl[1], vtl[2], vlo);
-        if constexpr (FLAT) {
-            Fl[4] = W2rh * vtl[D] - bl[0] * bl[1 + D] - fD;
-            const double c = vtl[D] * W2rh;
-            for (int a = 0; a < 3; ++a)
-                Fl[1 + a] = a == D ? -bl[1 + D] * blo[a] + ps + c * vlo[a] : -bl[1 + D] * blo[a] + c * vlo[a];
-        } else {
-            Fl[4] = W2rh * vtl[D] + ps * mf.beta[D] - mf.alp * mf.alp * bl[0] * bl[1 + D] - fD;
-            const double c = vtl[D] * W2rh * ia2;
-            for (int a = 0; a < 3; ++a)
-                Fl[1 + a] = mf.alp * (-bl[1 + D] * (blo[a] + bl[0] * bsh[a]) + (a == D ? ps : 0.0) + c * (vlo[a] + bsh[a]));
-        }
-        Fl[6] = vtl[D] * Esl;
-        Fl[5] = pL[YEL] * fD;
-    }
-    {
-        double rhoh = b2r + pR[EPSL] * pR[RHOL] + pR[PRESSL] + pR[RHOL];
-        double ps = 0.5 * b2r + pR[PRESSL];
-        double W2rh = wr * wr * rhoh;
-        double fD = vtr[D] * Dr;
-        Fr[0] = fD;
-        double blo[3]; lower3<FLAT>(mf.g, br[1], br[2], br[3], blo);
-        double vlo[3]; lower3<FLAT>(mf.g, vtr[0], vtr[1], vtr[2], vlo);
-        if constexpr (FLAT) {
-            Fr[4] = W2rh * vtr[D] - br[0] * br[1 + D] - fD;
-            const double c = vtr[D] * W2rh;
-            for (int a = 0; a < 3; ++a)
-                Fr[1 + a] = a == D ? -br[1 + D] * blo[a] + ps + c * vlo[a] : -br[1 + D] * blo[a] + c * vlo[a];
-        } else {
-            Fr[4] = W2rh * vtr[D] + ps * mf.beta[D] - mf.alp * mf.alp * br[0] * br[1 + D] - fD;
-            const double c = vtr[D] * W2rh * ia2;
-            for (int a = 0; a < 3; ++a)
-                Fr[1 + a] = mf.alp * (-br[1 + D] * (blo[a] + br[0] * bsh[a]) + (a == D ? ps : 0.0) + c * (vlo[a] + bsh[a]));
-        }
-        Fr[6] = vtr[D] * Esr;
-        Fr[5] = pR[YEL] * fD;
-    }
-    double* F = flux + q * NHRSC * nf + fo;
-    const double sg = mf.sqrtg;
-    F[DENS_ * nf] = sg * hll_r(Fl[0], Fr[0], Dl, Dr, cmin, cmax, ihll);
-    F[ENTROPYSTAR_ * nf] = sg * hll_r(Fl[6], Fr[6], Esl, Esr, cmin, cmax, ihll);
-    F[TAU_ * nf] = sg * hll_r(Fl[4], Fr[4], taul, taur, cmin, cmax, ihll);
-    F[SX_ * nf] = sg * hll_r(Fl[1], Fr[1], Sl[0], Sr[0], cmin, cmax, ihll);
-    F[SY_ * nf] = sg * hll_r(Fl[2], Fr[2], Sl[1], Sr[1], cmin, cmax, ihll);
-    F[SZ_ * nf] = sg * hll_r(Fl[3], Fr[3], Sl[2], Sr[2], cmin, cmax, ihll);
-    F[YESTAR_ * nf] = sg * hll_r(Fl[5], Fr[5], pL[YEL] * Dl, pR[YEL] * Dr, cmin, cmax, ihll);
-    if (o.emf == 1) {  // GS face EMFs (grmhd.hh:937-969)
-        if (D == 0) {
-            double a = -Bl[0] * vtl[2] + Bl[2] * vtl[0], b = -Br[0] * vtr[2] + Br[2] * vtr[0];
-            V[0] = sg * hll_r(a, b, Bl[2], Br[2], cmin, cmax, ihll);
-            a = -Bl[0] * vtl[1] + Bl[1] * vtl[0]; b = -Br[0] * vtr[1] + Br[1] * vtr[0];
-            V[nf] = -sg * hll_r(a, b, Bl[1], Br[1], cmin, cmax, ihll);
-        } else if (D == 1) {
-            double a = -Bl[1] * vtl[2] + Bl[2] * vtl[1], b = -Br[1] * vtr[2] + Br[2] * vtr[1];
-            V[0] = -sg * hll_r(a, b, Bl[2], Br[2], cmin, cmax, ihll);
-            a = Bl[0] * vtl[1] - Bl[1] * vtl[0]; b = Br[0] * vtr[1] - Br[1] * vtr[0];
-            V[nf] = sg * hll_r(a, b, Bl[0], Br[0], cmin, cmax, ihll);
-        } else {
-            double a = Bl[1] * vtl[2] - Bl[2] * vtl[1], b = Br[1] * vtr[2] - Br[2] * vtr[1];
-            V[0] = sg * hll_r(a, b, Bl[1], Br[1], cmin, cmax, ihll);
-            a = Bl[0] * vtl[2] - Bl[2] * vtl[0]; b = Br[0] * vtr[2] - Br[2] * vtr[0];
-            V[nf] = -sg * hll_r(a, b, Bl[0], Br[0], cmin, cmax, ihll);
-        }
-    }
-    if (push_nbr) {
-        // stages with shared ring faces: this interior face is a ring face of the
-        // neighbour across each block face within ngz of it (transverse
-        // index shifted by one block extent)
-        const int ng = G.ng;
-        constexpr int T0 = D == 0 ? 1 : 0, T1 = D == 2 ? 1 : 2;
-        const int loc[3] = {i, j, k};
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int td = t == 0 ? T0 : T1;
-            const int nt = G.n[td], it = loc[td] - ng;
-#pragma unroll
-            for (int hi = 0; hi < 2; ++hi) {
-                if (hi ? it < nt - ng : it >= ng) continue;
-                const int32_t qt = push_nbr[q * 6 + 2 * td + hi];
-                if (qt < 0) continue;
-                int l2[3] = {loc[0], loc[1], loc[2]};
-                l2[td] = hi ? it - nt + ng : it + nt + ng;
-                double* T = vbar + (int64_t)qt * 4 * nf + fidx<D>(G, l2[0], l2[1], l2[2]);
-                T[0] = vb0; T[nf] = vb1; T[2 * nf] = cmin; T[3 * nf] = cmax;
-            }
-        }
-    }
-}
+#include "flux.hh"
 
 // ---------------------------------------------------------------------------
 // UCT edge EMFs.  Face arrays: B faces (1 var), vbar (4 vars, stride nf).
@@ -534,51 +211,54 @@ __global__ __launch_bounds__(256) void k_emf_uct(DevGrid G, const double* __rest
     const int i = G.ng + ix0, j = G.ng + jy, k = G.ng + kz;
     const int64_t nfx = G.nface[0], nfy = G.nface[1], nfz = G.nface[2];
     const double* bx = Bx + q * nfx; const double* by = By + q * nfy; const double* bz = Bz + q * nfz;
-    const double* Vx = vx + q * 4 * nfx; const double* Vy = vy + q * 4 * nfy; const double* Vz = vz + q * 4 * nfz;
+    const int64_t ns = G.ns;
+    const double* Vx = vx + q * 4 * ns; const double* Vy = vy + q * 4 * ns; const double* Vz = vz + q * 4 * ns;
     // strides of the face arrays along each axis
     const int64_t sx_x = 1, sx_y = G.N[0] + 1, sx_z = (int64_t)(G.N[0] + 1) * G.N[1];
     const int64_t sy_x = 1, sy_y = G.N[0], sy_z = (int64_t)G.N[0] * (G.N[1] + 1);
     const int64_t sz_x = 1, sz_y = G.N[0], sz_z = (int64_t)G.N[0] * G.N[1];
-    double* E = emf + q * 3 * G.nedge;
-    const int64_t eo = eidx(G, i, j, k);
+    // strides and this site's offset in the context's arrays
+    const int64_t sy = G.sp, sz = (int64_t)G.sp * (G.N[1] + 1);
+    double* E = emf + q * 3 * ns;
+    const int64_t eo = sidx(G, i, j, k);
     if (i < G.n[0] + G.ng) {  // E^x at (i, j-1/2, k-1/2)
         int64_t fy = fidx<1>(G, i, j, k), fz = fidx<2>(G, i, j, k);
         double ByL, ByR, vzL, vzR, BzL, BzR, vyL, vyR;
         rec6<REC>(by + fy, sy_z, ByL, ByR);
-        rec6<REC>(Vy + nfy + fy, sy_z, vzL, vzR);
+        rec6<REC>(Vy + ns + eo, sz, vzL, vzR);
         rec6<REC>(bz + fz, sz_y, BzL, BzR);
-        rec6<REC>(Vz + nfz + fz, sz_y, vyL, vyR);
-        double cmin_y = fmax(Vy[2 * nfy + fy], Vy[2 * nfy + fy - sy_z]);
-        double cmax_y = fmax(Vy[3 * nfy + fy], Vy[3 * nfy + fy - sy_z]);
-        double cmin_z = fmax(Vz[2 * nfz + fz], Vz[2 * nfz + fz - sz_y]);
-        double cmax_z = fmax(Vz[3 * nfz + fz], Vz[3 * nfz + fz - sz_y]);
+        rec6<REC>(Vz + ns + eo, sy, vyL, vyR);
+        double cmin_y = fmax(Vy[2 * ns + eo], Vy[2 * ns + eo - sz]);
+        double cmax_y = fmax(Vy[3 * ns + eo], Vy[3 * ns + eo - sz]);
+        double cmin_z = fmax(Vz[2 * ns + eo], Vz[2 * ns + eo - sy]);
+        double cmax_z = fmax(Vz[3 * ns + eo], Vz[3 * ns + eo - sy]);
         E[eo] = hll(vzL * ByL, vzR * ByR, ByL, ByR, cmin_z, cmax_z) - hll(vyL * BzL, vyR * BzR, BzL, BzR, cmin_y, cmax_y);
     }
     if (j < G.n[1] + G.ng) {  // E^y at (i-1/2, j, k-1/2)
         int64_t fz = fidx<2>(G, i, j, k), fx = fidx<0>(G, i, j, k);
         double BzL, BzR, vxL, vxR, BxL, BxR, vzL, vzR;
         rec6<REC>(bz + fz, sz_x, BzL, BzR);
-        rec6<REC>(Vz + fz, sz_x, vxL, vxR);
+        rec6<REC>(Vz + eo, 1, vxL, vxR);
         rec6<REC>(bx + fx, sx_z, BxL, BxR);
-        rec6<REC>(Vx + nfx + fx, sx_z, vzL, vzR);
-        double cmin_z = fmax(Vz[2 * nfz + fz], Vz[2 * nfz + fz - sz_x]);
-        double cmax_z = fmax(Vz[3 * nfz + fz], Vz[3 * nfz + fz - sz_x]);
-        double cmin_x = fmax(Vx[2 * nfx + fx], Vx[2 * nfx + fx - sx_z]);
-        double cmax_x = fmax(Vx[3 * nfx + fx], Vx[3 * nfx + fx - sx_z]);
-        E[G.nedge + eo] = hll(vxL * BzL, vxR * BzR, BzL, BzR, cmin_x, cmax_x) - hll(vzL * BxL, vzR * BxR, BxL, BxR, cmin_z, cmax_z);
+        rec6<REC>(Vx + ns + eo, sz, vzL, vzR);
+        double cmin_z = fmax(Vz[2 * ns + eo], Vz[2 * ns + eo - 1]);
+        double cmax_z = fmax(Vz[3 * ns + eo], Vz[3 * ns + eo - 1]);
+        double cmin_x = fmax(Vx[2 * ns + eo], Vx[2 * ns + eo - sz]);
+        double cmax_x = fmax(Vx[3 * ns + eo], Vx[3 * ns + eo - sz]);
+        E[ns + eo] = hll(vxL * BzL, vxR * BzR, BzL, BzR, cmin_x, cmax_x) - hll(vzL * BxL, vzR * BxR, BxL, BxR, cmin_z, cmax_z);
     }
     if (k < G.n[2] + G.ng) {  // E^z at (i-1/2, j-1/2, k)
         int64_t fx = fidx<0>(G, i, j, k), fy = fidx<1>(G, i, j, k);
         double BxL, BxR, vyL, vyR, ByL, ByR, vxL, vxR;
         rec6<REC>(bx + fx, sx_y, BxL, BxR);
-        rec6<REC>(Vx + fx, sx_y, vyL, vyR);
+        rec6<REC>(Vx + eo, sy, vyL, vyR);
         rec6<REC>(by + fy, sy_x, ByL, ByR);
-        rec6<REC>(Vy + fy, sy_x, vxL, vxR);
-        double cmin_x = fmax(Vx[2 * nfx + fx], Vx[2 * nfx + fx - sx_y]);
-        double cmax_x = fmax(Vx[3 * nfx + fx], Vx[3 * nfx + fx - sx_y]);
-        double cmin_y = fmax(Vy[2 * nfy + fy], Vy[2 * nfy + fy - sy_x]);
-        double cmax_y = fmax(Vy[3 * nfy + fy], Vy[3 * nfy + fy - sy_x]);
-        E[2 * G.nedge + eo] = hll(vyL * BxL, vyR * BxR, BxL, BxR, cmin_y, cmax_y) - hll(vxL * ByL, vxR * ByR, ByL, ByR, cmin_x, cmax_x);
+        rec6<REC>(Vy + eo, 1, vxL, vxR);
+        double cmin_x = fmax(Vx[2 * ns + eo], Vx[2 * ns + eo - sy]);
+        double cmax_x = fmax(Vx[3 * ns + eo], Vx[3 * ns + eo - sy]);
+        double cmin_y = fmax(Vy[2 * ns + eo], Vy[2 * ns + eo - 1]);
+        double cmax_y = fmax(Vy[3 * ns + eo], Vy[3 * ns + eo - 1]);
+        E[2 * ns + eo] = hll(vyL * BxL, vyR * BxR, BxL, BxR, cmin_y, cmax_y) - hll(vxL * ByL, vxR * ByR, ByL, ByR, cmin_x, cmax_x);
     }
 }
 
@@ -602,21 +282,18 @@ __global__ __launch_bounds__(256) void k_emf_gs(DevGrid G, const double* __restr
     udivmod(r, R0 * R1, kz, rxy);
     udivmod(rxy, R0, jy, ix0);
     const int i = G.ng - wide + ix0, j = G.ng - wide + jy, k = G.ng - wide + kz;
-    const int64_t nfx = G.nface[0], nfy = G.nface[1], nfz = G.nface[2], nc = G.ncell;
+    const int64_t nc = G.ncell;
     auto EF = [&](int d, int c, int ii, int jj, int kk) {
         const double* base = d == 0 ? ef0 : (d == 1 ? ef1 : ef2);
-        int64_t nf = G.nface[d];
-        return base[q * 4 * nf + c * nf + fidx_d(G, d, ii, jj, kk)];
+        return base[(q * 4 + c) * G.ns + sidx(G, ii, jj, kk)];
     };
     auto EC = [&](int c, int ii, int jj, int kk) { return ec[q * 3 * nc + c * nc + cidx(G, ii, jj, kk)]; };
     auto FD = [&](int d, int ii, int jj, int kk) {
         const double* base = d == 0 ? f0 : (d == 1 ? f1 : f2);
-        int64_t nf = G.nface[d];
-        return base[q * NHRSC * nf + DENS_ * nf + fidx_d(G, d, ii, jj, kk)];
+        return base[(q * NHRSC + DENS_) * G.ns + sidx(G, ii, jj, kk)];
     };
-    (void)nfx; (void)nfy; (void)nfz;
-    double* E = emf + q * 3 * G.nedge;
-    const int64_t eo = eidx(G, i, j, k);
+    double* E = emf + q * 3 * G.ns + sidx(G, i, j, k);
+    const int64_t eo = eidx(G, i, j, k);   // of the tags
     if (i < G.n[0] + G.ng + wide && (!only || only[(q * 3 + 0) * G.nedge + eo])) {
         double Exzf = EF(2, 0, i, j, k), Exzfm = EF(2, 0, i, j - 1, k), Exyf = EF(1, 0, i, j, k), Exyfm = EF(1, 0, i, j, k - 1);
         double NE = EC(0, i, j, k), NW = EC(0, i, j - 1, k), SE = EC(0, i, j, k - 1), SW = EC(0, i, j - 1, k - 1);
@@ -627,7 +304,7 @@ __global__ __launch_bounds__(256) void k_emf_gs(DevGrid G, const double* __restr
         double Sz = copysign(1., FD(2, i, j, k)), Szm = copysign(1., FD(2, i, j - 1, k));
         double dE = (1. - Sz) * (NE - Exyf) + (1. + Sz) * (SE - Exyfm);
         double dW = (1. - Szm) * (Exyf - NW) + (1. + Szm) * (Exyfm - SW);
-        E[eo] = Eavg + (1. / 8.) * (dS - dN) + (1. / 8.) * (dW - dE);
+        E[0] = Eavg + (1. / 8.) * (dS - dN) + (1. / 8.) * (dW - dE);
     }
     if (j < G.n[1] + G.ng + wide && (!only || only[(q * 3 + 1) * G.nedge + eo])) {
         double Eyzf = EF(2, 1, i, j, k), Eyzfm = EF(2, 1, i - 1, j, k), Eyxf = EF(0, 0, i, j, k), Eyxfm = EF(0, 0, i, j, k - 1);
@@ -639,7 +316,7 @@ __global__ __launch_bounds__(256) void k_emf_gs(DevGrid G, const double* __restr
         double Sz = copysign(1., FD(2, i, j, k)), Szm = copysign(1., FD(2, i - 1, j, k));
         double dE = (1. - Sz) * (NE - Eyxf) + (1. + Sz) * (SE - Eyxfm);
         double dW = (1. - Szm) * (Eyxf - NW) + (1. + Szm) * (Eyxfm - SW);
-        E[G.nedge + eo] = Eavg + (1. / 8.) * (dS - dN) + (1. / 8.) * (dW - dE);
+        E[G.ns] = Eavg + (1. / 8.) * (dS - dN) + (1. / 8.) * (dW - dE);
     }
     if (k < G.n[2] + G.ng + wide && (!only || only[(q * 3 + 2) * G.nedge + eo])) {
         double Ezyf = EF(1, 1, i, j, k), Ezyfm = EF(1, 1, i - 1, j, k), Ezxf = EF(0, 1, i, j, k), Ezxfm = EF(0, 1, i, j - 1, k);
@@ -651,7 +328,7 @@ __global__ __launch_bounds__(256) void k_emf_gs(DevGrid G, const double* __restr
         double Sy = copysign(1., FD(1, i, j, k)), Sym = copysign(1., FD(1, i - 1, j, k));
         double dE = (1. - Sy) * (NE - Ezxf) + (1. + Sy) * (SE - Ezxfm);
         double dW = (1. - Sym) * (Ezxf - NW) + (1. + Sym) * (Ezxfm - SW);
-        E[2 * G.nedge + eo] = Eavg + (1. / 8.) * (dS - dN) + (1. / 8.) * (dW - dE);
+        E[2 * G.ns] = Eavg + (1. / 8.) * (dS - dN) + (1. / 8.) * (dW - dE);
     }
 }
 
@@ -794,7 +471,7 @@ __global__ __launch_bounds__(256) void k_metric_der(DevGrid G, const DevInst* __
 
 // MDER: the metric derivatives come from the static-metric cache a.mder
 // (the finite differences are not compiled in, which frees registers).
-template <bool FLAT, bool MDER = false>
+template <bool MDER>
 __global__ __launch_bounds__(256) void k_update(DevGrid G, UpdArgs a, int fd_order, int wpb) {
     // wpb workgroups per block over its (n+1)^3 sites (see wg_pos)
     const int R0 = G.n[0] + 1, R1 = G.n[1] + 1, R2 = G.n[2] + 1;
@@ -819,7 +496,7 @@ __global__ __launch_bounds__(256) void k_update(DevGrid G, UpdArgs a, int fd_ord
         double u[NHRSC];
 #pragma unroll
         for (int v = 0; v < NHRSC; ++v) u[v] = (a.cb == 0.0) ? An[v * nc] : a.ca * An[v * nc] + a.cb * Bn[v * nc];
-        if constexpr (!FLAT) {
+        {
             const double* M = a.mstate + q * (int64_t)a.mnv * nc + c;
             const double* X = a.aux + q * (int64_t)NAUX * nc + c;
             Met m;
@@ -849,26 +526,25 @@ __global__ __launch_bounds__(256) void k_update(DevGrid G, UpdArgs a, int fd_ord
             u[SY_] += m.sqrtg * (*a.dt) * a.dtfact * ss[1];
             u[SZ_] += m.sqrtg * (*a.dt) * a.dtfact * ss[2];
         }
-        const int64_t f0 = fidx<0>(G, i, j, k), f1 = fidx<1>(G, i, j, k), f2 = fidx<2>(G, i, j, k);
-        const double* F0 = a.flux[0] + q * NHRSC * G.nface[0];
-        const double* F1 = a.flux[1] + q * NHRSC * G.nface[1];
-        const double* F2 = a.flux[2] + q * NHRSC * G.nface[2];
-        const int64_t s1 = G.N[0], s2 = (int64_t)G.N[0] * (G.N[1] + 0);
+        const int64_t f = sidx(G, i, j, k), s1 = G.sp, s2 = (int64_t)G.sp * (G.N[1] + 1);
+        const double* F0 = a.flux[0] + q * NHRSC * G.ns + f;
+        const double* F1 = a.flux[1] + q * NHRSC * G.ns + f;
+        const double* F2 = a.flux[2] + q * NHRSC * G.ns + f;
 #pragma unroll
         for (int v = 0; v < NHRSC; ++v) {
-            double dFx = (F0[v * G.nface[0] + f0] - F0[v * G.nface[0] + f0 + 1]) * ix;
-            double dFy = (F1[v * G.nface[1] + f1] - F1[v * G.nface[1] + f1 + s1]) * iy;
-            double dFz = (F2[v * G.nface[2] + f2] - F2[v * G.nface[2] + f2 + s2]) * iz;
+            double dFx = (F0[v * G.ns] - F0[v * G.ns + 1]) * ix;
+            double dFy = (F1[v * G.ns] - F1[v * G.ns + s1]) * iy;
+            double dFz = (F2[v * G.ns] - F2[v * G.ns + s2]) * iz;
             u[v] += dtf * ((dFx + dFy) + dFz);
         }
 #pragma unroll
         for (int v = 0; v < NHRSC; ++v) Nn[v * nc] = u[v];
     }
     if (a.part == 1) return;
-    const double* E = a.emf + q * 3 * G.nedge;
-    auto Ex = [&](int ii, int jj, int kk) { return E[eidx(G, ii, jj, kk)]; };
-    auto Ey = [&](int ii, int jj, int kk) { return E[G.nedge + eidx(G, ii, jj, kk)]; };
-    auto Ez = [&](int ii, int jj, int kk) { return E[2 * G.nedge + eidx(G, ii, jj, kk)]; };
+    const double* E = a.emf + q * 3 * G.ns;
+    auto Ex = [&](int ii, int jj, int kk) { return E[sidx(G, ii, jj, kk)]; };
+    auto Ey = [&](int ii, int jj, int kk) { return E[G.ns + sidx(G, ii, jj, kk)]; };
+    auto Ez = [&](int ii, int jj, int kk) { return E[2 * G.ns + sidx(G, ii, jj, kk)]; };
     if (cj && ck) {  // x face (i in [ng, n+ng])
         int64_t f = q * G.nface[0] + fidx<0>(G, i, j, k);
         double b = (a.cb == 0.0) ? a.aB[0][f] : a.ca * a.aB[0][f] + a.cb * a.bB[0][f];
@@ -886,18 +562,17 @@ __global__ __launch_bounds__(256) void k_update(DevGrid G, UpdArgs a, int fd_ord
     }
 }
 
-// Flat-metric update over pairs of sites along x (i0, i0 + 1 with i0 even).
-// With even extents N[d] the cell arrays, the y- and z-face arrays (fluxes,
-// face B) have even row widths, so the two values of a pair sit in one
-// aligned 16-byte word and move with one access; the x-face and edge arrays
-// (odd row widths) keep 8-byte accesses, three x faces serving the pair's
-// two cells.  Per cell and face the arithmetic is that of k_update<true>,
-// operation for operation.  All loads of a pair are issued before its first
-// store (the stores may alias the loads: the third RK stage updates in
-// place), which takes 194 VGPRs, 2 waves per SIMD: measured faster in the
-// RK3 graph than k_update<true> and than a variant storing each variable as
-// it completes (48 VGPRs, 8 waves).  pairs = pairs per row; wpb workgroups
-// per block.
+// Flat-metric update over pairs of sites along x (i0, i0 + 1 from the first
+// interior one): the two values of a pair move with one 16-byte access, which
+// is aligned in the context's flux arrays and 8-byte aligned in the
+// boundary's; three x faces serve the pair's two cells, and the site after
+// the last pair holds the last x face.  Per cell and face the arithmetic is
+// that of k_update, operation for operation.  Every flat grid takes it,
+// whatever its extents (an odd extent's last pair holds one cell).  All loads
+// of a pair are issued before its first store (the stores may alias the
+// loads: the third RK stage updates in place), which takes 194 VGPRs, 2 waves
+// per SIMD.  Bound by memory: 456 bytes per zone and substep.  pairs = pairs
+// per row; wpb workgroups per block.
 __global__ __launch_bounds__(256, 2) void k_update_pairs(DevGrid G, UpdArgs a, int pairs, int wpb) {
     const int R1 = G.n[1] + 1, R2 = G.n[2] + 1;
     const WgPos wp = wg_pos(wpb);
@@ -908,25 +583,24 @@ __global__ __launch_bounds__(256, 2) void k_update_pairs(DevGrid G, UpdArgs a, i
     udivmod(r, pairs * R1, kz, rxy);
     udivmod(rxy, pairs, jy, px);
     const int ng = G.ng;
-    const int i0 = (ng & ~1) + 2 * px, j = ng + jy, k = ng + kz;
+    const int i0 = ng + 2 * px, j = ng + jy, k = ng + kz;
     const DevInst& I = a.inst[a.blk[q].inst];
     const double ix = I.idx[0], iy = I.idx[1], iz = I.idx[2];
     const double dtf = (*a.dt) * a.dtfact;
-    const int ilo = ng, ihi = G.n[0] + ng;             // cells [ilo, ihi), x faces [ilo, ihi]
-    const bool c0 = i0 >= ilo && i0 < ihi, c1 = i0 + 1 >= ilo && i0 + 1 < ihi;
+    const int ihi = G.n[0] + ng;                       // cells [ng, ihi), x faces [ng, ihi]
+    const bool c0 = i0 < ihi, c1 = i0 + 1 < ihi;
     const bool cj = j < G.n[1] + ng, ck = k < G.n[2] + ng;
     const int64_t nc = G.ncell;
-    typedef HIP_vector_type<double, 2> d2;
-    if (a.part != 2 && cj && ck && (c0 || c1)) {
+    typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+    if (a.part != 2 && cj && ck && c0) {
         const int64_t c = cidx(G, i0, j, k);
         double* Nn = a.nst + q * (int64_t)a.nnv * nc + c;
         const double* An = a.ast + q * (int64_t)a.anv * nc + c;
         const double* Bn = a.bst ? a.bst + q * (int64_t)a.bnv * nc + c : nullptr;
-        const int64_t f0 = fidx<0>(G, i0, j, k), f1 = fidx<1>(G, i0, j, k), f2 = fidx<2>(G, i0, j, k);
-        const double* F0 = a.flux[0] + q * NHRSC * G.nface[0];
-        const double* F1 = a.flux[1] + q * NHRSC * G.nface[1];
-        const double* F2 = a.flux[2] + q * NHRSC * G.nface[2];
-        const int64_t s1 = G.N[0], s2 = (int64_t)G.N[0] * G.N[1];
+        const int64_t f = sidx(G, i0, j, k), s1 = G.sp, s2 = (int64_t)G.sp * (G.N[1] + 1);
+        const double* F0 = a.flux[0] + q * NHRSC * G.ns + f;
+        const double* F1 = a.flux[1] + q * NHRSC * G.ns + f;
+        const double* F2 = a.flux[2] + q * NHRSC * G.ns + f;
         double u0[NHRSC], u1[NHRSC];
 #pragma unroll
         for (int v = 0; v < NHRSC; ++v) {
@@ -939,12 +613,12 @@ __global__ __launch_bounds__(256, 2) void k_update_pairs(DevGrid G, UpdArgs a, i
         }
 #pragma unroll
         for (int v = 0; v < NHRSC; ++v) {
-            const double* X = F0 + v * G.nface[0] + f0;
+            const double* X = F0 + v * G.ns;
             const double xa = X[0], xb = X[1], xc = X[2];
-            const d2 ya = *reinterpret_cast<const d2*>(F1 + v * G.nface[1] + f1);
-            const d2 yb = *reinterpret_cast<const d2*>(F1 + v * G.nface[1] + f1 + s1);
-            const d2 za = *reinterpret_cast<const d2*>(F2 + v * G.nface[2] + f2);
-            const d2 zb = *reinterpret_cast<const d2*>(F2 + v * G.nface[2] + f2 + s2);
+            const d2 ya = *reinterpret_cast<const d2*>(F1 + v * G.ns);
+            const d2 yb = *reinterpret_cast<const d2*>(F1 + v * G.ns + s1);
+            const d2 za = *reinterpret_cast<const d2*>(F2 + v * G.ns);
+            const d2 zb = *reinterpret_cast<const d2*>(F2 + v * G.ns + s2);
             {
                 double dFx = (xa - xb) * ix, dFy = (ya.x - yb.x) * iy, dFz = (za.x - zb.x) * iz;
                 u0[v] += dtf * ((dFx + dFy) + dFz);
@@ -956,27 +630,26 @@ __global__ __launch_bounds__(256, 2) void k_update_pairs(DevGrid G, UpdArgs a, i
         }
 #pragma unroll
         for (int v = 0; v < NHRSC; ++v) {
-            if (c0 && c1) *reinterpret_cast<d2*>(Nn + v * nc) = d2{u0[v], u1[v]};
-            else if (c0) Nn[v * nc] = u0[v];
-            else Nn[v * nc + 1] = u1[v];
+            if (c1) *reinterpret_cast<d2*>(Nn + v * nc) = d2{u0[v], u1[v]};
+            else Nn[v * nc] = u0[v];
         }
     }
     if (a.part == 1) return;
-    const double* E = a.emf + q * 3 * G.nedge;
-    auto Ex = [&](int ii, int jj, int kk) { return E[eidx(G, ii, jj, kk)]; };
-    auto Ey = [&](int ii, int jj, int kk) { return E[G.nedge + eidx(G, ii, jj, kk)]; };
-    auto Ez = [&](int ii, int jj, int kk) { return E[2 * G.nedge + eidx(G, ii, jj, kk)]; };
+    const double* E = a.emf + q * 3 * G.ns;
+    auto Ex = [&](int ii, int jj, int kk) { return E[sidx(G, ii, jj, kk)]; };
+    auto Ey = [&](int ii, int jj, int kk) { return E[G.ns + sidx(G, ii, jj, kk)]; };
+    auto Ez = [&](int ii, int jj, int kk) { return E[2 * G.ns + sidx(G, ii, jj, kk)]; };
     if (cj && ck) {  // x faces i0, i0 + 1 within [ilo, ihi]
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const int i = i0 + t;
-            if (i < ilo || i > ihi) continue;
+            if (i > ihi) continue;
             int64_t f = q * G.nface[0] + fidx<0>(G, i, j, k);
             double b = (a.cb == 0.0) ? a.aB[0][f] : a.ca * a.aB[0][f] + a.cb * a.bB[0][f];
             a.nB[0][f] = b + dtf * ((Ey(i, j, k + 1) - Ey(i, j, k)) * iz + (Ez(i, j, k) - Ez(i, j + 1, k)) * iy);
         }
     }
-    if (ck && (c0 || c1)) {  // y faces (cells' x positions, j in [ng, n+ng])
+    if (ck && c0) {  // y faces (cells' x positions, j in [ng, n+ng])
         const int64_t f = q * G.nface[1] + fidx<1>(G, i0, j, k);
         d2 b = *reinterpret_cast<const d2*>(a.aB[1] + f);
         if (a.cb != 0.0) {
@@ -986,11 +659,10 @@ __global__ __launch_bounds__(256, 2) void k_update_pairs(DevGrid G, UpdArgs a, i
         const double ez0 = Ez(i0, j, k), ez1 = Ez(i0 + 1, j, k), ez2 = Ez(i0 + 2, j, k);
         const double n0v = b.x + dtf * ((ez1 - ez0) * ix + (Ex(i0, j, k) - Ex(i0, j, k + 1)) * iz);
         const double n1v = b.y + dtf * ((ez2 - ez1) * ix + (Ex(i0 + 1, j, k) - Ex(i0 + 1, j, k + 1)) * iz);
-        if (c0 && c1) *reinterpret_cast<d2*>(a.nB[1] + f) = d2{n0v, n1v};
-        else if (c0) a.nB[1][f] = n0v;
-        else a.nB[1][f + 1] = n1v;
+        if (c1) *reinterpret_cast<d2*>(a.nB[1] + f) = d2{n0v, n1v};
+        else a.nB[1][f] = n0v;
     }
-    if (cj && (c0 || c1)) {  // z faces
+    if (cj && c0) {  // z faces
         const int64_t f = q * G.nface[2] + fidx<2>(G, i0, j, k);
         d2 b = *reinterpret_cast<const d2*>(a.aB[2] + f);
         if (a.cb != 0.0) {
@@ -1000,9 +672,8 @@ __global__ __launch_bounds__(256, 2) void k_update_pairs(DevGrid G, UpdArgs a, i
         const double n0v = b.x + dtf * ((Ex(i0, j + 1, k) - Ex(i0, j, k)) * iy + (Ey(i0, j, k) - Ey(i0 + 1, j, k)) * ix);
         const double n1v =
             b.y + dtf * ((Ex(i0 + 1, j + 1, k) - Ex(i0 + 1, j, k)) * iy + (Ey(i0 + 1, j, k) - Ey(i0 + 2, j, k)) * ix);
-        if (c0 && c1) *reinterpret_cast<d2*>(a.nB[2] + f) = d2{n0v, n1v};
-        else if (c0) a.nB[2][f] = n0v;
-        else a.nB[2][f + 1] = n1v;
+        if (c1) *reinterpret_cast<d2*>(a.nB[2] + f) = d2{n0v, n1v};
+        else a.nB[2][f] = n0v;
     }
 }
 
@@ -1059,24 +730,23 @@ __global__ __launch_bounds__(256) void k_fofc_flag(DevGrid G, EOS eos, Opts o, F
     auto lin = [&](int v, int64_t cc) {
         return a.cb == 0.0 ? A[v * nc + cc] : __dadd_rn(__dmul_rn(a.ca, A[v * nc + cc]), __dmul_rn(a.cb, Bs[v * nc + cc]));
     };
-    const int64_t f0 = fidx<0>(G, i, j, k), f1 = fidx<1>(G, i, j, k), f2 = fidx<2>(G, i, j, k);
-    const int64_t nf0 = G.nface[0], nf1 = G.nface[1], nf2 = G.nface[2];
-    const double* F0 = a.flux[0] + q * NHRSC * nf0;
-    const double* F1 = a.flux[1] + q * NHRSC * nf1;
-    const double* F2 = a.flux[2] + q * NHRSC * nf2;
-    const int64_t s1 = G.N[0], s2 = (int64_t)G.N[0] * G.N[1];
+    const int64_t nf0 = G.nface[0], nf1 = G.nface[1], nf2 = G.nface[2], ns = G.ns;
+    const int64_t f = sidx(G, i, j, k), s1 = G.sp, s2 = (int64_t)G.sp * (G.N[1] + 1);
+    const double* F0 = a.flux[0] + q * NHRSC * ns + f;
+    const double* F1 = a.flux[1] + q * NHRSC * ns + f;
+    const double* F2 = a.flux[2] + q * NHRSC * ns + f;
     double cons[NCONS];
     for (int v = 0; v < NHRSC; ++v) {
-        const double dFx = __dmul_rn(__dsub_rn(F0[v * nf0 + f0], F0[v * nf0 + f0 + 1]), ix);
-        const double dFy = __dmul_rn(__dsub_rn(F1[v * nf1 + f1], F1[v * nf1 + f1 + s1]), iy);
-        const double dFz = __dmul_rn(__dsub_rn(F2[v * nf2 + f2], F2[v * nf2 + f2 + s2]), iz);
+        const double dFx = __dmul_rn(__dsub_rn(F0[v * ns], F0[v * ns + 1]), ix);
+        const double dFy = __dmul_rn(__dsub_rn(F1[v * ns], F1[v * ns + s1]), iy);
+        const double dFz = __dmul_rn(__dsub_rn(F2[v * ns], F2[v * ns + s2]), iz);
         cons[v] = __dadd_rn(lin(v, c), __dmul_rn(dte, __dadd_rn(__dadd_rn(dFx, dFy), dFz)));
     }
     // ct_update_B{x,y,z}_face (grmhd_helpers.hh:441-475)
-    const double* E = a.emf + q * 3 * G.nedge;
-    auto Ex = [&](int ii, int jj, int kk) { return E[eidx(G, ii, jj, kk)]; };
-    auto Ey = [&](int ii, int jj, int kk) { return E[G.nedge + eidx(G, ii, jj, kk)]; };
-    auto Ez = [&](int ii, int jj, int kk) { return E[2 * G.nedge + eidx(G, ii, jj, kk)]; };
+    const double* E = a.emf + q * 3 * G.ns;
+    auto Ex = [&](int ii, int jj, int kk) { return E[sidx(G, ii, jj, kk)]; };
+    auto Ey = [&](int ii, int jj, int kk) { return E[G.ns + sidx(G, ii, jj, kk)]; };
+    auto Ez = [&](int ii, int jj, int kk) { return E[2 * G.ns + sidx(G, ii, jj, kk)]; };
     const double* bx = a.oB[0] + q * nf0;
     const double* by = a.oB[1] + q * nf1;
     const double* bz = a.oB[2] + q * nf2;
@@ -1709,6 +1379,7 @@ struct grmhd_ctx {
     // faces beyond which k_flux computes the ring itself; null when off
     int32_t* ring_nbr = nullptr;
     uint8_t* ring_own = nullptr;
+    bool ring_any = false;                    // some block has such a face
     // set by the RK3 step around the flux launches of its second and third
     // stages: their ring faces come from the neighbours' pushes and their
     // full faces read the cells beyond a block face from the neighbour's
@@ -1748,7 +1419,6 @@ struct grmhd_ctx {
     // side streams and fork/join events of the concurrent RK3 stages
     hipStream_t side[2] = {nullptr, nullptr};
     hipEvent_t fev[8] = {};
-    hipStream_t flux_s[3] = {nullptr, nullptr, nullptr};   // per-direction flux streams while set
     // graph
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -1822,6 +1492,7 @@ static void build_eos(grmhd_ctx* c) {
     c->ideal.gm1 = p.gamma - 1.0;
     c->ideal.gamma = c->ideal.gm1 + 1.0;
     c->ideal.ggm1 = c->ideal.gamma * c->ideal.gm1;
+    c->ideal.igm1 = 1.0 / c->ideal.gm1;
     c->ideal.eps_max = p.eps_max;
     c->ideal.temp_atm = p.temp_fl;
     c->ideal.ent_min = (p.temp_fl > 0.0) ? (p.temp_fl / c->ideal.gm1) : 1e-100;
@@ -1970,6 +1641,9 @@ static grmhd_status ctx_create_impl(const grmhd_params* p, const grmhd_grid* g, 
     G.ncell = (int64_t)G.N[0] * G.N[1] * G.N[2];
     for (int d = 0; d < 3; ++d) G.nface[d] = (int64_t)(G.N[0] + (d == 0)) * (G.N[1] + (d == 1)) * (G.N[2] + (d == 2));
     G.nedge = (int64_t)(G.N[0] + 1) * (G.N[1] + 1) * (G.N[2] + 1);
+    G.sp = (G.N[0] + 1 + 15) / 16 * 16;
+    G.so = (16 - G.ng % 16) % 16;
+    G.ns = (G.so + (int64_t)G.sp * (G.N[1] + 1) * (G.N[2] + 1) + 15) / 16 * 16;
     Opts& O = c->O;
     O.atmo = Atmo{p->rho_fl, p->temp_fl, p->ye_fl, p->atmo_tol};
     O.cp = C2PPar{p->c2p_tol, p->max_lorentz, p->max_sigma, p->beta_fallback, p->bh_alp_thresh, p->use_entropy_backup};
@@ -2000,10 +1674,10 @@ static grmhd_status ctx_create_impl(const grmhd_params* p, const grmhd_grid* g, 
     if ((e = hipMalloc(&c->blk_d, sizeof(DevBlk) * g->nq)) != hipSuccess) return fail("blk", e);
     if ((e = hipMemcpy(c->blk_d, blk.data(), sizeof(DevBlk) * g->nq, hipMemcpyHostToDevice)) != hipSuccess) return fail("blk copy", e);
     for (int d = 0; d < 3; ++d) {
-        if ((e = hipMalloc(&c->flux[d], sizeof(double) * NHRSC * G.nface[d] * G.nq)) != hipSuccess) return fail("flux", e);
-        if ((e = hipMalloc(&c->vbar[d], sizeof(double) * 4 * G.nface[d] * G.nq)) != hipSuccess) return fail("vbar", e);
+        if ((e = hipMalloc(&c->flux[d], sizeof(double) * NHRSC * G.ns * G.nq)) != hipSuccess) return fail("flux", e);
+        if ((e = hipMalloc(&c->vbar[d], sizeof(double) * 4 * G.ns * G.nq)) != hipSuccess) return fail("vbar", e);
     }
-    if ((e = hipMalloc(&c->emf, sizeof(double) * 3 * G.nedge * G.nq)) != hipSuccess) return fail("emf", e);
+    if ((e = hipMalloc(&c->emf, sizeof(double) * 3 * G.ns * G.nq)) != hipSuccess) return fail("emf", e);
     if (p->fofc) {
         for (int d = 0; d < 3; ++d)
             if ((e = hipMalloc(&c->ftag[d], G.nface[d] * G.nq)) != hipSuccess) return fail("fofc face tags", e);
@@ -2012,7 +1686,7 @@ static grmhd_status ctx_create_impl(const grmhd_params* p, const grmhd_grid* g, 
     if ((e = hipMalloc(&c->ecen, sizeof(double) * 3 * G.ncell * G.nq)) != hipSuccess) return fail("ecen", e);
     // E_center starts at zero, as the reference's freshly allocated view
     if ((e = hipMemset(c->ecen, 0, sizeof(double) * 3 * G.ncell * G.nq)) != hipSuccess) return fail("ecen clear", e);
-    if ((e = hipMemset(c->emf, 0, sizeof(double) * 3 * G.nedge * G.nq)) != hipSuccess) return fail("emf clear", e);
+    if ((e = hipMemset(c->emf, 0, sizeof(double) * 3 * G.ns * G.nq)) != hipSuccess) return fail("emf clear", e);
     c->n_dtpart = nblk((int64_t)G.n[0] * G.n[1] * G.n[2] * G.nq);
     if ((e = hipMalloc(&c->dtpart, sizeof(double) * c->n_dtpart)) != hipSuccess) return fail("dtpart", e);
     if ((e = hipMalloc(&c->stats, sizeof(DevStats))) != hipSuccess) return fail("stats", e);
@@ -2040,7 +1714,7 @@ static grmhd_status ctx_create_impl(const grmhd_params* p, const grmhd_grid* g, 
                 int bc[3] = {bq.b[0], bq.b[1], bq.b[2]};
                 bc[d] += dir;
                 if (bc[d] < 0 || bc[d] >= I.nb[d]) {
-                    if (I.bc[sd] != GRMHD_BC_PERIODIC) { own[q] |= (uint8_t)(1u << sd); continue; }
+                    if (I.bc[sd] != GRMHD_BC_PERIODIC) { own[q] |= (uint8_t)(1u << sd); c->ring_any = true; continue; }
                     bc[d] = (bc[d] + I.nb[d]) % I.nb[d];
                 }
                 nbr[(size_t)q * 6 + sd] = (int32_t)(I.q0 + bc[0] + (int64_t)I.nb[0] * (bc[1] + (int64_t)I.nb[1] * bc[2]));
@@ -2104,6 +1778,7 @@ static grmhd_status ctx_create_impl(const grmhd_params* p, const grmhd_grid* g, 
             c->cmap_h = fin->cmap;
             c->fblk_h = fin->fblk;
             for (int d = 0; d < 3; ++d) { ffh.nb[d] = fin->nb[d]; ffh.n[d] = G.n[d]; ffh.N[d] = G.N[d]; ffh.nface[d] = G.nface[d]; }
+            ffh.sp = G.sp; ffh.so = G.so; ffh.ns = G.ns;
             for (int d = 0; d < 6; ++d) ffh.bc[d] = fin->bc[d];
             ffh.ng = G.ng; ffh.ncell = G.ncell; ffh.nq = G.nq;
             ffh.cmap = c->cmap_h.data(); ffh.blk = c->fblk_h.data();
@@ -2360,52 +2035,66 @@ static grmhd_status launch_check(const char* what) {
 // ---- dispatch helpers -------------------------------------------------------
 // only != null: FOFC correction pass over the tagged faces with the options O
 // (donor cell + LLF); otherwise every face the later passes read.
-template <typename EOS, int REC, bool FLAT>
-static void launch_flux3(grmhd_ctx* c, const EOS& eos, const double* aux, const double* ms, int mnv,
-                         const double* const B[3], hipStream_t s0, const Opts& O, uint8_t* const* only) {
-    const DevGrid& G = c->G;
-    const bool uct = c->P.emf != GRMHD_EMF_GS;
-    int nf[3];
+static FluxArgs flux_args(grmhd_ctx* c, const double* aux, const double* ms, int mnv, const double* const B[3]) {
+    FluxArgs f{};
+    f.aux = aux; f.mstate = ms; f.mnv = mnv;
     for (int d = 0; d < 3; ++d) {
-        const int t0 = d == 0 ? 1 : 0, t1 = d == 2 ? 1 : 2;
-        const int Rn = G.n[d] + 1, n0 = G.n[t0], n1 = G.n[t1];
-        nf[d] = uct ? Rn * (n0 * n1 + 2 * G.ng * (n0 + n1)) : (Rn + 2 * O.fofc) * G.N[t0] * G.N[t1];
-    }
-    static const char* fam[3] = {"flux_x", "flux_y", "flux_z"};
-    for (int d = 0; d < 3; ++d) {
-        const hipStream_t s = c->flux_s[d] ? c->flux_s[d] : s0;
-        Scope sc(c, only ? "fofc" : fam[d], s);
-        const int bs = c->tune.flux[d];
-        const int wpb = (int)nblk_bs(nf[d], bs);
-        const dim3 grid((unsigned)(wpb * G.nq));
-        const uint8_t* od = only ? only[d] : nullptr;
-        const uint8_t* ro = (only || !c->ring_copy_now) ? nullptr : c->ring_own;
-        // the prefetching variant is built for WENO-Z only (the other
-        // reconstructions load one or three values per side)
-        bool pf = false;
-        if constexpr (REC == 0) pf = c->tune.flux_prefetch[d] != 0 && !only;
-        const int32_t* pn = ro ? c->ring_nbr : nullptr;
+        f.B[d] = B[d]; f.flux[d] = c->flux[d]; f.vbar[d] = c->vbar[d];
         // (x faces interpolate from four adjacent cells of a row, which is
         // cheaper than streaming 13 cached values: cache for y and z only)
-        const double* fm = (!FLAT && d > 0 && c->fmet[d] && ms == c->mder_src && mnv == NSTATE) ? c->fmet[d] : nullptr;
-#define FLUXL(DD, PFV) k_flux<EOS, REC, FLAT, DD, PFV><<<grid, bs, 0, s>>>(G, eos, O, aux, ms, mnv, B[DD], c->flux[DD], c->vbar[DD], wpb, od, ro, pn, fm)
-        if constexpr (REC == 0) {
-            if (pf) { if (d == 0) FLUXL(0, true); else if (d == 1) FLUXL(1, true); else FLUXL(2, true); }
-            else { if (d == 0) FLUXL(0, false); else if (d == 1) FLUXL(1, false); else FLUXL(2, false); }
-        } else {
-            if (d == 0) FLUXL(0, false); else if (d == 1) FLUXL(1, false); else FLUXL(2, false);
+        f.fmc[d] = (!c->P.flat_metric && d > 0 && c->fmet[d] && ms == c->mder_src && mnv == NSTATE) ? c->fmet[d] : nullptr;
+    }
+    return f;
+}
+template <typename EOS, bool FLAT>
+static void launch_flux_tagged(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O,
+                               uint8_t* const* only) {
+    const DevGrid& G = c->G;
+    for (int d = 0; d < 3; ++d) {
+        Scope sc(c, "fofc", s);
+        const int64_t n = (int64_t)(G.n[d] + 1) * G.N[(d + 1) % 3] * G.N[(d + 2) % 3];
+        const int bs = c->tune.flux[d];
+        f.tiles = (int)nblk_bs(n, bs);
+        const dim3 grid((unsigned)(f.tiles * G.nq));
+        if (d == 0) k_flux_tagged<EOS, FLAT, 0><<<grid, bs, 0, s>>>(G, eos, O, f, only[0]);
+        else if (d == 1) k_flux_tagged<EOS, FLAT, 1><<<grid, bs, 0, s>>>(G, eos, O, f, only[1]);
+        else k_flux_tagged<EOS, FLAT, 2><<<grid, bs, 0, s>>>(G, eos, O, f, only[2]);
+    }
+}
+// The three directions in one launch; one by one where each is timed.
+template <typename EOS, int REC, bool FLAT>
+static void launch_flux(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O) {
+    const DevGrid& G = c->G;
+    const bool uct = c->P.emf != GRMHD_EMF_GS;
+    static const char* fam[3] = {"flux_x", "flux_y", "flux_z"};
+    f.ring_own = c->ring_copy_now ? c->ring_own : nullptr;
+    f.push_nbr = f.ring_own ? c->ring_nbr : nullptr;
+    f.ndir = c->timing ? 1 : 3;
+    for (f.dir0 = 0; f.dir0 < 3; f.dir0 += f.ndir) {
+        Scope sc(c, fam[f.dir0], s);
+        const int bs = c->tune.flux[f.dir0];
+        f.tiles = f.tilesr = 0;
+        for (int d = f.dir0; d < f.dir0 + f.ndir; ++d) {
+            const int t0 = d == 0 ? 1 : 0, t1 = d == 2 ? 1 : 2;
+            const int64_t faces = G.n[d] + 1 + (uct ? 0 : 2 * O.fofc);
+            const int64_t full = uct ? G.n[t0] * G.n[t1] : G.N[t0] * G.N[t1];
+            const int64_t ring = !uct || (f.ring_own && !c->ring_any) ? 0 : 2 * G.ng * (G.n[t0] + G.n[t1]);
+            f.tiles = std::max(f.tiles, (int)nblk_bs(faces * full, bs));
+            f.tilesr = std::max(f.tilesr, (int)nblk_bs(faces * ring, bs));
         }
-#undef FLUXL
+        k_flux<EOS, REC, FLAT><<<dim3((unsigned)((f.tiles + f.tilesr) * f.ndir * G.nq)), bs, 0, s>>>(G, eos, O, f);
     }
 }
 template <typename EOS, bool FLAT>
 static void flux_rec(grmhd_ctx* c, const EOS& eos, const double* aux, const double* ms, int mnv,
                      const double* const B[3], hipStream_t s, int recon, const Opts& O, uint8_t* const* only) {
+    const FluxArgs f = flux_args(c, aux, ms, mnv, B);
+    if (only) { launch_flux_tagged<EOS, FLAT>(c, eos, f, s, O, only); return; }
     switch (recon) {
-        case 0: launch_flux3<EOS, 0, FLAT>(c, eos, aux, ms, mnv, B, s, O, only); break;
-        case 1: launch_flux3<EOS, 1, FLAT>(c, eos, aux, ms, mnv, B, s, O, only); break;
-        case 2: launch_flux3<EOS, 2, FLAT>(c, eos, aux, ms, mnv, B, s, O, only); break;
-        default: launch_flux3<EOS, 3, FLAT>(c, eos, aux, ms, mnv, B, s, O, only); break;
+        case 0: launch_flux<EOS, 0, FLAT>(c, eos, f, s, O); break;
+        case 1: launch_flux<EOS, 1, FLAT>(c, eos, f, s, O); break;
+        case 2: launch_flux<EOS, 2, FLAT>(c, eos, f, s, O); break;
+        default: launch_flux<EOS, 3, FLAT>(c, eos, f, s, O); break;
     }
 }
 static void launch_fluxes(grmhd_ctx* c, const double* aux, const double* ms, int mnv, const double* const B[3],
@@ -2456,15 +2145,6 @@ static void launch_emf(grmhd_ctx* c, const double* const B[3], hipStream_t s) {
         }
     });
 }
-// k_update_pairs needs an even row width (the cell and y/z-face arrays then
-// put a pair's two values in one aligned 16-byte word) and 16-byte aligned
-// arrays
-static bool update_pairs_ok(const DevGrid& G, const UpdArgs& a) {
-    auto al = [](const void* p) { return p == nullptr || ((uintptr_t)p & 15) == 0; };
-    bool ok = (G.N[0] % 2) == 0 && al(a.nst) && al(a.ast) && al(a.bst);
-    for (int d = 1; d < 3; ++d) ok = ok && al(a.flux[d]) && al(a.nB[d]) && al(a.aB[d]) && al(a.bB[d]);
-    return ok;
-}
 static void launch_update(grmhd_ctx* c, UpdArgs& a, hipStream_t s) {
     Scope sc(c, "update", s);
     const DevGrid& G = c->G;
@@ -2472,15 +2152,14 @@ static void launch_update(grmhd_ctx* c, UpdArgs& a, hipStream_t s) {
     for (int d = 0; d < 3; ++d) a.flux[d] = c->flux[d];
     a.emf = c->emf;
     a.mder = (c->mder && a.mstate == c->mder_src && a.mnv == NSTATE) ? c->mder : nullptr;
-    if (c->P.flat_metric && update_pairs_ok(G, a)) {
-        const int pairs = (((G.n[0] + G.ng) & ~1) - (G.ng & ~1)) / 2 + 1;
+    if (c->P.flat_metric) {
+        const int pairs = G.n[0] / 2 + 1;
         const int wpb = (int)nblk_bs((int64_t)pairs * (G.n[1] + 1) * (G.n[2] + 1), c->tune.update);
         k_update_pairs<<<dim3((unsigned)(wpb * G.nq)), c->tune.update, 0, s>>>(G, a, pairs, wpb);
         return;
     }
     site_launch(G, c->tune.update, [&](dim3 g, int wpb) {
-        if (c->P.flat_metric) k_update<true><<<g, c->tune.update, 0, s>>>(G, a, c->P.fd_order, wpb);
-        else if (a.mder) k_update<false, true><<<g, c->tune.update, 0, s>>>(G, a, c->P.fd_order, wpb);
+        if (a.mder) k_update<true><<<g, c->tune.update, 0, s>>>(G, a, c->P.fd_order, wpb);
         else k_update<false><<<g, c->tune.update, 0, s>>>(G, a, c->P.fd_order, wpb);
     });
 }
@@ -2558,7 +2237,7 @@ static void launch_reflux(grmhd_ctx* c, hipStream_t s, int part = 0) {
     const DevGrid& G = c->G;
     if (c->n_rflux > 0 && part != 2)
         k_reflux_flux<<<dim3(nblk(c->n_rflux), NHRSC), 256, 0, s>>>(c->rflux, (int)c->n_rflux, c->flux[0], c->flux[1],
-                                                                    c->flux[2], G.nface[0], G.nface[1], G.nface[2]);
+                                                                    c->flux[2], G.ns);
     if (c->n_remf > 0 && part != 1) k_reflux_emf<<<nblk(c->n_remf), 256, 0, s>>>(c->remf, (int)c->n_remf, c->emf);
 }
 
@@ -3080,22 +2759,15 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
     if (!conc) k_reset_diag<<<nblk(G.ncell * G.nq), 256, 0, s>>>(G.ncell, G.nq, aux);
     for (int sidx = 0; sidx < 3; ++sidx) {
         Stage& S = st[sidx];
-        if (conc) {
-            fork(0, s, c->side[0]);
+        const bool reset_aside = conc && sidx == 0;
+        if (reset_aside) {
             fork(0, s, c->side[1]);
-            if (sidx == 0) k_reset_diag<<<nblk(G.ncell * G.nq), 256, 0, c->side[1]>>>(G.ncell, G.nq, aux);
-            c->flux_s[1] = c->side[0]; c->flux_s[2] = c->side[1];
-            c->ring_copy_now = sidx > 0;
-            launch_fluxes(c, aux, state, NSTATE, S.oB, s);
-            c->ring_copy_now = false;
-            c->flux_s[1] = c->flux_s[2] = nullptr;
-            fork(1, c->side[0], s);
-            fork(2, c->side[1], s);
-        } else {
-            c->ring_copy_now = sidx > 0;
-            launch_fluxes(c, aux, state, NSTATE, S.oB, s);
-            c->ring_copy_now = false;
+            k_reset_diag<<<nblk(G.ncell * G.nq), 256, 0, c->side[1]>>>(G.ncell, G.nq, aux);
         }
+        c->ring_copy_now = sidx > 0;
+        launch_fluxes(c, aux, state, NSTATE, S.oB, s);
+        c->ring_copy_now = false;
+        if (reset_aside) fork(2, c->side[1], s);
         // the cell part of the update needs only the fluxes (on a forest
         // after their reflux): it runs on side[0] beside the edge EMFs, the
         // face (CT) part after them (and their reflux) on s.  Not with GS
@@ -3307,45 +2979,19 @@ extern "C" grmhd_status grmhd_autotune(grmhd_ctx* c, const double* state, const 
     double* const B1[3] = {c->B1[0], c->B1[1], c->B1[2]};
     const double* const B1c[3] = {c->B1[0], c->B1[1], c->B1[2]};
     grmhd_tuning keep = c->tune;
-    // the three flux launches as the RK3 stages run them: on three streams
-    // when the stages use side streams, and in the form of the second and
-    // third stages (ring faces pushed, reads across block faces) when the
-    // context shares ring faces; the directions run concurrently, so each
-    // choice is timed against the other two
     const bool conc = c->P.stage_streams && !c->P.fofc && c->side[0] && c->side[1];
-    auto fluxes_as_in_step = [&] {
-        if (conc) {
-            for (int k = 0; k < 2; ++k) {
-                (void)hipEventRecord(c->fev[k], s);
-                (void)hipStreamWaitEvent(c->side[k], c->fev[k], 0);
-            }
-            c->flux_s[1] = c->side[0]; c->flux_s[2] = c->side[1];
-        }
-        c->ring_copy_now = c->ring_own != nullptr;
-        launch_fluxes(c, aux, state, NSTATE, Bc, s);
-        c->ring_copy_now = false;
-        if (conc) {
-            c->flux_s[1] = c->flux_s[2] = nullptr;
-            for (int k = 0; k < 2; ++k) {
-                (void)hipEventRecord(c->fev[2 + k], c->side[k]);
-                (void)hipStreamWaitEvent(s, c->fev[2 + k], 0);
-            }
-        }
-    };
-    for (int d = 0; d < 3; ++d) {
-        // one direction at a time (the other two run at their current
-        // choice): workgroup size and, for WENO-Z, the prefetching variant
-        float best = 1e30f;
-        int bs = c->tune.flux[d], bp = c->tune.flux_prefetch[d];
-        for (int pf = 0; pf < (c->P.recon == GRMHD_RECON_WENOZ ? 2 : 1); ++pf)
-            for (int v : cand) {
-                c->tune.flux[d] = v;
-                c->tune.flux_prefetch[d] = pf;
-                const float ms = time_it(fluxes_as_in_step);
-                if (ms < best) { best = ms; bs = v; bp = pf; }
-            }
-        c->tune.flux[d] = bs;
-        c->tune.flux_prefetch[d] = bp;
+    // the flux launch in the form of the second and third RK stages (ring
+    // faces pushed, reads across block faces) when the context shares ring
+    // faces; one workgroup size for its three directions
+    {
+        int v = c->tune.flux[0];
+        pick(&v, [&] {
+            for (int d = 0; d < 3; ++d) c->tune.flux[d] = v;
+            c->ring_copy_now = c->ring_own != nullptr;
+            launch_fluxes(c, aux, state, NSTATE, Bc, s);
+            c->ring_copy_now = false;
+        });
+        for (int d = 0; d < 3; ++d) c->tune.flux[d] = v;
     }
     // the edge EMFs and the update as the stages run them: the update's cell
     // part beside the EMFs on a side stream, its face part after them

@@ -46,6 +46,40 @@ enum { EOS_RHO_TOO_HIGH = 0, EOS_RHO_TOO_LOW, EOS_EPS_TOO_HIGH, EOS_EPS_TOO_LOW,
 
 GHD double sq(double x) { return x * x; }
 
+// 1/b for a normal, finite b: the hardware reciprocal refined by two
+// Newton-Raphson steps r <- r + r (1 - b r) (within 1 ulp of 1/b; about half
+// the instructions of an IEEE division, which also handles zero, infinity and
+// denormal operands).  Host builds divide.
+GHD double nr_rcp(double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r = __builtin_amdgcn_rcp(b);
+#else
+    double r = 1.0 / b;
+#endif
+    double e = fma(-b, r, 1.0);
+    r = fma(e, r, r);
+    e = fma(-b, r, 1.0);
+    return fma(e, r, r);
+}
+// sqrt(x) and 1/sqrt(x) for a normal, finite x > 0: the hardware's reciprocal
+// root (about 24 bits) and two coupled Newton steps, the last one on the
+// residual x - g^2; half the instructions of the library's root and a
+// division.  Host builds use those.
+GHD void nr_sqrt(double x, double& g, double& ig) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double y = __builtin_amdgcn_rsq(x);
+#else
+    const double y = 1.0 / sqrt(x);
+#endif
+    double h = 0.5 * y;
+    g = x * y;
+    double r = fma(-g, h, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    r = fma(-g, h, 0.5);
+    ig = 2.0 * fma(h, r, h);
+}
 // ---- 3-metric -------------------------------------------------------------
 struct Met {
     double g[6], gi[6], beta[3], alp, sqrtg;
@@ -78,6 +112,7 @@ struct Met {
 struct EosIdeal {
     static constexpr bool has_ye = false, is_ideal = true;
     double gm1, gamma, ggm1, eps_max, ent_min, temp_atm;
+    double igm1;             // 1 / gm1
     double ls_min, ls_max;   // log(ent_min)/gm1, log(eps_max)/gm1 (entropy bounds are these minus log rho)
     GHD double hmin() const { return 1. + 1e-15; }
     GHD double rhomax() const { return 1e100; }
@@ -124,14 +159,23 @@ struct EosIdeal {
         cs2 = ggm1 * eps / h; ent = ent_of(eps, rho);
         return p;
     }
-    // press_eps_csnd2__temp_rho_ye (face EOS)
-    GHD double press_from_temp(double& eps, double& cs2, double& temp, double rho, unsigned& e) const {
+    // press_eps_csnd2__temp_rho_ye and eps_h_csnd2_temp_entropy__press_rho_ye
+    // for face states: eps, p and rho h c_s^2 (which the wave speeds need and
+    // which takes no division).  T / gm1 as a product with one correction
+    // step, the quotient to the last bit or next to it.
+    GHD double face_from_temp(double& eps, double& a2, double temp, double rho) const {
+        unsigned e = 0;
         limit_temp(temp, e);
-        eps = temp / gm1;
-        double p = gm1 * eps * rho;
-        double h = 1.0 + gamma * eps;
-        cs2 = ggm1 * eps / h;
+        const double q = temp * igm1;
+        eps = fma(fma(-gm1, q, temp), igm1, q);
+        const double p = gm1 * eps * rho;
+        a2 = gamma * p;
         return p;
+    }
+    GHD double face_from_press(double& eps, double& a2, double press, double rho) const {
+        eps = press / (gm1 * rho);
+        a2 = gamma * press;
+        return press;
     }
     GHD double press_h_cs2_from_temp(double& h, double& cs2, double& temp, double rho, unsigned& e) const {
         limit_temp(temp, e);
@@ -139,13 +183,6 @@ struct EosIdeal {
         double p = gm1 * eps * rho;
         h = 1.0 + gamma * eps; cs2 = ggm1 * eps / h;
         return p;
-    }
-    // eps_h_csnd2_temp_entropy__press_rho_ye
-    GHD double eps_from_press(double& h, double& cs2, double& temp, double& ent, double& press, double rho,
-                              unsigned&) const {
-        double eps = press / (gm1 * rho);
-        h = 1.0 + gamma * eps; cs2 = ggm1 * eps / h; ent = ent_of(eps, rho); temp = eps * gm1;
-        return eps;
     }
 };
 
@@ -242,15 +279,25 @@ struct EosHybrid {
         cs2 = cs2_of(rho, eth, h); ent = ent_of(eth, rho);
         return p;
     }
-    GHD double press_from_temp(double& eps, double& cs2, double& temp, double rho, unsigned& e) const {
+    GHD double a2_of(double rho, double eth) const { return rho * (dpcold(rho) + gth_m1 * (gth_m1 + 1) * eth); }
+    GHD double face_from_temp(double& eps, double& a2, double temp, double rho) const {
+        unsigned e = 0;
         chk_rho(rho, e); chk_temp(temp, e);
         double ec; double pc = pcold(ec, rho);
         double eth = eth_of_t(temp);
-        double p = pc + eth * rho * gth_m1;
         eps = ec + eth;
-        double h = 1. + eps + p / rho;
-        cs2 = cs2_of(rho, eth, h);
-        return p;
+        a2 = a2_of(rho, eth);
+        return pc + eth * rho * gth_m1;
+    }
+    GHD double face_from_press(double& eps, double& a2, double press, double rho) const {
+        unsigned e = 0;
+        chk_rho(rho, e);
+        double ec; double pc = pcold(ec, rho);
+        press = fmax(press, pc);
+        double eth = fmax(0, (press - pc) / (rho * gth_m1));
+        eps = eth + ec;
+        a2 = a2_of(rho, eth);
+        return press;
     }
     GHD double press_h_cs2_from_temp(double& h, double& cs2, double& temp, double rho, unsigned& e) const {
         chk_rho(rho, e); chk_temp(temp, e);
@@ -259,16 +306,6 @@ struct EosHybrid {
         double p = pc + eth * rho * gth_m1;
         h = 1. + ec + eth + p / rho; cs2 = cs2_of(rho, eth, h);
         return p;
-    }
-    GHD double eps_from_press(double& h, double& cs2, double& temp, double& ent, double& press, double rho,
-                              unsigned& e) const {
-        chk_rho(rho, e);
-        double ec; double pc = pcold(ec, rho);
-        press = fmax(press, pc);
-        double eth = fmax(0, (press - pc) / (rho * gth_m1));
-        double eps = eth + ec;
-        h = 1. + eps + press / rho; cs2 = cs2_of(rho, eth, h); ent = ent_of(eth, rho); temp = t_of(eth);
-        return eps;
     }
 };
 
@@ -998,21 +1035,6 @@ GHD void weno_betas(double b0, double b1, double b2, double& d0, double& d1, dou
     d0 = b0 + eps; d1 = b1 + eps; d2 = b2 + eps;
     t5 = fabs(b0 - b2);
 }
-// 1/b for a normal, finite b: the hardware reciprocal refined by two
-// Newton-Raphson steps r <- r + r (1 - b r) (within 1 ulp of 1/b; about half
-// the instructions of an IEEE division, which also handles zero, infinity and
-// denormal operands).  Host builds divide.
-GHD double nr_rcp(double b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    double r = __builtin_amdgcn_rcp(b);
-#else
-    double r = 1.0 / b;
-#endif
-    double e = fma(-b, r, 1.0);
-    r = fma(e, r, r);
-    e = fma(-b, r, 1.0);
-    return fma(e, r, r);
-}
 GHD void wenoz(double um3, double um2, double um1, double u0, double up1, double up2, double& uL, double& uR) {
     const double c0 = 13.0 / 12.0, c1 = 0.25;
     // right state (cell i stencils; a0 pairs with i2, a2 with i0 on this side)
@@ -1045,6 +1067,79 @@ GHD void wenoz(double um3, double um2, double um1, double u0, double up1, double
     // SS >= 36 (every a >= its linear weight)
     if (SS < 1e300) { const double inv = nr_rcp(SS); uR = rn * lS * inv; uL = ln * rS * inv; }
     else { uR = rn / rS; uL = ln / lS; }
+}
+// WENO-Z from the cell's side: both face values of the cell of u0 (its lower
+// face's right state and its upper face's left state) from um2..up2.  The
+// candidates pair with the linear weights in opposite order.  Everything is
+// formed from the four differences of neighbours, and a face value is u0 plus
+// a correction, so that smooth data lose no digits to the candidates' large
+// coefficients.  The multiply-adds are written out: a value that two blocks
+// form (a face on their common boundary) then has the same bits wherever this
+// is inlined.  Here every ratio is divided by itself (values of any size):
+// the wide form, taken where wenoz_face says so.
+struct WenoCell { double d0, d1, d2, cl[3], ch[3]; };
+GHD void weno_cell_parts(double um2, double um1, double u0, double up1, double up2, WenoCell& w) {
+#pragma clang fp contract(off)
+    const double c0 = 13.0 / 12.0, c1 = 0.25, eps = 1.0e-42;
+    const double dm = um1 - um2, dl = u0 - um1, dr = up1 - u0, dp = up2 - up1;
+    const double a0 = dl - dm, a1 = dr - dl, a2 = dp - dr;
+    const double f0 = fma(2.0, dl, a0), f1 = dl + dr, f2 = fma(-2.0, dr, a2);
+    w.d0 = fma(c1 * f0, f0, fma(c0 * a0, a0, eps));
+    w.d1 = fma(c1 * f1, f1, fma(c0 * a1, a1, eps));
+    w.d2 = fma(c1 * f2, f2, fma(c0 * a2, a2, eps));
+    const double T = 3.0 * dl, Q = 3.0 * dr;
+    w.ch[0] = fma(2.0, a0, T); w.ch[1] = Q - a1; w.ch[2] = Q - a2;
+    w.cl[0] = fma(2.0, a2, -Q); w.cl[1] = -T - a1; w.cl[2] = -T - a0;
+}
+GHD void wenoz_cell_wide(double um2, double um1, double u0, double up1, double up2, double& lo, double& hi) {
+#pragma clang fp contract(off)
+    WenoCell w;
+    weno_cell_parts(um2, um1, u0, up1, up2, w);
+    const double t5 = fabs(w.d0 - w.d2);
+    const double s0 = 1.0 + sq(t5 / w.d0), s1 = 6.0 * (1.0 + sq(t5 / w.d1)), s2 = 1.0 + sq(t5 / w.d2);
+    const double s0h = 3.0 * s0, s2h = 3.0 * s2;
+    lo = u0 + (w.cl[0] * s2 + w.cl[1] * s1 + w.cl[2] * s0h) / (6.0 * (s2 + s1 + s0h));
+    hi = u0 + (w.ch[0] * s0 + w.ch[1] * s1 + w.ch[2] * s2h) / (6.0 * (s0 + s1 + s2h));
+}
+// Both states of a face from the six cells around it: the upper value of the
+// cell below and the lower value of the cell above, in the forms above, with
+// the indicators' common parts and one reciprocal each of the indicators'
+// product and of the weights' sums shared by the two sides.  False where a
+// product is too large for its reciprocal (or NaN) and the caller has to take
+// wenoz_face_wide: the test of many variables then costs one branch.  (The
+// product is >= 1e-252 from the 1e-42 floors, the sums' >= 100.)
+GHD bool wenoz_face(double um3, double um2, double um1, double u0, double up1, double up2, double& uL, double& uR) {
+#pragma clang fp contract(off)
+    const double c0 = 13.0 / 12.0, c1 = 0.25, eps = 1.0e-42;
+    const double e0 = um2 - um3, e1 = um1 - um2, e2 = u0 - um1, e3 = up1 - u0, e4 = up2 - up1;
+    const double a0 = e1 - e0, a1 = e2 - e1, a2 = e3 - e2, a3 = e4 - e3;
+    const double g1 = fma(c0 * a1, a1, eps), g2 = fma(c0 * a2, a2, eps);
+    const double lf0 = fma(2.0, e1, a0), lf1 = e1 + e2, lf2 = fma(-2.0, e2, a2);
+    const double rf0 = fma(2.0, e2, a1), rf1 = e2 + e3, rf2 = fma(-2.0, e3, a3);
+    const double l0 = fma(c1 * lf0, lf0, fma(c0 * a0, a0, eps)), l1 = fma(c1 * lf1, lf1, g1), l2 = fma(c1 * lf2, lf2, g2);
+    const double r0 = fma(c1 * rf0, rf0, g1), r1 = fma(c1 * rf1, rf1, g2), r2 = fma(c1 * rf2, rf2, fma(c0 * a3, a3, eps));
+    const double lt = fabs(l0 - l2), rt = fabs(r0 - r2);
+    const double lP01 = l0 * l1, lP = lP01 * l2, rP01 = r0 * r1, rP = rP01 * r2, PP = lP * rP;
+    const double ip = nr_rcp(PP), lr = lt * rP * ip, rr = rt * lP * ip;
+    const double lq0 = l1 * l2 * lr, lq1 = l0 * l2 * lr, lq2 = lP01 * lr;
+    const double rq0 = r1 * r2 * rr, rq1 = r0 * r2 * rr, rq2 = rP01 * rr;
+    const double ls0 = fma(lq0, lq0, 1.0), ls1 = 6.0 * fma(lq1, lq1, 1.0), ls2 = 3.0 * fma(lq2, lq2, 1.0);
+    const double rs2 = fma(rq2, rq2, 1.0), rs1 = 6.0 * fma(rq1, rq1, 1.0), rs0 = 3.0 * fma(rq0, rq0, 1.0);
+    // corrections to um1 (upper value of the cell below) and u0 (lower value
+    // of the cell above)
+    const double T = 3.0 * e2;
+    const double ln = fma(fma(2.0, a0, 3.0 * e1), ls0, fma(T - a1, ls1, (T - a2) * ls2));
+    const double rn = fma(fma(2.0, a3, -3.0 * e3), rs2, fma(-T - a2, rs1, (-T - a1) * rs0));
+    const double lS = ls0 + ls1 + ls2, rS = rs0 + rs1 + rs2, SS = lS * rS;
+    const double is = nr_rcp(SS) * (1.0 / 6.0);
+    uL = fma(ln, rS * is, um1);
+    uR = fma(rn, lS * is, u0);
+    return PP < 1e300 && SS < 1e300;
+}
+GHD void wenoz_face_wide(double um3, double um2, double um1, double u0, double up1, double up2, double& uL, double& uR) {
+    double x;
+    wenoz_cell_wide(um3, um2, um1, u0, up1, x, uL);
+    wenoz_cell_wide(um2, um1, u0, up1, up2, uR, x);
 }
 GHD double mc2(double sL, double sR) {
     double sC = 0.5 * (sR + sL), sg = copysign(1.0, sR);

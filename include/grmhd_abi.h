@@ -335,15 +335,16 @@ grmhd_status grmhd_set_static_metric(grmhd_ctx* ctx, const double* state, int32_
 /* Workgroup sizes (threads) of the kernel families, chosen by
  * grmhd_autotune; every size is one of 64, 128, 256. */
 typedef struct {
-    int32_t flux[3];        /* face-flux kernels, x/y/z */
+    int32_t flux[3];        /* face-flux kernel; x, y, z where each direction is
+                             * a launch of its own (timing, FOFC), x where one
+                             * launch holds the three */
     int32_t emf;            /* edge EMFs */
     int32_t update;         /* fused RK update + CT */
     int32_t gather_faces;   /* ghost gather of face B */
     int32_t gather_cells;   /* ghost gather of cell variables */
     int32_t c2p;            /* c2p over cells */
-    int32_t flux_prefetch[3]; /* 1: face-flux kernel x/y/z loads its whole WENO-Z
-                               * stencil before reconstructing (more loads in
-                               * flight, fewer waves); 0 or 1, same results */
+    int32_t flux_prefetch[3]; /* 0 or 1; without effect (the flux kernel always
+                               * loads ahead of its reconstruction) */
 } grmhd_tuning;
 
 /* Times each kernel family of one RK3 substep on the context's own block
