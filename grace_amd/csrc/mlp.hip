@@ -101,136 +101,175 @@ __global__ __launch_bounds__(256) void k_mlp_forward(int64_t n, MlpDev w, const 
 }
 
 // ---------------------------------------------------------------------------
-// Loss gradient of one 64-state chunk per workgroup (one wave).
+// Loss gradient, 64-state chunks over workgroups of four waves.
 // loss = inv_n * sum_s sum_j m_sj (y_sj - t_sj)^2 in normalised units, with
 // m_sj = 0 for NaN targets and states beyond n.  Forward: the MFMA tiles of
-// the inference path (bf16 operands, FP32 accumulation).  Backward in FP32:
+// the inference path (bf16 operands, FP32 accumulation), 16 states a wave.
+// Backward in FP32:
 //   d3 = 2 m (y - t) inv_n
 //   dz2 = (d3 W3q^T) [h2 > 0]        dz1 = (dz2 W2q^T) [h1 > 0]
 //   dW3 = bf(h2)^T d3   dW2 = bf(h1)^T dz2   dW1 = bf(x)^T dz1   db = sums
 // with Wq the bf16-rounded weights and bf() the bf16 rounding the forward
-// applied to each layer input.  Partial sums go to part[wg][MLP_NP + 1]
-// (last entry: loss).
+// applied to each layer input.  The products are FP32 matrix instructions
+// (v_mfma_f32_16x16x4_f32: FP32 operands, products and sums): wave w owns the
+// rows 16w.. of dW2 and dW3 and the columns 16w.. of dz1 and dW1.  A
+// contraction step takes the four indices s, s + 16, s + 32, s + 48: with a
+// row stride of 65 floats the operands of either orientation then lie in 64
+// different banks.  A workgroup runs over the chunks blockIdx.x + i gridDim.x
+// and keeps its sums in registers; they go to part[wg][MLP_NP + 1] (last
+// entry: loss).
+//
+// Bound by latency: a chunk is some 5000 cycles of matrix instructions per
+// SIMD between five barriers.  With k_mlp_reduce 12.6 us for 4096 states,
+// against 66.8 with one wave per chunk that kept a row of every product per
+// lane, and one thread per column of the sum.
 // ---------------------------------------------------------------------------
 constexpr int HS = MLP_H + 1;   // LDS row stride (floats) of the [64][64] tiles
+// Workgroups of k_mlp_grad: two on a compute unit; more would only add
+// partial sums to write and read (21 KB each).
+constexpr int64_t MLP_GRAD_WG = 512;
 
-__global__ __launch_bounds__(64) void k_mlp_grad(int64_t n, int64_t ld, MlpDev w, const float* __restrict__ wq,
-                                                 const float* __restrict__ w2t, const float* __restrict__ feat,
-                                                 const float* __restrict__ target, float inv_n,
-                                                 float* __restrict__ part) {
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(256) void k_mlp_grad(int64_t n, int64_t ld, MlpDev w, const float* __restrict__ wq,
+                                                  const float* __restrict__ w2t, const float* __restrict__ feat,
+                                                  const float* __restrict__ target, float inv_n,
+                                                  float* __restrict__ part) {
     __shared__ __align__(16) uint16_t xs[64 * MLP_KP];
     __shared__ float H1[64 * HS];
     __shared__ float H2[64 * HS];     // reused for dz1 once dW3 is formed
     __shared__ float DZ2[64 * HS];
-    __shared__ float D3[64 * 2];
-    const int l = threadIdx.x;
-    const int64_t s = (int64_t)blockIdx.x * 64 + l;
-    const bool act = s < n;
-    float f[MLP_NF];
-    for (int k = 0; k < MLP_NF; ++k) f[k] = act ? feat[k * ld + s] : w.norm[k];
-    mlp_stage_features(w, f, xs);
-    __syncthreads();
+    __shared__ float Y[64 * 2], D3[64 * 2];
+    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, li = l & 15, lq = l >> 4, rowoff = 4 * lq;
     bf16x4 A[MLP_NFRAG];
     mlp_load_frags(w, A);
     MlpBias b;
     mlp_load_bias(w, b);
-    const int rowoff = 4 * (l >> 4);
-    for (int t = 0; t < 4; ++t) {
-        const uint2 xv = *reinterpret_cast<const uint2*>(xs + (t * 16 + (l & 15)) * MLP_KP + rowoff);
-        f32x4 h1[4], h2[4];
-        f32x4 o = mlp_tile<true>(A, b, as_bf16x4(xv), h1, h2);
-        const int st = t * 16 + (l & 15);
-        for (int jb = 0; jb < 4; ++jb)
-            for (int e = 0; e < 4; ++e) {
-                H1[st * HS + jb * 16 + rowoff + e] = h1[jb][e];
-                H2[st * HS + jb * 16 + rowoff + e] = h2[jb][e];
+    float w2b[16];                    // this wave's 16 columns of W2q^T
+#pragma unroll
+    for (int t = 0; t < 16; ++t) w2b[t] = w2t[(t + 16 * lq) * MLP_H + wv * 16 + li];
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 gW2[4] = {zero, zero, zero, zero}, gW1 = zero, gW3 = zero;
+    float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, loss = 0.0f;
+    for (int64_t c0 = (int64_t)blockIdx.x * 64; c0 < n; c0 += (int64_t)gridDim.x * 64) {
+        const int64_t s = c0 + l;
+        const bool act = s < n;
+        if (wv == 0) {
+            float f[MLP_NF];
+            for (int k = 0; k < MLP_NF; ++k) f[k] = act ? feat[k * ld + s] : w.norm[k];
+            mlp_stage_features(w, f, xs);
+        }
+        float tv[2];
+        for (int j = 0; j < 2; ++j) tv[j] = act ? target[j * ld + s] : NAN;
+        __syncthreads();
+        {
+            const int st = wv * 16 + li;
+            const uint2 xv = *reinterpret_cast<const uint2*>(xs + st * MLP_KP + rowoff);
+            f32x4 h1[4], h2[4];
+            const f32x4 o = mlp_tile<true>(A, b, as_bf16x4(xv), h1, h2);
+#pragma unroll
+            for (int jb = 0; jb < 4; ++jb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    H1[st * HS + jb * 16 + rowoff + e] = h1[jb][e];
+                    H2[st * HS + jb * 16 + rowoff + e] = h2[jb][e];
+                }
+            if (l < 16) { Y[st * 2] = o[0]; Y[st * 2 + 1] = o[1]; }
+        }
+        __syncthreads();
+        // output error of the state of this lane (every wave), then this
+        // wave's 16 columns of dz2
+        float d3[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const float tn = (tv[j] - w.norm[2 * MLP_NF + j]) / w.norm[2 * MLP_NF + 2 + j];
+            const float d = act && (tv[j] == tv[j]) ? Y[l * 2 + j] - tn : 0.0f;
+            if (wv == 0) loss += d * d * inv_n;
+            d3[j] = 2.0f * d * inv_n;
+            if (wv == j) { D3[l * 2 + j] = d3[j]; gb3 += d3[j]; }
+        }
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const int k = wv * 16 + t;
+            const float dh = d3[0] * wq[MLP_W3 + k * MLP_NO] + d3[1] * wq[MLP_W3 + k * MLP_NO + 1];
+            DZ2[l * HS + k] = dh * mlp_act_slope(H2[l * HS + k]);
+        }
+        __syncthreads();
+        // rows 16 wv.. of dW3 and dW2, columns 16 wv.. of dz1 (all states)
+        f32x4 z[4] = {zero, zero, zero, zero};
+        float sb = 0.0f;
+#pragma unroll 4
+        for (int t = 0; t < 16; ++t) {
+            const int st = t + 16 * lq;
+            const float h1 = bf2f(f2bf(H1[st * HS + wv * 16 + li])), h2 = bf2f(f2bf(H2[st * HS + wv * 16 + li]));
+            gW3 = mfma_f32(h2, li < MLP_NO ? D3[st * 2 + li] : 0.0f, gW3);
+#pragma unroll
+            for (int jb = 0; jb < 4; ++jb) {
+                const float dz = DZ2[st * HS + jb * 16 + li];
+                if (jb == wv) sb += dz;
+                gW2[jb] = mfma_f32(h1, dz, gW2[jb]);
             }
-        if (l < 16) { D3[st * 2] = o[0]; D3[st * 2 + 1] = o[1]; }
-    }
-    __syncthreads();
-    // per-state output error (lane = state)
-    float loss = 0.0f, d3[2];
-    for (int j = 0; j < 2; ++j) {
-        float tv = act ? target[j * ld + s] : NAN;
-        float y = D3[l * 2 + j];
-        float tn = (tv - w.norm[2 * MLP_NF + j]) / w.norm[2 * MLP_NF + 2 + j];
-        bool ok = act && (tv == tv);
-        float d = ok ? (y - tn) : 0.0f;
-        loss += d * d * inv_n;
-        d3[j] = 2.0f * d * inv_n;
-    }
-    __syncthreads();
-    D3[l * 2] = d3[0]; D3[l * 2 + 1] = d3[1];
-    for (int k = 0; k < MLP_H; ++k) {
-        float h = H2[l * HS + k];
-        float dh = d3[0] * wq[MLP_W3 + k * MLP_NO] + d3[1] * wq[MLP_W3 + k * MLP_NO + 1];
-        DZ2[l * HS + k] = dh * mlp_act_slope(h);
-    }
-    __syncthreads();
-    float* P = part + (int64_t)blockIdx.x * (MLP_NP + 1);
-    // thread l owns row l of W3/W2 and column l of W1
-    {
-        float g0 = 0.0f, g1 = 0.0f;
-        for (int st = 0; st < 64; ++st) {
-            float h = bf2f(f2bf(H2[st * HS + l]));
-            g0 += h * D3[st * 2]; g1 += h * D3[st * 2 + 1];
         }
-        P[MLP_W3 + l * MLP_NO] = g0; P[MLP_W3 + l * MLP_NO + 1] = g1;
-        if (l < MLP_NO) {
-            float gb = 0.0f;
-            for (int st = 0; st < 64; ++st) gb += D3[st * 2 + l];
-            P[MLP_B3 + l] = gb;
-        }
-        float gw[MLP_H];
-        for (int j = 0; j < MLP_H; ++j) gw[j] = 0.0f;
-        float gb2 = 0.0f;
-        for (int st = 0; st < 64; ++st) {
-            float h = bf2f(f2bf(H1[st * HS + l]));
-            gb2 += DZ2[st * HS + l];
-            for (int j = 0; j < MLP_H; ++j) gw[j] += h * DZ2[st * HS + j];
-        }
-        for (int j = 0; j < MLP_H; ++j) P[MLP_W2 + l * MLP_H + j] = gw[j];
-        P[MLP_B2 + l] = gb2;
-    }
-    __syncthreads();
-    // dz1 of this lane's state into the H2 buffer
-    {
-        float acc[MLP_H];
-        for (int k = 0; k < MLP_H; ++k) acc[k] = 0.0f;
-        for (int j = 0; j < MLP_H; ++j) {
-            float dz = DZ2[l * HS + j];
-            for (int k = 0; k < MLP_H; ++k) acc[k] += dz * w2t[j * MLP_H + k];
-        }
-        for (int k = 0; k < MLP_H; ++k) {
-            float h = H1[l * HS + k];
-            H2[l * HS + k] = acc[k] * mlp_act_slope(h);
-        }
-    }
-    __syncthreads();
-    {
-        float gw[MLP_KP], gb1 = 0.0f;
-        for (int k = 0; k < MLP_KP; ++k) gw[k] = 0.0f;
-        for (int st = 0; st < 64; ++st) {
-            float dz = H2[st * HS + l];
+        gb2 += sb;
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+#pragma unroll
+            for (int sb4 = 0; sb4 < 4; ++sb4) z[sb4] = mfma_f32(DZ2[(sb4 * 16 + li) * HS + t + 16 * lq], w2b[t], z[sb4]);
+        __syncthreads();
+        // dz1 of every state, this wave's columns, into the H2 buffer
+#pragma unroll
+        for (int sb4 = 0; sb4 < 4; ++sb4)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int at = (sb4 * 16 + rowoff + e) * HS + wv * 16 + li;
+                H2[at] = z[sb4][e] * mlp_act_slope(H1[at]);
+            }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const int st = t + 16 * lq;
+            const float dz = H2[st * HS + wv * 16 + li];
             gb1 += dz;
-            for (int k = 0; k < MLP_NF; ++k) gw[k] += bf2f(xs[st * MLP_KP + k]) * dz;
+            gW1 = mfma_f32(bf2f(xs[st * MLP_KP + li]), dz, gW1);
         }
-        for (int k = 0; k < MLP_KP; ++k) P[MLP_W1 + k * MLP_H + l] = gw[k];
-        P[MLP_B1 + l] = gb1;
+        __syncthreads();              // xs, H2 and D3 are rewritten by the next chunk
     }
-    // loss: wave sum
-    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
-    if (l == 0) P[MLP_NP] = loss;
+    float* P = part + (int64_t)blockIdx.x * (MLP_NP + 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int r = rowoff + e, k = wv * 16 + r;
+#pragma unroll
+        for (int jb = 0; jb < 4; ++jb) P[MLP_W2 + k * MLP_H + jb * 16 + li] = gW2[jb][e];
+        P[MLP_W1 + r * MLP_H + wv * 16 + li] = r < MLP_NF ? gW1[e] : 0.0f;
+        if (li < MLP_NO) P[MLP_W3 + k * MLP_NO + li] = gW3[e];
+    }
+    // column sums: the four lanes of a column
+    for (int off = 16; off < 64; off <<= 1) { gb1 += __shfl_xor(gb1, off); gb2 += __shfl_xor(gb2, off); }
+    if (l < 16) { P[MLP_B1 + wv * 16 + l] = gb1; P[MLP_B2 + wv * 16 + l] = gb2; }
+    for (int off = 32; off > 0; off >>= 1) { loss += __shfl_xor(loss, off); gb3 += __shfl_xor(gb3, off); }
+    if (l == 0 && wv < MLP_NO) P[MLP_B3 + wv] = gb3;
+    if (threadIdx.x == 0) P[MLP_NP] = loss;
 }
 
-// grad[p] = sum over workgroups in index order (deterministic)
-__global__ __launch_bounds__(256) void k_mlp_reduce(int64_t nwg, const float* __restrict__ part,
-                                                    float* __restrict__ grad) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > MLP_NP) return;
+// grad[p] = sum over workgroups, in an order that depends on their number
+// alone (deterministic): 32 columns a workgroup (128 bytes of a row), eight
+// threads per column over every eighth row, then the eight.
+__global__ __launch_bounds__(256) void k_mlp_reduce(int nwg, const float* __restrict__ part, float* __restrict__ grad) {
+    __shared__ float S[8][32];
+    const int c = threadIdx.x & 31, r = threadIdx.x >> 5, p = blockIdx.x * 32 + c;
     float acc = 0.0f;
-    for (int64_t w = 0; w < nwg; ++w) acc += part[w * (MLP_NP + 1) + p];
-    grad[p] = acc;
+    if (p <= MLP_NP) {
+#pragma unroll 8
+        for (int g = r; g < nwg; g += 8) acc += part[(int64_t)g * (MLP_NP + 1) + p];
+    }
+    S[r][c] = acc;
+    __syncthreads();
+    if (r == 0 && p <= MLP_NP) {
+        for (int t = 1; t < 8; ++t) acc += S[t][c];
+        grad[p] = acc;
+    }
 }
 
 __global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ grad, float* master, float* m, float* v,
@@ -413,15 +452,15 @@ extern "C" grmhd_status grmhd_mlp_targets(int64_t n, const double* roots, const 
 
 static grmhd_status grad_into(grmhd_mlp* m, int64_t n, int64_t ld, const float* feat, const float* target,
                               float* grad, hipStream_t s) {
-    const int64_t nwg = (n + 63) / 64;
+    const int64_t nwg = std::min((n + 63) / 64, MLP_GRAD_WG);
     if (nwg > m->part_cap) {
         if (m->part) (void)hipFree(m->part);
         m->part = nullptr; m->part_cap = 0;
         MHIP_TRY(hipMalloc(&m->part, sizeof(float) * (MLP_NP + 1) * nwg));
         m->part_cap = nwg;
     }
-    k_mlp_grad<<<(unsigned)nwg, 64, 0, s>>>(n, ld, m->dev(), m->wq, m->w2t, feat, target, 1.0f / (float)n, m->part);
-    k_mlp_reduce<<<(MLP_NP + 1 + 255) / 256, 256, 0, s>>>(nwg, m->part, grad);
+    k_mlp_grad<<<(unsigned)nwg, 256, 0, s>>>(n, ld, m->dev(), m->wq, m->w2t, feat, target, 1.0f / (float)n, m->part);
+    k_mlp_reduce<<<(MLP_NP + 1 + 31) / 32, 256, 0, s>>>((int)nwg, m->part, grad);
     return mlaunch_check("mlp_grad");
 }
 

@@ -123,6 +123,33 @@ def test_gpu_mlp_grad_matches_oracle(dev):
     assert np.all(gg[M.W1 + 10 * 64:M.B1] == 0)
 
 
+@pytest.mark.parametrize("n", [1, 17, 64, 65, 512 * 64, 513 * 64 + 7])
+def test_gpu_mlp_grad_chunk_edges(dev, n):
+    """One state, one chunk of 64 and its neighbours, one chunk for every
+    workgroup of the largest launch, and workgroups with a second, partly
+    filled chunk: the oracle's gradient at the bound above, and the same bits
+    from a second call."""
+    import torch
+    st, feat, p, scale, target = problem(max(n, 64), 21)   # (one state has no scaling of its own)
+    feat, target = np.ascontiguousarray(feat[:, :n]), np.ascontiguousarray(target[:, :n])
+    mlp = ga.Mlp()
+    mlp.set_params(p)
+    mlp.set_scaling(scale)
+    fd, td = to_dev(feat, dev), to_dev(target, dev)
+    g = [torch.full((ga.MLP_NPARAM + 1,), float("nan"), dtype=torch.float32, device=dev) for _ in range(2)]
+    for out in g:
+        mlp.grad(n, fd, td, out)
+    torch.cuda.synchronize()
+    assert torch.equal(g[0], g[1])
+    gg = to_host(g[0]).astype(np.float64)
+    ref, loss = M.grad(p, scale, feat, target, quant=True)
+    assert abs(gg[-1] - loss) < 1e-3 * loss + 1e-6
+    for name, a, b in (("W1", M.W1, M.B1), ("b1", M.B1, M.W2), ("W2", M.W2, M.B2), ("b2", M.B2, M.W3),
+                       ("W3", M.W3, M.B3), ("b3", M.B3, M.NP)):
+        assert np.linalg.norm(gg[a:b] - ref[a:b]) <= 2e-2 * np.linalg.norm(ref[a:b]), name
+    assert np.all(gg[M.W1 + 10 * 64:M.B1] == 0)
+
+
 def test_gpu_mlp_adam_step(dev):
     """One train_step equals Adam (0.9, 0.999, 1e-8, bias-corrected) applied
     to the gradient the library reports for the same batch."""
