@@ -796,7 +796,7 @@ __global__ __launch_bounds__(256) void k_fofc_flag(DevGrid G, EOS eos, Opts o, F
     C2PGuess gs{0, 0, 0, 0, 0, 0};
     C2PRoots rt{-1, -1, -1, -1};
     const double rad = o.ex.by_radius ? cell_radius(o.ex, I, a.blk[q].b, G.n, G.ng, i, j, k) : 1e300;
-    const C2POut out = c2p(cons, pr, m, eos, o.atmo, o.ex, cp, rad, err, true, cnt, gs, rt);
+    const C2POut out = c2p<FLAT>(cons, pr, m, eos, o.atmo, o.ex, cp, rad, err, true, cnt, gs, rt);
     if (!(out.floored || dmp)) return;
     for (int t = 0; t < 2; ++t) {
         a.ftag[0][q * nf0 + fidx<0>(G, i + t, j, k)] = 1;
@@ -1153,7 +1153,7 @@ __global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_cells(DevGrid G, EO
         A[BX_ * nc] = Bc0 / m.sqrtg; A[BY_ * nc] = Bc1 / m.sqrtg; A[BZ_ * nc] = Bc2 / m.sqrtg;
         C2PRoots rt{-1, -1, -1, -1};
         const double rad = o.ex.by_radius ? cell_radius(o.ex, inst[blk[q].inst], blk[q].b, G.n, G.ng, i, j, k) : 1e300;
-        out = c2p(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad, err, false, cnt, gs, rt);
+        out = c2p<FLAT>(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad, err, false, cnt, gs, rt);
         if (out.fatal && o.fatal_count) atomicAdd(o.fatal_count, 1ull);
         A[RHO_ * nc] = pr[RHOL]; A[EPS_ * nc] = pr[EPSL]; A[PRESS_ * nc] = pr[PRESSL];
         A[TEMP_ * nc] = pr[TEMPL]; A[ENTROPY_ * nc] = pr[ENTL]; A[YE_ * nc] = pr[YEL];
@@ -1240,7 +1240,7 @@ __global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_batch(int64_t n, EO
     C2PCount cnt;
     C2POut out{false, false};
     if (active) {
-        out = c2p(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad ? rad[s] : 1e300, err, dry_run != 0, cnt, gs, rt);
+        out = c2p<false>(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad ? rad[s] : 1e300, err, dry_run != 0, cnt, gs, rt);
         if (out.fatal && o.fatal_count) atomicAdd(o.fatal_count, 1ull);
         if (roots) { roots[s] = rt.x_e; roots[n + s] = rt.x_s; roots[2 * n + s] = rt.m_e; roots[3 * n + s] = rt.m_s; }
         for (int v = 0; v < NPRIM; ++v) prims[v * n + s] = pr[v];

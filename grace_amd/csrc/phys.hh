@@ -53,13 +53,25 @@ GHD double sq(double x) { return x * x; }
 GHD double nr_rcp(double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
     double r = __builtin_amdgcn_rcp(b);
-#else
-    double r = 1.0 / b;
-#endif
     double e = fma(-b, r, 1.0);
     r = fma(e, r, r);
     e = fma(-b, r, 1.0);
     return fma(e, r, r);
+#else
+    return 1.0 / b;
+#endif
+}
+// a / b from a reciprocal ib of b good to a few ulp, shared by several
+// quotients: one correction by the remainder (half an ulp but for ties), and
+// the hardware's fixup for zero, infinite and NaN operands, which gives what
+// an IEEE division does.
+GHD double quot(double a, double b, double ib) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double q = a * ib;
+    return __builtin_amdgcn_div_fixup(fma(fma(-b, q, a), ib, q), b, a);
+#else
+    return a / b;
+#endif
 }
 // sqrt(x) and 1/sqrt(x) for a normal, finite x > 0: the hardware's reciprocal
 // root (about 24 bits) and two coupled Newton steps, the last one on the
@@ -68,9 +80,6 @@ GHD double nr_rcp(double b) {
 GHD void nr_sqrt(double x, double& g, double& ig) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const double y = __builtin_amdgcn_rsq(x);
-#else
-    const double y = 1.0 / sqrt(x);
-#endif
     double h = 0.5 * y;
     g = x * y;
     double r = fma(-g, h, 0.5);
@@ -79,6 +88,10 @@ GHD void nr_sqrt(double x, double& g, double& ig) {
     g = fma(fma(-g, g, x), h, g);
     r = fma(-g, h, 0.5);
     ig = 2.0 * fma(h, r, h);
+#else
+    g = sqrt(x);
+    ig = 1.0 / g;
+#endif
 }
 // ---- 3-metric -------------------------------------------------------------
 struct Met {
@@ -148,6 +161,14 @@ struct EosIdeal {
         double p = gm1 * eps * rho;
         h = 1.0 + gamma * eps; temp = eps * gm1; cs2 = ggm1 * eps / h;
         return p;
+    }
+    // eps of press_full_ent alone
+    GHD double eps_from_ent(double ent, double rho, bool* clamped = nullptr) const {
+        const double lr = log(rho), smin = ls_min - lr, smax = ls_max - lr;
+        if (clamped) *clamped = ent < smin || ent > smax;
+        if (ent < smin) ent = smin;
+        if (ent > smax) ent = smax;
+        return exp(gm1 * (ent + lr));
     }
     // press_eps_csnd2_entropy__temp_rho_ye
     GHD double press_from_temp_ent(double& eps, double& cs2, double& ent, double& temp, double rho,
@@ -341,25 +362,38 @@ GHD void lower3(const double g[6], double x, double y, double z, double o[3]) {
         o[2] = g[2] * x + g[4] * y + g[5] * z;
     }
 }
+// v^i v_i and s_i s^i
+template <bool FL>
+GHD double norm_up(const Met& m, double x, double y, double z) {
+    if constexpr (FL) return x * x + y * y + z * z;
+    else return m.sqv(x, y, z);
+}
+template <bool FL>
+GHD double norm_low(const Met& m, double x, double y, double z) {
+    if constexpr (FL) return x * x + y * y + z * z;
+    else return m.sqcov(x, y, z);
+}
 template <bool FL = false>
 GHD double lorentz(const double g[6], const double z[3]) {
-    double zl[3]; lower3<FL>(g, z[0], z[1], z[2], zl);
-    return sqrt(z[0] * zl[0] + z[1] * zl[1] + z[2] * zl[2] + 1);
+    double zl[3], W, iW; lower3<FL>(g, z[0], z[1], z[2], zl);
+    nr_sqrt(z[0] * zl[0] + z[1] * zl[1] + z[2] * zl[2] + 1, W, iW);
+    return W;
 }
 template <bool FL = false>
 GHD void smallb(const Met& m, const double B[3], const double z[3], double W, double b[4], double& b2) {
     double zl[3]; lower3<FL>(m.g, z[0], z[1], z[2], zl);
     double Bz = B[0] * zl[0] + B[1] * zl[1] + B[2] * zl[2];
-    double iW = 1. / W;
+    const double iW = nr_rcp(W);
     if constexpr (FL) {
         b[0] = Bz;
         for (int i = 0; i < 3; ++i) b[1 + i] = iW * (B[i] + Bz * z[i]);
     } else {
-        b[0] = Bz / m.alp;
-        for (int i = 0; i < 3; ++i) b[1 + i] = iW * (B[i] + Bz * (z[i] - W * m.beta[i] / m.alp));
+        const double ia = nr_rcp(m.alp);
+        b[0] = quot(Bz, m.alp, ia);
+        for (int i = 0; i < 3; ++i) b[1 + i] = iW * (B[i] + Bz * (z[i] - quot(W * m.beta[i], m.alp, ia)));
     }
     double Bl[3]; lower3<FL>(m.g, B[0], B[1], B[2], Bl);
-    b2 = (B[0] * Bl[0] + B[1] * Bl[1] + B[2] * Bl[2] + Bz * Bz) / (W * W);
+    b2 = quot(B[0] * Bl[0] + B[1] * Bl[1] + B[2] * Bl[2] + Bz * Bz, W * W, iW * iW);
 }
 GHD void vtilde(const Met& m, const double z[3], double W, double vt[3]) {
     double iW = 1. / W;
@@ -420,16 +454,19 @@ __host__ __device__ inline double brent_fab(F& f, double a, double b, double fa,
         if (fabs(mm) <= tol || fb == 0.0) break;
         if (fabs(e) < tol || fabs(fa) <= fabs(fb)) { e = mm; d = e; }
         else {
-            double s = fb / fa, p, q;
+            // (fa, fc: non-zero here; the quotients only shape the step)
+            const double iac = nr_rcp(fa * fc);
+            double s = fb * (fc * iac), p, q;
             if (sa == c) { p = 2.0 * mm * s; q = 1.0 - s; }
             else {
-                double qq = fa / fc, r = fb / fc;
+                const double ic = fa * iac;
+                double qq = fa * ic, r = fb * ic;
                 p = s * (2.0 * mm * qq * (qq - r) - (sb - sa) * (r - 1.0));
                 q = (qq - 1.0) * (r - 1.0) * (s - 1.0);
             }
             if (0.0 < p) q = -q; else p = -p;
             s = e; e = d;
-            if (2.0 * p < 3.0 * mm * q - fabs(tol * q) && p < fabs(0.5 * s * q)) d = p / q;
+            if (2.0 * p < 3.0 * mm * q - fabs(tol * q) && p < fabs(0.5 * s * q)) d = p * nr_rcp(q);
             else { e = mm; d = e; }
         }
         sa = sb; fa = fb;
@@ -458,7 +495,7 @@ __host__ __device__ inline double newton_br(double sa, double sb, F& f, int maxi
     do {
         xold = x; f(x, fx, dfx);
         if (fx * fb > 0) { fb = fx; b = x; } else if (fx * fa > 0) { fa = fx; a = x; }
-        x -= fx / dfx;
+        x -= fx * nr_rcp(dfx);
         t = 2. * macheps * fabs(x) + tol;
         if (fabs(x - xold) < t || fx == 0) { err = 0; return x; }
         if (x > b || x < a) x = 0.5 * (b + a);
@@ -471,16 +508,22 @@ __host__ __device__ inline double newton_br(double sa, double sb, F& f, int maxi
 // ---- Kastaun master functions ----------------------------------------------------
 struct FBr {
     double rsqr, bsqr, rbsqr, h0sqr; int* cnt;
-    GHD double xm(double mu) const { return 1. / (1. + mu * bsqr); }
+    GHD double xm(double mu) const { return nr_rcp(1. + mu * bsqr); }
     GHD double rb(double mu, double x) const { return x * (rsqr * x + mu * (x + 1.0) * rbsqr); }
     GHD void operator()(double mu, double& f, double& df) {
         (*cnt)++;
         double x = xm(mu), x2 = x * x;
-        double hw = sqrt(h0sqr + rb(mu, x));
+        double hw, ihw;
+        nr_sqrt(h0sqr + rb(mu, x), hw, ihw);
         double bb = x * (x2 * rsqr + mu * (1 + x + x2) * rbsqr);
-        f = mu * hw - 1.; df = (h0sqr + bb) / hw;
+        f = mu * hw - 1.; df = (h0sqr + bb) * ihw;
     }
-    GHD double operator()(double mu) { (*cnt)++; double x = xm(mu); return mu * sqrt(h0sqr + rb(mu, x)) - 1.; }
+    GHD double operator()(double mu) {
+        (*cnt)++;
+        double hw, ihw;
+        nr_sqrt(h0sqr + rb(mu, xm(mu)), hw, ihw);
+        return mu * hw - 1.;
+    }
     GHD void bracket(double& lo, double& hi) const {
         lo = 1. / (h0sqr + rsqr);
         double mu0 = 1. / sqrt(h0sqr);
@@ -493,20 +536,37 @@ struct FBr {
 template <typename EOS>
 struct FMu {
     const EOS& eos;
-    double d, qtot, rsqr, bsqr, rbsqr, brosqr, vsqrmax, wmax; int* cnt;
+    double d, qtot, rsqr, bsqr, rbsqr, brosqr, vsqrmax, wmax, iwmax; int* cnt;
     GHD FMu(const EOS& e, double d_, double q_, double r2, double rb2, double b2, double h0, int* c)
         : eos(e), d(d_), qtot(q_), rsqr(r2), bsqr(b2), rbsqr(rb2), brosqr(r2 * b2 - rb2), cnt(c) {
         double zs = rsqr / (h0 * h0), ws = 1 + zs;
-        wmax = sqrt(ws); vsqrmax = zs / ws;
+        nr_sqrt(ws, wmax, iwmax);
+        vsqrmax = zs / ws;
     }
-    GHD double xm(double mu) const { return 1. / (1. + mu * bsqr); }
+    GHD double xm(double mu) const { return nr_rcp(1. + mu * bsqr); }
     GHD double rf(double mu, double x) const { return x * (rsqr * x + mu * (x + 1.0) * rbsqr); }
     GHD double qf(double mu, double x) const { double mx = mu * x; return qtot - 0.5 * (bsqr + mx * mx * brosqr); }
     GHD double epsraw(double mu, double q, double r, double w) const { return w * (q - mu * r * (1.0 - mu * w / (1 + w))); }
+    // Ideal gas: rho cancels from a = p / (rho (1 + eps)) = (gamma - 1) eps /
+    // (1 + eps), and h = (1 + eps)(1 + a) = 1 + gamma eps, so that three
+    // reciprocals and one root are left of nine divisions and one; the
+    // quotient that the root's last digits come from is corrected by its
+    // remainder.
     GHD double operator()(double mu) {
         (*cnt)++;
         double x = xm(mu), r = rf(mu, x), q = qf(mu, x);
         double vs = r * mu * mu, w;
+        if constexpr (EOS::is_ideal) {
+            double iw;
+            nr_sqrt(fmax(1 - vs, 1e-280), iw, w);
+            if (vs > vsqrmax) { w = wmax; iw = iwmax; }
+            const double rm = mu * r;
+            double eps = w * (q - rm * (1.0 - mu * nr_rcp(1 + iw)));
+            eps = fmin(eos.eps_max, fmax(0.0, eps));
+            const double e1 = 1 + eps, h = fma(eos.gm1, eps, e1);
+            const double den = h * fmax(1 + q - rm, iw * e1) + rm * e1, i = nr_rcp(den), k = e1 * i;
+            return mu - fma(fma(-den, k, e1), i, k);
+        }
         if (vs > vsqrmax) { w = wmax; } else w = 1 / sqrt(1 - vs);
         double rho = fmin(eos.rhomax(), fmax(eos.rhomin(), d / w));
         double eps = epsraw(mu, q, r, w);
@@ -528,26 +588,24 @@ struct FMu {
         const double r = rf(mu, x), dr = 2.0 * rsqr * x * dx + rbsqr * (x * (x + 1.0) + mu * dx * (2.0 * x + 1.0));
         const double mx = mu * x, q = qf(mu, x), dq = -mx * (x + mu * dx) * brosqr;
         const double vs = r * mu * mu, dvs = dr * mu * mu + 2.0 * r * mu;
-        double w, dw;
-        if (vs > vsqrmax) { w = wmax; dw = 0.0; } else { w = 1 / sqrt(1 - vs); dw = 0.5 * w * w * w * dvs; }
-        const double rho = fmin(eos.rhomax(), fmax(eos.rhomin(), d / w));
-        const double i1w = 1.0 / (1.0 + w);
+        double w, iw, dw;
+        nr_sqrt(fmax(1 - vs, 1e-280), iw, w);
+        dw = 0.5 * w * w * w * dvs;
+        if (vs > vsqrmax) { w = wmax; iw = iwmax; dw = 0.0; }
+        const double i1w = nr_rcp(1.0 + w);
         const double u = mu * w * i1w, du = (w * (1.0 + w) + mu * dw) * i1w * i1w;
         const double g = mu * r * (1.0 - u), dg = (r + mu * dr) * (1.0 - u) - mu * r * du;
         double eps = w * (q - g), deps = dw * (q - g) + w * (dq - dg);
-        double emin, emax; eos.eps_range(emin, emax, rho);
-        if (eps > emax || eps < emin) deps = 0.0;
-        eps = fmin(emax, fmax(emin, eps));
-        unsigned ee = 0;
-        const double p = eos.press_eps(eps, rho, ee);
-        const double i1e = 1.0 / (1 + eps);
-        const double a = p / (rho * (1 + eps)), da = eos.gm1 * deps * i1e * i1e;
-        const double h = (1 + eps) * (1 + a), dh = deps * (1 + a) + (1 + eps) * da;
-        const double A = (1 + a) * (1 + q - mu * r), B = h / w;
+        if (eps > eos.eps_max || eps < 0.0) deps = 0.0;
+        eps = fmin(eos.eps_max, fmax(0.0, eps));
+        const double i1e = nr_rcp(1 + eps);
+        const double a = eos.gm1 * eps * i1e, da = eos.gm1 * deps * i1e * i1e;
+        const double h = 1 + eos.gamma * eps, dh = eos.gamma * deps;
+        const double A = (1 + a) * (1 + q - mu * r), B = h * iw;
         double hbw, dhbw;
         if (A >= B) { hbw = A; dhbw = da * (1 + q - mu * r) + (1 + a) * (dq - r - mu * dr); }
-        else { hbw = B; dhbw = (dh - h * dw / w) / w; }
-        const double den = hbw + r * mu, iden = 1.0 / den;
+        else { hbw = B; dhbw = (dh - h * dw * iw) * iw; }
+        const double den = hbw + r * mu, iden = nr_rcp(den);
         f = mu - iden;
         df = 1.0 + (dhbw + r + mu * dr) * iden * iden;
     }
@@ -577,20 +635,26 @@ struct FMu {
 template <typename EOS>
 struct FMuEnt {
     const EOS& eos;
-    double d, s, rsqr, bsqr, rbsqr, vsqrmax, wmax; int* cnt;
+    double d, s, rsqr, bsqr, rbsqr, vsqrmax, wmax, iwmax; int* cnt;
     GHD FMuEnt(const EOS& e, double d_, double r2, double rb2, double b2, double s_, double h0, int* c)
         : eos(e), d(d_), s(s_), rsqr(r2), bsqr(b2), rbsqr(rb2), cnt(c) {
         double zs = rsqr / (h0 * h0), ws = 1 + zs;
-        wmax = sqrt(ws); vsqrmax = zs / ws;
+        nr_sqrt(ws, wmax, iwmax);
+        vsqrmax = zs / ws;
     }
-    GHD double xm(double mu) const { return 1. / (1. + mu * bsqr); }
+    GHD double xm(double mu) const { return nr_rcp(1. + mu * bsqr); }
     GHD double rf(double mu, double x) const { return x * (rsqr * x + mu * (x + 1.0) * rbsqr); }
     GHD double operator()(double mu) {
         (*cnt)++;
         double x = xm(mu), r = rf(mu, x);
-        double vs = r * mu * mu, w = 1 / sqrt(1 - vs);
-        if (vs > vsqrmax) w = wmax;
-        double rho = fmin(eos.rhomax(), fmax(eos.rhomin(), d / w));
+        double vs = r * mu * mu, w, iw;
+        nr_sqrt(fmax(1 - vs, 1e-280), iw, w);
+        if (vs > vsqrmax) { w = wmax; iw = iwmax; }
+        double rho = fmin(eos.rhomax(), fmax(eos.rhomin(), d * iw));
+        if constexpr (EOS::is_ideal) {
+            const double h = 1 + eos.gamma * eos.eps_from_ent(s, rho), den = h * iw + r * mu;
+            return mu - quot(1.0, den, nr_rcp(den));
+        }
         double hh, cs2, temp, eps, sl = s; unsigned ee = 0;
         double p = eos.press_full_ent(hh, cs2, temp, eps, sl, rho, ee);
         double a = p / (rho * (1 + eps));
@@ -604,20 +668,20 @@ struct FMuEnt {
         const double x = xm(mu), dx = -bsqr * x * x;
         const double r = rf(mu, x), dr = 2.0 * rsqr * x * dx + rbsqr * (x * (x + 1.0) + mu * dx * (2.0 * x + 1.0));
         const double vs = r * mu * mu, dvs = dr * mu * mu + 2.0 * r * mu;
-        double w = 1 / sqrt(1 - vs), dw = 0.5 * w * w * w * dvs;
-        if (vs > vsqrmax) { w = wmax; dw = 0.0; }
-        const double rr = d / w;
+        double w, iw;
+        nr_sqrt(fmax(1 - vs, 1e-280), iw, w);
+        double dw = 0.5 * w * w * w * dvs;
+        if (vs > vsqrmax) { w = wmax; iw = iwmax; dw = 0.0; }
+        const double rr = d * iw;
         const double rho = fmin(eos.rhomax(), fmax(eos.rhomin(), rr));
-        const double drho = (rr == rho) ? -rho * dw / w : 0.0;
-        double hh, cs2, temp, eps, sl = s; unsigned ee = 0;
-        const double p = eos.press_full_ent(hh, cs2, temp, eps, sl, rho, ee);
-        const double deps = (ee & (BIT(EOS_ENTROPY_TOO_LOW) | BIT(EOS_ENTROPY_TOO_HIGH))) ? 0.0 : eos.gm1 * eps * drho / rho;
-        const double i1e = 1.0 / (1 + eps);
-        const double a = p / (rho * (1 + eps)), da = eos.gm1 * deps * i1e * i1e;
-        const double h = (1 + eps) * (1 + a), dh = deps * (1 + a) + (1 + eps) * da;
-        const double den = h / w + r * mu, iden = 1.0 / den;
+        const double dlr = (rr == rho) ? -dw * iw : 0.0;   // d log rho
+        bool clamped;
+        const double eps = eos.eps_from_ent(s, rho, &clamped);
+        const double deps = clamped ? 0.0 : eos.gm1 * eps * dlr;
+        const double h = 1 + eos.gamma * eps, dh = eos.gamma * deps;
+        const double den = h * iw + r * mu, iden = nr_rcp(den);
         f = mu - iden;
-        df = 1.0 + ((dh - h * dw / w) / w + r + mu * dr) * iden * iden;
+        df = 1.0 + ((dh - h * dw * iw) * iw + r + mu * dr) * iden * iden;
     }
     GHD double prims(double mu, unsigned& sig, double& x, double& w, double& rho, double& press, double& eps,
                      double& temp, double& ent) {
@@ -642,29 +706,24 @@ struct FMuEnt {
 
 // Invariants of the undensitised conserved state shared by both inversions.
 struct C2PIn {
-    double D, q, s, ye, r2, Bt2, rBt, rBt2, h0;
+    double D, q, s, r2, Bt2, rBt, rBt2, h0;
     double r[3], Bt[3], B[3];
 };
-template <typename EOS>
+template <bool FL, typename EOS>
 GHD void c2p_setup(const EOS& eos, const Met& m, double cons[NCONS], C2PIn& c) {
     c.h0 = eos.hmin();
     cons[DENSL] = fmax(0., cons[DENSL]);
     c.D = cons[DENSL];
-    double iD = 1.0 / c.D;
-    c.q = cons[TAUL] / c.D;
-    c.s = cons[ENTSL] / c.D;
-    double rl0 = cons[STXL] / c.D, rl1 = cons[STYL] / c.D, rl2 = cons[STZL] / c.D;
-    (void)iD;
-    double sD = sqrt(c.D);
-    for (int i = 0; i < 3; ++i) { c.Bt[i] = cons[BSXL + i] / sD; c.B[i] = cons[BSXL + i]; }
-    c.r2 = m.sqcov(rl0, rl1, rl2);
-    c.Bt2 = m.sqv(c.Bt[0], c.Bt[1], c.Bt[2]);
+    const double iD = nr_rcp(c.D), sD = sqrt(c.D), isD = nr_rcp(sD);
+    c.q = quot(cons[TAUL], c.D, iD);
+    c.s = quot(cons[ENTSL], c.D, iD);
+    const double rl0 = quot(cons[STXL], c.D, iD), rl1 = quot(cons[STYL], c.D, iD), rl2 = quot(cons[STZL], c.D, iD);
+    for (int i = 0; i < 3; ++i) { c.Bt[i] = quot(cons[BSXL + i], sD, isD); c.B[i] = cons[BSXL + i]; }
+    c.r2 = norm_low<FL>(m, rl0, rl1, rl2);
+    c.Bt2 = norm_up<FL>(m, c.Bt[0], c.Bt[1], c.Bt[2]);
     c.rBt = rl0 * c.Bt[0] + rl1 * c.Bt[1] + rl2 * c.Bt[2];
     c.rBt2 = c.rBt * c.rBt;
-    c.r[0] = m.gi[0] * rl0 + m.gi[1] * rl1 + m.gi[2] * rl2;
-    c.r[1] = m.gi[1] * rl0 + m.gi[3] * rl1 + m.gi[4] * rl2;
-    c.r[2] = m.gi[2] * rl0 + m.gi[4] * rl1 + m.gi[5] * rl2;
-    c.ye = cons[YESL] / c.D;
+    lower3<FL>(m.gi, rl0, rl1, rl2, c.r);
 }
 
 struct C2PCount { int root = 0, bracket = 0; int guess_used = 0; };
@@ -884,28 +943,30 @@ GHD bool handle_eos_sig(unsigned e, bool lenient, uint64_t& err) {
 }
 
 // prims_to_conservs with W and b^mu of pr already at hand
+template <bool FL>
 GHD void p2c_wb(const double pr[NPRIM], double cons[NCONS], const Met& m, double W, const double b[4], double b2) {
     const double* z = &pr[ZXL];
     double D, tau, S[3], Ss;
-    conserved(m, pr[RHOL], pr[PRESSL], pr[EPSL], z, pr[ENTL], W, b2, b, D, tau, S, Ss);
+    conserved<FL>(m, pr[RHOL], pr[PRESSL], pr[EPSL], z, pr[ENTL], W, b2, b, D, tau, S, Ss);
     cons[DENSL] = m.sqrtg * D;
     cons[STXL] = m.sqrtg * S[0]; cons[STYL] = m.sqrtg * S[1]; cons[STZL] = m.sqrtg * S[2];
     cons[TAUL] = m.sqrtg * tau; cons[ENTSL] = m.sqrtg * Ss;
     cons[YESL] = cons[DENSL] * pr[YEL];
 }
+template <bool FL = false>
 GHD void p2c(const double pr[NPRIM], double cons[NCONS], const Met& m) {
-    double W = lorentz(m.g, &pr[ZXL]);
-    double b[4], b2; smallb(m, &pr[BXL], &pr[ZXL], W, b, b2);
-    p2c_wb(pr, cons, m, W, b, b2);
+    double W = lorentz<FL>(m.g, &pr[ZXL]);
+    double b[4], b2; smallb<FL>(m, &pr[BXL], &pr[ZXL], W, b, b2);
+    p2c_wb<FL>(pr, cons, m, W, b, b2);
 }
 
-template <typename EOS>
+template <bool FL, typename EOS>
 GHD void atmo_reset(double cons[NCONS], double pr[NPRIM], const Met& m, const Atmo& at, const EOS& eos, uint64_t& err) {
     pr[RHOL] = at.rho_fl; pr[YEL] = at.ye_fl; pr[TEMPL] = at.temp_fl;
     pr[ZXL] = pr[ZYL] = pr[ZZL] = 0.;
     unsigned ee = 0; double cs2;
     pr[PRESSL] = eos.press_from_temp_ent(pr[EPSL], cs2, pr[ENTL], pr[TEMPL], pr[RHOL], ee);
-    p2c(pr, cons, m);
+    p2c<FL>(pr, cons, m);
     set_all_resets(err);
     err |= BIT(E_ATMO_RESET);
 }
@@ -913,7 +974,7 @@ GHD void atmo_reset(double cons[NCONS], double pr[NPRIM], const Met& m, const At
 struct C2POut { bool floored, fatal; };
 
 // conservs_to_prims (c2p.cpp:188-414).  cons densitised in, re-densitised out.
-template <typename EOS>
+template <bool FL, typename EOS>
 GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eos, const Atmo& at,
                const ExcPar& ex, const C2PPar& cp, double radius, uint64_t& err, bool dry_run, C2PCount& cnt,
                const C2PGuess& gs, C2PRoots& rt) {
@@ -921,24 +982,26 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
     bool failed = false, floored = false;
     unsigned ret = 0;
     err = BIT(E_RESET_ENTROPY);
-    double isg = 1.0 / m.sqrtg;
-    (void)isg;
-    for (int i = 0; i < NCONS; ++i) cons[i] /= m.sqrtg;
+    if constexpr (!FL) {
+        const double isg = nr_rcp(m.sqrtg);
+        for (int i = 0; i < NCONS; ++i) cons[i] = quot(cons[i], m.sqrtg, isg);
+    }
     pr[BXL] = cons[BSXL]; pr[BYL] = cons[BSYL]; pr[BZL] = cons[BSZL];
-    if (cons[DENSL] < 0) { atmo_reset(cons, pr, m, at, eos, err); out.floored = true; return out; }
-    pr[YEL] = cons[YESL] / cons[DENSL];
+    if (cons[DENSL] < 0) { atmo_reset<FL>(cons, pr, m, at, eos, err); out.floored = true; return out; }
+    const double iD = nr_rcp(cons[DENSL]);
+    pr[YEL] = quot(cons[YESL], cons[DENSL], iD);
     if (pr[YEL] > eos.yemax()) { pr[YEL] = eos.yemax(); err |= BIT(E_RESET_YE); }
     if (pr[YEL] < eos.yemin()) { pr[YEL] = eos.yemin(); err |= BIT(E_RESET_YE); }
     bool lenient = m.alp < cp.alp_bh_thresh;
     {   // limit_conservatives (c2p.cpp:117-157)
         double emin, emax; eos.eps_range(emin, emax, cons[DENSL]);
-        double B2 = m.sqv(cons[BSXL], cons[BSYL], cons[BSZL]);
-        if (cons[TAUL] / cons[DENSL] - 0.5 * B2 / cons[DENSL] < fmin(0.0, emin)) {
+        double B2 = norm_up<FL>(m, cons[BSXL], cons[BSYL], cons[BSZL]);
+        if (quot(cons[TAUL], cons[DENSL], iD) - quot(0.5 * B2, cons[DENSL], iD) < fmin(0.0, emin)) {
             cons[TAUL] = emin * cons[DENSL] + 0.5 * B2;
             err |= BIT(E_RESET_TAU); floored = true;
         }
-        double st2max = sq(cons[TAUL] / cons[DENSL] + 1);
-        double st2 = m.sqcov(cons[STXL], cons[STYL], cons[STZL]) / sq(cons[DENSL]);
+        double st2max = sq(quot(cons[TAUL], cons[DENSL], iD) + 1);
+        double st2 = norm_low<FL>(m, cons[STXL], cons[STYL], cons[STZL]) / sq(cons[DENSL]);
         if (st2 > st2max) {
             double f = sqrt(st2max / st2);
             cons[STXL] *= f; cons[STYL] *= f; cons[STZL] *= f;
@@ -949,13 +1012,13 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
     if (cons[DENSL] >= at.rho_fl * (1 + at.atmo_tol)) {
         // both inversions start from the same invariants of the (limited)
         // conserved state, so they are formed once
-        C2PIn ci; c2p_setup(eos, m, cons, ci);
+        C2PIn ci; c2p_setup<FL>(eos, m, cons, ci);
         double res = kastaun(eos, ci, pr, ret, cnt, gs, rt);
         failed = (fabs(res) > cp.tol) || (ret & BIT(SIG_RHO_TOO_HIGH)) || (ret & BIT(SIG_EPS_TOO_HIGH)) || !isfinite(res);
         double beta;
         {
-            double W = lorentz(m.g, &pr[ZXL]);
-            double b[4], b2; smallb(m, &pr[BXL], &pr[ZXL], W, b, b2);
+            double W = lorentz<FL>(m.g, &pr[ZXL]);
+            double b[4], b2; smallb<FL>(m, &pr[BXL], &pr[ZXL], W, b, b2);
             beta = 2.0 * pr[PRESSL] / fmax(b2, 1e-50);
         }
         bool distrust = failed || (ret & BIT(SIG_EPS_TOO_LOW)) || (beta <= cp.beta_fallback);
@@ -981,7 +1044,7 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
     }
     bool excise = ex.by_radius ? (radius <= ex.r_ex) : (m.alp <= ex.alp_ex);
     if ((pr[RHOL] < (1. + at.atmo_tol) * at.rho_fl) || failed || excise) {
-        atmo_reset(cons, pr, m, at, eos, err);
+        atmo_reset<FL>(cons, pr, m, at, eos, err);
         floored = true;
     } else if (pr[TEMPL] < at.temp_fl) {
         pr[TEMPL] = at.temp_fl;
@@ -993,14 +1056,14 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
     } else {   // limit_primitives (c2p.cpp:63-115)
         unsigned sg = 0;
         double z2max = sq(cp.max_w) - 1.;
-        double z2 = m.sqv(pr[ZXL], pr[ZYL], pr[ZZL]);
+        double z2 = norm_up<FL>(m, pr[ZXL], pr[ZYL], pr[ZZL]);
         if (z2 >= z2max) {
             double zn = 0.99 * sqrt(z2max / z2);
             pr[ZXL] *= zn; pr[ZYL] *= zn; pr[ZZL] *= zn;
             sg |= BIT(SIG_VEL_TOO_HIGH);
         }
-        const double W = lorentz(m.g, &pr[ZXL]);
-        double b[4], b2; smallb(m, &pr[BXL], &pr[ZXL], W, b, b2);
+        const double W = lorentz<FL>(m.g, &pr[ZXL]);
+        double b[4], b2; smallb<FL>(m, &pr[BXL], &pr[ZXL], W, b, b2);
         double sigma = b2 / pr[RHOL];
         if (sigma >= cp.max_sigma) {
             pr[RHOL] *= 1.001 * sigma / cp.max_sigma;
@@ -1011,11 +1074,11 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
         if (!handle_sig<EOS>(sg, lenient, err)) out.fatal = true;
         if (sg & (BIT(SIG_VEL_TOO_HIGH) | BIT(SIG_SIGMA_TOO_HIGH))) floored = true;
         // the sigma limit changes rho and p only: W and b^mu still hold
-        p2c_wb(pr, cons, m, W, b, b2);
+        p2c_wb<FL>(pr, cons, m, W, b, b2);
         out.floored = floored;
         return out;
     }
-    p2c(pr, cons, m);
+    p2c<FL>(pr, cons, m);
     out.floored = floored;
     return out;
 }
