@@ -939,13 +939,39 @@ __global__ __launch_bounds__(256) void k_gather_list(const int4* __restrict__ en
     C.base[((int64_t)t.x * C.nv + C.v) * C.n + t.y] = C.base[((int64_t)t.z * C.nv + C.v) * C.n + t.w];
 }
 
+// Explicit entries copied by the workgroups behind those of k_gather_faces:
+// single ghost faces ({block, face, source block, source face}, nf[d] of each
+// direction) and conserved ghost cells (all nv channels from st on).  One
+// launch for what reads interior cells and faces only.
+struct GatherLists {
+    const int4* faces; int nf[3];
+    const int4* cells; int ncells;
+    double* st; int stv, vc; int64_t nc;
+};
 // Face ghosts of the three face-B arrays (wpb workgroups per block): the
-// first m0 / m1 / m2 of the nfg0 / nfg1 / nfg2 entries of each direction.
+// first m0 / m1 / m2 of the nfg0 / nfg1 / nfg2 entries of each direction;
+// then the lists.
 __global__ __launch_bounds__(256) void k_gather_faces(const int32_t* __restrict__ list, const int2* __restrict__ src,
                                                       int per, int ncg, int nfg0, int nfg1, int m0, int m1, int m2,
-                                                      int wpb, double* B0, double* B1, double* B2, int64_t nf0,
-                                                      int64_t nf1, int64_t nf2) {
-    const WgPos wp = wg_pos(wpb);
+                                                      int wpb, uint32_t nblocks, double* B0, double* B1, double* B2,
+                                                      int64_t nf0, int64_t nf1, int64_t nf2, GatherLists ls) {
+    if (blockIdx.x >= nblocks) {
+        const int r = (int)((blockIdx.x - nblocks) * blockDim.x + threadIdx.x);
+        const int f0 = ls.nf[0], f1 = f0 + ls.nf[1], f2 = f1 + ls.nf[2];
+        if (r < f2) {
+            const int4 t = ls.faces[r];
+            double* B = r < f0 ? B0 : (r < f1 ? B1 : B2);
+            const int64_t nf = r < f0 ? nf0 : (r < f1 ? nf1 : nf2);
+            B[(int64_t)t.x * nf + t.y] = B[(int64_t)t.z * nf + t.w];
+        } else if (r - f2 < ls.ncells) {
+            const int4 t = ls.cells[r - f2];
+            double* D = ls.st + (int64_t)t.x * ls.stv * ls.nc + t.y;
+            const double* S = ls.st + (int64_t)t.z * ls.stv * ls.nc + t.w;
+            for (int v = 0; v < ls.vc; ++v) D[v * ls.nc] = S[v * ls.nc];
+        }
+        return;
+    }
+    const WgPos wp = wg_pos_in(blockIdx.x, nblocks, wpb);
     const int r = wp.tile * (int)blockDim.x + (int)threadIdx.x;
     if (r >= m0 + m1 + m2) return;
     const int64_t q = wp.q;
@@ -1057,8 +1083,11 @@ static __device__ __align__(256) DevStats scratch[GRMHD_NOALLOC_MAX_STATES / 256
 #endif
 // Cell sets: CS_INTERIOR (the interior cells of every block, wpb workgroups
 // per block, see wg_pos), CS_SHELL (the ghost-shell cells of every block),
-// CS_LIST (explicit {block, cell} pairs).
-enum { CS_INTERIOR = 0, CS_SHELL = 1, CS_LIST = 2 };
+// CS_LIST (explicit {block, cell} pairs), CS_STAGE (the interior cells in the
+// first nint workgroups, then the pairs).
+// fresh: the error fields start from zero (the first stage of a step)
+// instead of adding to what they hold.
+enum { CS_INTERIOR = 0, CS_SHELL = 1, CS_LIST = 2, CS_STAGE = 3 };
 // GUESS 1 (learned): the root solves start from the MLP's prediction (ideal
 // gas: Newton finish, as k_c2p_batch<EOS, true, true>; other EOS: brackets).
 // GUESS 2 (warm start, ideal gas): the Newton finish starts from the cell's
@@ -1071,11 +1100,17 @@ __global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_cells(DevGrid G, EO
                                                    const double* __restrict__ mstate, int mnv,
                                                    const double* __restrict__ Bx, const double* __restrict__ By,
                                                    const double* __restrict__ Bz, double* aux, double* ecen,
-                                                   DevStats* stats, int cset, const int32_t* __restrict__ shell,
-                                                   const int2* __restrict__ cl, int ne, int wpb, MlpDev mlp) {
+                                                   DevStats* stats, int cset, uint32_t nint, bool fresh,
+                                                   const int32_t* __restrict__ shell, const int2* __restrict__ cl,
+                                                   int ne, int nlist, int wpb, MlpDev mlp) {
+    uint32_t wg = blockIdx.x;
+    if (cset == CS_STAGE) {
+        if (wg < nint) cset = CS_INTERIOR;
+        else { cset = CS_LIST; wg -= nint; ne = nlist; }
+    }
     WgPos wp{0, 0};
-    if (cset != CS_LIST) wp = wg_pos(wpb);
-    const int e = cset == CS_LIST ? (int)(blockIdx.x * blockDim.x + threadIdx.x)
+    if (cset != CS_LIST) wp = wg_pos_in(wg, nint, wpb);
+    const int e = cset == CS_LIST ? (int)(wg * blockDim.x + threadIdx.x)
                                   : wp.tile * (int)blockDim.x + (int)threadIdx.x;
     bool active = e < ne;
     const int ee = active ? e : 0;
@@ -1181,12 +1216,16 @@ __global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_cells(DevGrid G, EO
         A[RHO_ * nc] = pr[RHOL]; A[EPS_ * nc] = pr[EPSL]; A[PRESS_ * nc] = pr[PRESSL];
         A[TEMP_ * nc] = pr[TEMPL]; A[ENTROPY_ * nc] = pr[ENTL]; A[YE_ * nc] = pr[YEL];
         A[ZVECX_ * nc] = pr[ZXL]; A[ZVECY_ * nc] = pr[ZYL]; A[ZVECZ_ * nc] = pr[ZZL];
-        if (err & BIT(E_RESET_DENS)) { A[C2P_DENS_ERR_ * nc] += S[DENS_ * nc] - cons[DENSL]; S[DENS_ * nc] = cons[DENSL]; }
+        if (err & BIT(E_RESET_DENS)) {
+            const double was = fresh ? 0.0 : A[C2P_DENS_ERR_ * nc];
+            A[C2P_DENS_ERR_ * nc] = was + (S[DENS_ * nc] - cons[DENSL]);
+            S[DENS_ * nc] = cons[DENSL];
+        } else if (fresh) A[C2P_DENS_ERR_ * nc] = 0.0;
         if (err & BIT(E_RESET_STILDE)) { S[SX_ * nc] = cons[STXL]; S[SY_ * nc] = cons[STYL]; S[SZ_ * nc] = cons[STZL]; }
         if (err & BIT(E_RESET_TAU)) S[TAU_ * nc] = cons[TAUL];
         if (err & BIT(E_RESET_ENTROPY)) S[ENTROPYSTAR_ * nc] = cons[ENTSL];
         if (err & BIT(E_RESET_YE)) S[YESTAR_ * nc] = cons[YESL];
-        uint64_t prev = (uint64_t)A[C2P_ERR_ * nc];
+        const uint64_t prev = fresh ? 0 : (uint64_t)A[C2P_ERR_ * nc];
         A[C2P_ERR_ * nc] = (double)(prev | err);
         const DevInst& I = inst[blk[q].inst];
         A[BDIV_ * nc] = ((bx1 - bx0) * I.idx[0] + (by1 - by0) * I.idx[1] + (bz1 - bz0) * I.idx[2]) / m.sqrtg;
@@ -1355,14 +1394,6 @@ __global__ __launch_bounds__(256) void k_dt_final(const double* __restrict__ par
 // A host value into a device scalar, in stream order (host-dt entry points).
 __global__ void k_set_scalar(double* p, double v) { *p = v; }
 
-__global__ __launch_bounds__(256) void k_reset_diag(int64_t ncell, int64_t nq, double* aux) {
-    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ncell * nq) return;
-    int64_t q = t / ncell, c = t - q * ncell;
-    aux[(q * NAUX + C2P_DENS_ERR_) * ncell + c] = 0.0;
-    aux[(q * NAUX + C2P_ERR_) * ncell + c] = 0.0;
-}
-
 // ---------------------------------------------------------------------------
 // Host side: context
 // ---------------------------------------------------------------------------
@@ -1440,7 +1471,7 @@ struct grmhd_ctx {
     std::vector<TimerRec> timers;
     std::vector<hipEvent_t> ev_pool;
     // side streams and fork/join events of the concurrent RK3 stages
-    hipStream_t side[2] = {nullptr, nullptr};
+    hipStream_t side = nullptr;
     hipEvent_t fev[8] = {};
     // graph
     hipGraph_t graph = nullptr;
@@ -1553,7 +1584,7 @@ static void free_ctx(grmhd_ctx* c) {
     for (auto& t : c->timers) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
     for (auto e : c->ev_pool) (void)hipEventDestroy(e);
     for (auto e : c->fev) if (e) (void)hipEventDestroy(e);
-    for (auto t : c->side) if (t) (void)hipStreamDestroy(t);
+    if (c->side) (void)hipStreamDestroy(c->side);
 }
 
 // Host description of a two-level forest (grmhd_ctx_create_forest).
@@ -2189,25 +2220,27 @@ static void launch_update(grmhd_ctx* c, UpdArgs& a, hipStream_t s) {
 static void launch_gather(grmhd_ctx* c, const GatherArgs& a, hipStream_t s) {
     const DevGrid& G = c->G;
     const int per = (int)(c->ncg + c->nfg[0] + c->nfg[1] + c->nfg[2]);
+    // the conserved of the ghosts that run their own c2p read interior cells
+    // only, as the faces read interior faces: one launch for both
+    const bool own_with_faces = a.B[0] && a.cell_mode == 2 && !a.aux && !a.ecen && c->n_own_gather > 0;
     if (a.B[0]) {
         Scope sc(c, "ghost_faces", s);
         const int64_t* m = a.faces_slab ? c->nfg_slab : c->nfg;
         const int wpb = (int)nblk_bs(m[0] + m[1] + m[2], c->tune.gather_faces);
-        k_gather_faces<<<dim3((unsigned)(wpb * G.nq)), c->tune.gather_faces, 0, s>>>(
-            c->ghost_list, c->ghost_src, per, (int)c->ncg, (int)c->nfg[0], (int)c->nfg[1], (int)m[0], (int)m[1],
-            (int)m[2], wpb, a.B[0], a.B[1], a.B[2], G.nface[0], G.nface[1], G.nface[2]);
+        GatherLists ls{};
         if (a.faces_slab) {
-            int64_t o = 0;
-            for (int d = 0; d < 3; ++d) {
-                if (c->n_ofl[d] > 0) {
-                    GatherChans fc{};
-                    fc.c[0] = GatherChan{a.B[d], 1, 0, G.nface[d]};
-                    fc.nch = 1;
-                    k_gather_list<<<dim3(nblk(c->n_ofl[d]), 1, 1), 256, 0, s>>>(c->ofl_faces + o, (int)c->n_ofl[d], fc);
-                }
-                o += c->n_ofl[d];
-            }
+            ls.faces = c->ofl_faces;
+            for (int d = 0; d < 3; ++d) ls.nf[d] = (int)c->n_ofl[d];
         }
+        if (own_with_faces) {
+            ls.cells = c->own_gather; ls.ncells = (int)c->n_own_gather;
+            ls.st = a.st + a.v0 * G.ncell; ls.stv = a.nv; ls.vc = a.vc; ls.nc = G.ncell;
+        }
+        const unsigned nb = (unsigned)(wpb * G.nq);
+        const unsigned nl = nblk_bs(ls.nf[0] + ls.nf[1] + ls.nf[2] + ls.ncells, c->tune.gather_faces);
+        k_gather_faces<<<dim3(nb + nl), c->tune.gather_faces, 0, s>>>(
+            c->ghost_list, c->ghost_src, per, (int)c->ncg, (int)c->nfg[0], (int)c->nfg[1], (int)m[0], (int)m[1],
+            (int)m[2], wpb, nb, a.B[0], a.B[1], a.B[2], G.nface[0], G.nface[1], G.nface[2], ls);
         // the second pass reads what the copies and the first pass wrote
         if (c->n_amr_faces > 0)
             k_amr_faces<<<nblk(c->n_amr_faces), 256, 0, s>>>(c->amr_faces, (int)c->n_amr_faces, a.B[0], a.B[1], a.B[2], c->ff);
@@ -2235,7 +2268,7 @@ static void launch_gather(grmhd_ctx* c, const GatherArgs& a, hipStream_t s) {
     // coarse-fine ghost cells of the state (they run their own c2p)
     const bool amr = a.st && a.cell_mode <= 2 && c->n_amr_cells > 0;
     if (a.cell_mode == 2) {
-        if (c->n_own_gather > 0)
+        if (c->n_own_gather > 0 && !own_with_faces)
             k_gather_list<<<dim3(nblk(c->n_own_gather), 1, ch.nch), 256, 0, s>>>(c->own_gather, (int)c->n_own_gather, ch);
         if (amr) k_amr_cells<<<nblk(c->n_amr_cells), 256, 0, s>>>(c->amr_cells, (int)c->n_amr_cells, a.st, a.nv, a.v0, a.vc, c->ff);
         return;
@@ -2267,7 +2300,7 @@ static void launch_reflux(grmhd_ctx* c, hipStream_t s, int part = 0) {
 // c2p over the cells of every block: the interior cells, plus either every
 // ghost cell (all) or only the ghost cells that need their own c2p.
 static void launch_c2p_cells(grmhd_ctx* c, double* st, int snv, const double* ms, int mnv, const double* const B[3],
-                             double* aux, bool with_stats, bool selective, hipStream_t s,
+                             double* aux, bool with_stats, bool selective, bool fresh, hipStream_t s,
                              hipStream_t s_list = nullptr) {
     Scope sc(c, "c2p", s);
     const DevGrid& G = c->G;
@@ -2282,11 +2315,11 @@ static void launch_c2p_cells(grmhd_ctx* c, double* st, int snv, const double* ms
     // the explicit-list launch may go to its own stream (no statistics then:
     // k_stats_final below reads every partial record on s)
     const hipStream_t sl = (s_list && !with_stats) ? s_list : s;
-    auto launch = [&](int cset, int ne, dim3 grid, int wpb) {
+    auto launch = [&](int cset, int ne, unsigned grid, int wpb, unsigned nint, int nlist) {
         DevStats* part = with_stats ? c->stats_part + npart : nullptr;
-        npart += (int64_t)grid.x * grid.y;
+        npart += grid;
         const hipStream_t ls = cset == CS_LIST ? sl : s;
-#define C2PL(EOSV, FL, LR) k_c2p_cells<decltype(EOSV), FL, LR><<<grid, bs, 0, ls>>>(G, EOSV, c->O, c->inst_d, c->blk_d, st, snv, ms, mnv, B[0], B[1], B[2], aux, ec, part, cset, c->ghost_list, c->own_cells, ne, wpb, md)
+#define C2PL(EOSV, FL, LR) k_c2p_cells<decltype(EOSV), FL, LR><<<grid, bs, 0, ls>>>(G, EOSV, c->O, c->inst_d, c->blk_d, st, snv, ms, mnv, B[0], B[1], B[2], aux, ec, part, cset, nint, fresh, c->ghost_list, c->own_cells, ne, nlist, wpb, md)
         if (warm) {
             if (flat) C2PL(c->ideal, true, 2); else C2PL(c->ideal, false, 2);
         } else if (c->mlp) {
@@ -2300,10 +2333,15 @@ static void launch_c2p_cells(grmhd_ctx* c, double* st, int snv, const double* ms
     };
     {
         const int wi = (int)nblk_bs(ni, bs), ws = (int)nblk_bs(c->ncg, bs);
-        launch(CS_INTERIOR, ni, dim3((unsigned)(wi * G.nq)), wi);
-        if (!selective) launch(CS_SHELL, (int)c->ncg, dim3((unsigned)(ws * G.nq)), ws);
+        const unsigned gi = (unsigned)(wi * G.nq), gs = (unsigned)(ws * G.nq);
+        const int nl = selective ? (int)c->n_own : 0;
+        if (nl > 0 && sl == s) launch(CS_STAGE, ni, gi + nblk_bs(nl, bs), wi, gi, nl);
+        else {
+            launch(CS_INTERIOR, ni, gi, wi, gi, 0);
+            if (nl > 0) launch(CS_LIST, nl, nblk_bs(nl, bs), 0, 0, 0);
+        }
+        if (!selective) launch(CS_SHELL, (int)c->ncg, gs, ws, gs, 0);
     }
-    if (selective && c->n_own > 0) launch(CS_LIST, (int)c->n_own, dim3(nblk_bs(c->n_own, bs), 1), 0);
     if (with_stats) {
         sum_stats(c->stats_part, npart, c->stats, s);
         c->last_c2p_n = G.ncell * G.nq;
@@ -2433,7 +2471,7 @@ extern "C" grmhd_status grmhd_fill_metric_ghosts(grmhd_ctx* c, double* state, gr
 extern "C" grmhd_status grmhd_compute_auxiliaries(grmhd_ctx* c, double* state, const double* const B[3], double* aux,
                                                   grmhd_stream_t stream) {
     if (!c || !state || !B || !aux) { set_err("null argument"); return GRMHD_ERR_INVALID; }
-    launch_c2p_cells(c, state, NSTATE, state, NSTATE, B, aux, true, false, (hipStream_t)stream);
+    launch_c2p_cells(c, state, NSTATE, state, NSTATE, B, aux, true, false, false, (hipStream_t)stream);
     return launch_check("compute_auxiliaries");
 }
 
@@ -2728,8 +2766,7 @@ extern "C" grmhd_status grmhd_find_stable_timestep(grmhd_ctx* c, const double* s
 static grmhd_status ensure_stage_buffers(grmhd_ctx* c) {
     if (c->U1) return GRMHD_OK;
     const DevGrid& G = c->G;
-    for (auto& t : c->side)
-        if (!t) HIP_TRY(hipStreamCreateWithFlags(&t, hipStreamNonBlocking));
+    if (!c->side) HIP_TRY(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
     for (auto& e : c->fev)
         if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     HIP_TRY(hipMalloc(&c->U1, sizeof(double) * NHRSC * G.ncell * G.nq));
@@ -2739,6 +2776,22 @@ static grmhd_status ensure_stage_buffers(grmhd_ctx* c) {
         HIP_TRY(hipMalloc(&c->B2[d], sizeof(double) * G.nface[d] * G.nq));
     }
     return GRMHD_OK;
+}
+
+// Whether the independent launches of a stage run on a side stream beside the
+// main one, from 2^18 interior cells on.  Below, a launch does not fill the
+// card for longer than a fork and a join cost, and one stream also lets
+// launches merge (update cells with faces, ghost faces with conserved, interior
+// c2p with that of the ghosts: six launches a stage).  RK3 steps with / without
+// the side stream, 16^3 blocks, us eager and as a graph: 8 blocks 335 / 187
+// and 224 / 195, 27 blocks 401 / 333 and 354 / 346, 48 blocks 564 / 506 and
+// 521 / 518, 64 blocks 692 / 680 and 658 / 684, 100 blocks 980 / 1009 and
+// 945 / 1012; curved, 27 blocks 609 / 519 and 532 / 532, 64 blocks
+// 1110 / 1074 and 1068 / 1070.
+constexpr int64_t CONC_MIN_CELLS = 1 << 18;
+static bool stage_conc(const grmhd_ctx* c) {
+    const DevGrid& G = c->G;
+    return c->P.stage_streams && !c->P.fofc && c->side && G.nq * G.n[0] * G.n[1] * G.n[2] >= CONC_MIN_CELLS;
 }
 
 // The fused RK3 step.  Stage buffers hold only the 7 hydro conserved; the
@@ -2762,43 +2815,34 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
         {c->U2, NHRSC, state, NSTATE, c->U1, NHRSC, 0.75, 0.25, 0.25, nB2, Bc, B1c, c->U1, NHRSC, B1c},
         {state, NSTATE, state, NSTATE, c->U2, NHRSC, 1. / 3, 2. / 3., 2. / 3., B, Bc, B2c, c->U2, NHRSC, B2c},
     };
-    // Without FOFC, independent launches of a stage run side by side: the
-    // three flux directions; then the ghost-face passes (copies and, on a
+    // Without FOFC, independent launches of a stage of a large grid run side
+    // by side: the ghost-face passes (copies and, on a
     // forest, the coarse-fine face passes) and the c2p of the ghosts that run
     // their own (outflow and coarse-fine ghosts) next to the c2p of the
     // interior cells.  The conserved fills those ghost c2p read (copies and
     // coarse-fine prolongation/restriction from interior cells) stay on s
     // ahead of the interior c2p, which may rewrite interior conserved.
     // Ordering by events, so the same sequence is captured into the step's
-    // graph.  (grmhd_params.stage_streams = 0 or per-family timing: every
-    // launch on s.)
-    const bool conc = c->P.stage_streams && !c->timing && !c->P.fofc && c->side[0] && c->side[1];
+    // graph.  (Small grids, see stage_conc, grmhd_params.stage_streams = 0 or
+    // per-family timing: every launch on s.)
+    const bool conc = stage_conc(c) && !c->timing;
     auto fork = [&](int k, hipStream_t from, hipStream_t to) {
         (void)hipEventRecord(c->fev[k], from);
         (void)hipStreamWaitEvent(to, c->fev[k], 0);
     };
-    // the c2p error fields are cleared once per step; only the c2p reads
-    // them, so with side streams the clear runs beside the first fluxes
-    if (!conc) k_reset_diag<<<nblk(G.ncell * G.nq), 256, 0, s>>>(G.ncell, G.nq, aux);
     for (int sidx = 0; sidx < 3; ++sidx) {
         Stage& S = st[sidx];
-        const bool reset_aside = conc && sidx == 0;
-        if (reset_aside) {
-            fork(0, s, c->side[1]);
-            k_reset_diag<<<nblk(G.ncell * G.nq), 256, 0, c->side[1]>>>(G.ncell, G.nq, aux);
-        }
         c->ring_copy_now = sidx > 0;
         launch_fluxes(c, aux, state, NSTATE, S.oB, s);
         c->ring_copy_now = false;
-        if (reset_aside) fork(2, c->side[1], s);
         // the cell part of the update needs only the fluxes (on a forest
-        // after their reflux): it runs on side[0] beside the edge EMFs, the
+        // after their reflux): it runs on side beside the edge EMFs, the
         // face (CT) part after them (and their reflux) on s.  Not with GS
         // EMFs on a forest: those read the mass fluxes the reflux rewrites.
         const bool split_update = conc && !(c->forest && c->P.emf == GRMHD_EMF_GS);
         if (split_update) {
-            fork(6, s, c->side[0]);
-            launch_reflux(c, c->side[0], 1);
+            fork(6, s, c->side);
+            launch_reflux(c, c->side, 1);
         }
         launch_emf(c, S.oB, s);
         if (c->P.fofc)
@@ -2812,10 +2856,10 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
         if (split_update) {
             UpdArgs ac = a;
             ac.part = 1;
-            launch_update(c, ac, c->side[0]);
+            launch_update(c, ac, c->side);
             a.part = 2;
             launch_update(c, a, s);
-            fork(7, c->side[0], s);
+            fork(7, c->side, s);
         } else {
             launch_update(c, a, s);
         }
@@ -2826,21 +2870,21 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
         // outflow faces their own faces
         const bool faces_slab = sidx < 2 && c->ring_own != nullptr;
         if (conc) {
-            // side[0]: ghost faces, then (after the conserved fills on s) the
+            // side: ghost faces, then (after the conserved fills on s) the
             // c2p of the ghosts that run their own; s: conserved fills,
             // interior c2p.
-            fork(3, s, c->side[0]);
+            fork(3, s, c->side);
             GatherArgs gf{};
             for (int d = 0; d < 3; ++d) gf.B[d] = S.nB[d];
             gf.cell_mode = 0;
             gf.faces_slab = faces_slab;
-            launch_gather(c, gf, c->side[0]);
+            launch_gather(c, gf, c->side);
             GatherArgs gc{};
             gc.st = S.nst; gc.nv = S.nnv; gc.v0 = 0; gc.vc = NHRSC; gc.cell_mode = 2;
             launch_gather(c, gc, s);
-            fork(4, s, c->side[0]);
-            launch_c2p_cells(c, S.nst, S.nnv, state, NSTATE, nBc, aux, false, true, s, c->side[0]);
-            fork(5, c->side[0], s);
+            fork(4, s, c->side);
+            launch_c2p_cells(c, S.nst, S.nnv, state, NSTATE, nBc, aux, false, true, sidx == 0, s, c->side);
+            fork(5, c->side, s);
         } else {
             {   // ghost faces everywhere; conserved only where a ghost runs its own c2p
                 // (everywhere with FOFC: its next-stage tests read the ghost layer)
@@ -2850,7 +2894,7 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
                 g.faces_slab = faces_slab;
                 launch_gather(c, g, s);
             }
-            launch_c2p_cells(c, S.nst, S.nnv, state, NSTATE, nBc, aux, false, true, s);
+            launch_c2p_cells(c, S.nst, S.nnv, state, NSTATE, nBc, aux, false, true, sidx == 0, s);
         }
         {   // c2p outputs into the other ghost cells: the reconstructed
             // primitives (and the GS cell E, which the next stage's edge EMFs
@@ -3002,7 +3046,7 @@ extern "C" grmhd_status grmhd_autotune(grmhd_ctx* c, const double* state, const 
     double* const B1[3] = {c->B1[0], c->B1[1], c->B1[2]};
     const double* const B1c[3] = {c->B1[0], c->B1[1], c->B1[2]};
     grmhd_tuning keep = c->tune;
-    const bool conc = c->P.stage_streams && !c->P.fofc && c->side[0] && c->side[1];
+    const bool conc = stage_conc(c);
     // the flux launch in the form of the second and third RK stages (ring
     // faces pushed, reads across block faces) when the context shares ring
     // faces; one workgroup size for its three directions
@@ -3027,14 +3071,14 @@ extern "C" grmhd_status grmhd_autotune(grmhd_ctx* c, const double* state, const 
         u.dt = dt0; u.dtfact = 1.0;
         if (split) {
             (void)hipEventRecord(c->fev[0], s);
-            (void)hipStreamWaitEvent(c->side[0], c->fev[0], 0);
+            (void)hipStreamWaitEvent(c->side, c->fev[0], 0);
             UpdArgs uc = u;
             uc.part = 1;
-            launch_update(c, uc, c->side[0]);
+            launch_update(c, uc, c->side);
             launch_emf(c, Bc, s);
             u.part = 2;
             launch_update(c, u, s);
-            (void)hipEventRecord(c->fev[1], c->side[0]);
+            (void)hipEventRecord(c->fev[1], c->side);
             (void)hipStreamWaitEvent(s, c->fev[1], 0);
         } else {
             launch_emf(c, Bc, s);
@@ -3059,7 +3103,7 @@ extern "C" grmhd_status grmhd_autotune(grmhd_ctx* c, const double* state, const 
         for (int d = 0; d < 3; ++d) g.B[d] = B1[d];
         launch_gather(c, g, s);
     }
-    pick(&c->tune.c2p, [&] { launch_c2p_cells(c, c->U1, NHRSC, state, NSTATE, B1c, aux2, false, true, s); });
+    pick(&c->tune.c2p, [&] { launch_c2p_cells(c, c->U1, NHRSC, state, NSTATE, B1c, aux2, false, true, false, s); });
     (void)hipStreamSynchronize(s);
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(b);
