@@ -161,16 +161,15 @@ struct FluxArgs {
     // ring_own (per block, bit 2 d + side for the six block faces): when
     // given, a ring face is computed only if its ghost side lies beyond an
     // outflow face of the instance; the others are interior faces of the
-    // neighbouring block, whose threads write them through push_nbr (the
-    // neighbour across each of the six block faces; with periodicity per
-    // dimension the relation is symmetric).  With push_nbr (the second and
-    // third RK stages, whose gathers leave the face slabs alone) a full face
-    // takes a cell beyond a block face from the neighbouring block's
-    // interior (normal index shifted by one block extent); beyond an outflow
-    // face (no neighbour) and on ring faces, from its own ghosts, which run
-    // their own c2p or copy one that does.
+    // neighbouring block, from which the edge EMFs then take them.
+    // With nbr (the neighbour across each of the six block faces, in the
+    // second and third RK stages, whose gathers leave the face slabs alone) a
+    // full face takes a cell beyond a block face from the neighbouring
+    // block's interior (normal index shifted by one block extent); beyond an
+    // outflow face (no neighbour) and on ring faces, from its own ghosts,
+    // which run their own c2p or copy one that does.
     const uint8_t* ring_own;
-    const int32_t* push_nbr;
+    const int32_t* nbr;
     int dir0, ndir;                    // directions of this launch: dir0 .. dir0 + ndir - 1
     int tiles, tilesr;                 // workgroups per block and direction: full faces, ring faces
 };
@@ -230,38 +229,6 @@ GHD bool line_pos(const DevGrid& G, int T0, int T1, bool uct, bool ring, int p, 
     return !use_own || ((own >> side) & 1);
 }
 
-// Neighbours of block q across its six faces (-1: none) in scalar registers,
-// read once ahead of the first store: read where they are used, each would
-// wait for every store before it.
-struct Nbrs { int32_t q[6]; };
-__device__ __forceinline__ Nbrs block_nbrs(const int32_t* push_nbr, int64_t q) {
-    Nbrs n;
-#pragma unroll
-    for (int s = 0; s < 6; ++s) n.q[s] = push_nbr ? __builtin_amdgcn_readfirstlane(push_nbr[q * 6 + s]) : -1;
-    return n;
-}
-// The UCT values of an interior face within ngz of a block face, stored into
-// the ring slot of the neighbour across that face as well: the same face
-// there has its transverse index one block extent further out.  fo: the
-// face's offset, t0/t1 its transverse indices.
-template <int D>
-__device__ __forceinline__ void push_ring(const DevGrid& G, const Nbrs& nb, double* vbar, uint32_t fo, int t0, int t1,
-                                          const double V[4]) {
-    constexpr int T0 = D == 0 ? 1 : 0, T1 = D == 2 ? 1 : 2;
-    const int64_t ns = G.ns;
-    const uint32_t row = (uint32_t)G.sp * 8u, plane = row * (uint32_t)(G.N[1] + 1);
-    const uint32_t s0 = (D == 0 ? row : 8u) * (uint32_t)G.n[T0], s1 = (D == 2 ? row : plane) * (uint32_t)G.n[T1];
-    auto put = [&](int32_t qt, bool near, uint32_t to) {
-        if (qt < 0 || !near) return;
-        double* T = vbar + (int64_t)qt * 4 * ns;
-        st_off(T, to, V[0]); st_off(T + ns, to, V[1]); st_off(T + 2 * ns, to, V[2]); st_off(T + 3 * ns, to, V[3]);
-    };
-    put(nb.q[2 * T0], t0 < 2 * G.ng, fo + s0);
-    put(nb.q[2 * T0 + 1], t0 >= G.n[T0], fo - s0);
-    put(nb.q[2 * T1], t1 < 2 * G.ng, fo + s1);
-    put(nb.q[2 * T1 + 1], t1 >= G.n[T1], fo - s1);
-}
-
 // Metric of face (i, j, k): the cache (only the inverse component this
 // direction uses: cmcp, the LLF speed limit) or the interpolation.
 template <bool FLAT, int D>
@@ -312,18 +279,22 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
     const int64_t nc = G.ncell, nf = G.nface[D];
     const int64_t st = D == 0 ? 1 : (D == 1 ? G.N[0] : (int64_t)G.N[0] * G.N[1]);
     const double Bf = ld_off(f.B[D] + q * nf, (uint32_t)fidx<D>(G, i, j, k) * 8u);
-    const Nbrs nb = block_nbrs(FLAT && !ring ? f.push_nbr : nullptr, q);
-    const int32_t nl = nb.q[2 * D], nh = nb.q[2 * D + 1];
+    // (scalar registers; -1: none)
+    int32_t nl = -1, nh = -1;
+    if (FLAT && !ring && f.nbr) {
+        nl = __builtin_amdgcn_readfirstlane(f.nbr[q * 6 + 2 * D]);
+        nh = __builtin_amdgcn_readfirstlane(f.nbr[q * 6 + 2 * D + 1]);
+    }
     const int64_t c0 = cidx(G, i, j, k);
     const double* P[6];
+    {
+        // points 0 to 2 can only lie before the block, the others only beyond
+        const double* own = f.aux + q * NAUX * nc + c0;
+        const int64_t dl = nl < 0 ? 0 : (nl - q) * NAUX * nc + nD * st, dh = nh < 0 ? 0 : (nh - q) * NAUX * nc - nD * st;
 #pragma unroll
-    for (int t = 0; t < 6; ++t) {
-        const int m = m0 + t - 3;
-        int64_t qb = q;
-        int sh = t - 3;
-        if (nl >= 0 && m < ng) { qb = nl; sh += nD; }
-        else if (nh >= 0 && m >= nD + ng) { qb = nh; sh -= nD; }
-        P[t] = f.aux + qb * NAUX * nc + c0 + sh * st;
+        for (int t = 0; t < 3; ++t) P[t] = own + (t - 3) * st + (m0 + t - 3 < ng ? dl : 0);
+#pragma unroll
+        for (int t = 3; t < 6; ++t) P[t] = own + (t - 3) * st + (m0 + t - 3 >= nD + ng ? dh : 0);
     }
     auto load = [&](int v, double* u, uint32_t z) {
         const int64_t ov = fq_aux<D>(v, o.thermo) * nc + z;
@@ -343,7 +314,7 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
             const double* w = u[v % 3];
             if (ring && (v == FQ_YE || v == FQ_ENT)) { L[v] = 0.0; R[v] = 0.0; }
             else if constexpr (REC == 0) ok = wenoz_face(w[0], w[1], w[2], w[3], w[4], w[5], L[v], R[v]) && ok;
-            else recon<REC>(w[0], w[1], w[2], w[3], w[4], w[5], L[v], R[v]);
+            else recon<REC>(w[1], w[2], w[3], w[4], L[v], R[v]);
             settle(L[v], R[v]);
         }
         if constexpr (REC == 0)
@@ -382,7 +353,6 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
     double* F0 = f.flux[D] + q * NHRSC * ns;
 #pragma unroll
     for (int v = 0; v < NHRSC; ++v) st_off(F0 + v * ns, so, F[v]);
-    if (FLAT) push_ring<D>(G, nb, f.vbar[D], so, b, c, V);
 }
 
 // The faces of f.ndir directions of every block, one thread per face.  The
@@ -393,15 +363,17 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
 // behind the full faces of all blocks: their threads are shorter.
 //
 // Bound by the FP64 units (about 350 us of arithmetic for 512 blocks of
-// 16^3) beside the stores of fluxes, face values and ring copies: 555 us per
-// launch there in the RK stages that push, 488 without the flux stores, 493
-// without the ring copies, 430 without either; one launch per direction over
-// rows in the boundary's layout took 3 x 245.  A thread per face with nine
-// variables one after another needs 127 VGPRs (4 waves per SIMD; curved 165,
-// 3 waves).  A thread that walks along a line of faces saves the shared half
-// of the reconstruction but keeps the stencils of nine variables: 230 VGPRs,
-// 2 waves, 1.0 ms for y and 0.9 for z per three stages against 0.77 and 0.67
-// here; with the stencil read again at each step 1.1 and 1.0.
+// 16^3) beside the stores of fluxes and face values: 500 us per launch there
+// in the RK stages that share ring faces, 430 without the flux stores; one
+// launch per direction over rows in the boundary's layout, which also copied
+// its outer face values into the neighbours' ring slots, took 3 x 245.  (The
+// edge EMFs read them from the neighbour instead: 130 MB less to write.)  A
+// thread per face with nine variables one after another needs 126 VGPRs (4
+// waves per SIMD; curved 165, 3 waves).  A thread that walks along a line of
+// faces saves the shared half of the reconstruction but keeps the stencils of
+// nine variables: 230 VGPRs, 2 waves, 1.0 ms for y and 0.9 for z per three
+// stages against 0.67 and 0.64 here; with the stencil read again at each step
+// 1.1 and 1.0.
 template <typename EOS, int REC, bool FLAT>
 __global__ __launch_bounds__(256, FLAT ? 3 : 2) void k_flux(DevGrid G, EOS eos, Opts o, FluxArgs f) {
     const uint32_t nfull = (uint32_t)(f.tiles * f.ndir) * (uint32_t)G.nq;

@@ -5,7 +5,7 @@
 //                  launch: reconstruction, face metric, EOS, HLLE/LLF fluxes,
 //                  vbar/Eface (reference: evolve.cpp:813-1068,
 //                  grmhd.hh:551-970)
-//   k_emf_uct      one thread per edge triple: UCT edge EMFs (evolve.cpp:1130-1340)
+//   k_emf_uct      one thread per edge: UCT edge EMFs (evolve.cpp:1130-1340)
 //   k_emf_gs       Gardiner-Stone edge EMFs (grmhd_helpers.hh:492-627)
 //   k_update       fused RK linear combination + geometric sources + flux
 //                  divergence + CT face update (tstep_utils.hh:140-220,
@@ -187,78 +187,132 @@ constexpr int FMC = 13;
 #include "flux.hh"
 
 // ---------------------------------------------------------------------------
-// UCT edge EMFs.  Face arrays: B faces (1 var), vbar (4 vars, stride nf).
+// UCT edge EMFs (evolve.cpp:1130-1340), one thread per edge.
 // ---------------------------------------------------------------------------
-template <int REC>
-GHD void rec6(const double* P, int64_t s, double& uL, double& uR) {
-    recon<REC>(P[-3 * s], P[-2 * s], P[-s], P[0], P[s], P[2 * s], uL, uR);
+struct EmfArgs {
+    const double* B[3];   // face B
+    const double* V[3];   // UCT face values: two transverse velocities, two speeds
+    double* emf;
+    // neighbour of each block across its six faces, or null: when given, the
+    // face values beyond a block face are the neighbour's own (the same
+    // global faces), and only those beyond the grid's end (no neighbour: -1)
+    // stand in the block's ring slots
+    const int32_t* nbr;
+    int tiles;            // workgroups per block and component
+};
+
+// Addresses of the six face values around cell index m of a direction (points
+// m - 3 .. m + 2, m in [ng, n + ng]; own: point m; st: its stride): dl / dh
+// take a point before / beyond the block into the neighbour's array (0: the
+// block's own ring slots).  Points 0 to 2 can only lie before, the others
+// only beyond.
+__device__ __forceinline__ void face_line(const double* own, int m, int n, int ng, int64_t dl, int64_t dh, int64_t st,
+                                          const double* P[6]) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t) P[t] = own + (t - 3) * st + (m + t - 3 < ng ? dl : 0);
+#pragma unroll
+    for (int t = 3; t < 6; ++t) P[t] = own + (t - 3) * st + (m + t - 3 >= n + ng ? dh : 0);
 }
 
-template <int REC>
-__global__ __launch_bounds__(256) void k_emf_uct(DevGrid G, const double* __restrict__ Bx,
-                                                 const double* __restrict__ By, const double* __restrict__ Bz,
-                                                 const double* __restrict__ vx, const double* __restrict__ vy,
-                                                 const double* __restrict__ vz, double* __restrict__ emf, int wpb) {
-    // wpb workgroups per block over its (n+1)^3 sites (see wg_pos)
-    const int R0 = G.n[0] + 1, R1 = G.n[1] + 1, R2 = G.n[2] + 1;
-    const WgPos wp = wg_pos(wpb);
-    const int r = wp.tile * (int)blockDim.x + (int)threadIdx.x;
-    if (r >= R0 * R1 * R2) return;
-    const int64_t q = wp.q;
-    int kz, rxy, jy, ix0;
-    udivmod(r, R0 * R1, kz, rxy);
-    udivmod(rxy, R0, jy, ix0);
-    const int i = G.ng + ix0, j = G.ng + jy, k = G.ng + kz;
-    const int64_t nfx = G.nface[0], nfy = G.nface[1], nfz = G.nface[2];
-    const double* bx = Bx + q * nfx; const double* by = By + q * nfy; const double* bz = Bz + q * nfz;
+// Component C at edge (i, j, k): with P, Q the next two directions in cyclic
+// order, the HLL averages of v^Q B^P across Q and of v^P B^Q across P.
+template <int REC, int C>
+__device__ __forceinline__ void emf_edge(const DevGrid& G, const EmfArgs& a, int64_t q, int e) {
+    constexpr int P = (C + 1) % 3, Q = (C + 2) % 3;
+    // slot of the velocity along Q among P's transverse ones, and vice versa
+    constexpr int SQ = Q == (P == 0 ? 1 : 0) ? 0 : 1, SP = P == (Q == 0 ? 1 : 0) ? 0 : 1;
+    const int R0 = G.n[0] + (C != 0), R1 = G.n[1] + (C != 1), R2 = G.n[2] + (C != 2);
+    if (e >= R0 * R1 * R2) return;
+    int i, j, k, r;
+    udivmod(e, R0, r, i);
+    udivmod(r, R1, k, j);
+    i += G.ng; j += G.ng; k += G.ng;
     const int64_t ns = G.ns;
-    const double* Vx = vx + q * 4 * ns; const double* Vy = vy + q * 4 * ns; const double* Vz = vz + q * 4 * ns;
-    // strides of the face arrays along each axis
-    const int64_t sx_x = 1, sx_y = G.N[0] + 1, sx_z = (int64_t)(G.N[0] + 1) * G.N[1];
-    const int64_t sy_x = 1, sy_y = G.N[0], sy_z = (int64_t)G.N[0] * (G.N[1] + 1);
-    const int64_t sz_x = 1, sz_y = G.N[0], sz_z = (int64_t)G.N[0] * G.N[1];
-    // strides and this site's offset in the context's arrays
-    const int64_t sy = G.sp, sz = (int64_t)G.sp * (G.N[1] + 1);
-    double* E = emf + q * 3 * ns;
-    const int64_t eo = sidx(G, i, j, k);
-    if (i < G.n[0] + G.ng) {  // E^x at (i, j-1/2, k-1/2)
-        int64_t fy = fidx<1>(G, i, j, k), fz = fidx<2>(G, i, j, k);
-        double ByL, ByR, vzL, vzR, BzL, BzR, vyL, vyR;
-        rec6<REC>(by + fy, sy_z, ByL, ByR);
-        rec6<REC>(Vy + ns + eo, sz, vzL, vzR);
-        rec6<REC>(bz + fz, sz_y, BzL, BzR);
-        rec6<REC>(Vz + ns + eo, sy, vyL, vyR);
-        double cmin_y = fmax(Vy[2 * ns + eo], Vy[2 * ns + eo - sz]);
-        double cmax_y = fmax(Vy[3 * ns + eo], Vy[3 * ns + eo - sz]);
-        double cmin_z = fmax(Vz[2 * ns + eo], Vz[2 * ns + eo - sy]);
-        double cmax_z = fmax(Vz[3 * ns + eo], Vz[3 * ns + eo - sy]);
-        E[eo] = hll(vzL * ByL, vzR * ByR, ByL, ByR, cmin_z, cmax_z) - hll(vyL * BzL, vyR * BzR, BzL, BzR, cmin_y, cmax_y);
+    auto stride = [&](int d) { return (int64_t)(d == 0 ? 1 : (d == 1 ? G.sp : G.sp * (G.N[1] + 1))); };
+    auto bstride = [&](int f, int d) {   // of face array f
+        const int n0 = G.N[0] + (f == 0), n1 = G.N[1] + (f == 1);
+        return d == 0 ? 1 : (d == 1 ? n0 : n0 * n1);
+    };
+    const uint32_t eo = (uint32_t)sidx(G, i, j, k) * 8u;
+    const int64_t bs = 4 * ns, stP = stride(P), stQ = stride(Q);
+    int64_t d[4] = {0, 0, 0, 0};       // across the faces below and above along P and Q
+    if (a.nbr) {
+        const int32_t* N = a.nbr + q * 6;
+        auto across = [&](int side, int64_t shift) {
+            const int32_t x = __builtin_amdgcn_readfirstlane(N[side]);
+            return x < 0 ? 0 : (x - q) * bs + shift;
+        };
+        d[0] = across(2 * P, G.n[P] * stP); d[1] = across(2 * P + 1, -G.n[P] * stP);
+        d[2] = across(2 * Q, G.n[Q] * stQ); d[3] = across(2 * Q + 1, -G.n[Q] * stQ);
     }
-    if (j < G.n[1] + G.ng) {  // E^y at (i-1/2, j, k-1/2)
-        int64_t fz = fidx<2>(G, i, j, k), fx = fidx<0>(G, i, j, k);
-        double BzL, BzR, vxL, vxR, BxL, BxR, vzL, vzR;
-        rec6<REC>(bz + fz, sz_x, BzL, BzR);
-        rec6<REC>(Vz + eo, 1, vxL, vxR);
-        rec6<REC>(bx + fx, sx_z, BxL, BxR);
-        rec6<REC>(Vx + ns + eo, sz, vzL, vzR);
-        double cmin_z = fmax(Vz[2 * ns + eo], Vz[2 * ns + eo - 1]);
-        double cmax_z = fmax(Vz[3 * ns + eo], Vz[3 * ns + eo - 1]);
-        double cmin_x = fmax(Vx[2 * ns + eo], Vx[2 * ns + eo - sz]);
-        double cmax_x = fmax(Vx[3 * ns + eo], Vx[3 * ns + eo - sz]);
-        E[ns + eo] = hll(vxL * BzL, vxR * BzR, BzL, BzR, cmin_x, cmax_x) - hll(vzL * BxL, vzR * BxR, BxL, BxR, cmin_z, cmax_z);
+    const int mP = P == 0 ? i : (P == 1 ? j : k), mQ = Q == 0 ? i : (Q == 1 ? j : k);
+    const double *VP[6], *VQ[6];   // v^Q of the P faces along Q, v^P of the Q faces along P
+    face_line(a.V[P] + q * bs + SQ * ns + (eo >> 3), mQ, G.n[Q], G.ng, d[2], d[3], stQ, VP);
+    face_line(a.V[Q] + q * bs + SP * ns + (eo >> 3), mP, G.n[P], G.ng, d[0], d[1], stP, VQ);
+    const double* BP = a.B[P] + q * G.nface[P];
+    const double* BQ = a.B[Q] + q * G.nface[Q];
+    const uint32_t oP = (uint32_t)fidx<P>(G, i, j, k) * 8u, oQ = (uint32_t)fidx<Q>(G, i, j, k) * 8u;
+    const uint32_t sP = (uint32_t)bstride(P, Q) * 8u, sQ = (uint32_t)bstride(Q, P) * 8u;
+    double u[4][6], L[4], R[4];
+    // the four reconstructed fields
+    auto load = [&](int v, double* w, uint32_t z) {
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+            w[t] = v == 0   ? ld_off(BP, oP + (uint32_t)(t - 3) * sP + z)
+                   : v == 1 ? VP[t][z]
+                   : v == 2 ? ld_off(BQ, oQ + (uint32_t)(t - 3) * sQ + z)
+                            : VQ[t][z];
+    };
+#pragma unroll
+    for (int v = 0; v < 2; ++v) load(v, u[v], 0u);
+    const int64_t lQ = (2 - SP) * ns, lP = (2 - SQ) * ns;   // from those to the speeds
+    const double cminQ = fmax(VQ[3][lQ], VQ[2][lQ]), cmaxQ = fmax(VQ[3][lQ + ns], VQ[2][lQ + ns]);
+    const double cminP = fmax(VP[3][lP], VP[2][lP]), cmaxP = fmax(VP[3][lP + ns], VP[2][lP + ns]);
+    bool ok = true;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        if (v + 2 < 4) load(v + 2, u[v + 2], 0u);
+        __builtin_amdgcn_sched_barrier(0);
+        const double* w = u[v];
+        if constexpr (REC == 0) {
+            ok = wenoz_face(w[0], w[1], w[2], w[3], w[4], w[5], L[v], R[v]) && ok;
+            settle(L[v], R[v]);
+        } else recon<REC>(w[1], w[2], w[3], w[4], L[v], R[v]);
     }
-    if (k < G.n[2] + G.ng) {  // E^z at (i-1/2, j-1/2, k)
-        int64_t fx = fidx<0>(G, i, j, k), fy = fidx<1>(G, i, j, k);
-        double BxL, BxR, vyL, vyR, ByL, ByR, vxL, vxR;
-        rec6<REC>(bx + fx, sx_y, BxL, BxR);
-        rec6<REC>(Vx + eo, sy, vyL, vyR);
-        rec6<REC>(by + fy, sy_x, ByL, ByR);
-        rec6<REC>(Vy + eo, 1, vxL, vxR);
-        double cmin_x = fmax(Vx[2 * ns + eo], Vx[2 * ns + eo - sy]);
-        double cmax_x = fmax(Vx[3 * ns + eo], Vx[3 * ns + eo - sy]);
-        double cmin_y = fmax(Vy[2 * ns + eo], Vy[2 * ns + eo - 1]);
-        double cmax_y = fmax(Vy[3 * ns + eo], Vy[3 * ns + eo - 1]);
-        E[2 * ns + eo] = hll(vyL * BxL, vyR * BxR, BxL, BxR, cmin_y, cmax_y) - hll(vxL * ByL, vxR * ByR, ByL, ByR, cmin_x, cmax_x);
+    if constexpr (REC == 0)
+        if (!ok) {
+            uint32_t again = 0;
+            asm volatile("" : "+v"(again));
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                load(v, u[0], again);
+                wenoz_face_wide(u[0][0], u[0][1], u[0][2], u[0][3], u[0][4], u[0][5], L[v], R[v]);
+                settle(L[v], R[v]);
+            }
+        }
+    const double E = hll_r(L[1] * L[0], R[1] * R[0], L[0], R[0], cminQ, cmaxQ, nr_rcp(cmaxQ + cminQ)) -
+                     hll_r(L[3] * L[2], R[3] * R[2], L[2], R[2], cminP, cmaxP, nr_rcp(cmaxP + cminP));
+    a.emf[(q * 3 + C) * ns + (eo >> 3)] = E;
+}
+
+// The three components of a block follow each other, then the next block's
+// (as in k_flux: they read the same face values, from one XCD's L2).
+// Bound by the vector units (about 600 instructions per edge, 140 us for 512
+// blocks of 16^3) and the L1 (rows of 17 edges: 20 line accesses per load of
+// a wave, about as long) together: 195 us there, 50 for 125 blocks; 7 for 8
+// blocks, where one thread per edge triple took 14.  Two fields are loaded
+// ahead of the one that is reconstructed: all four at once spill at four
+// waves per SIMD (270 us) and leave three without the bound (214).
+template <int REC>
+__global__ __launch_bounds__(256, 4) void k_emf_uct(DevGrid G, EmfArgs a) {
+    const WgPos wp = wg_pos(a.tiles * 3);
+    int t, c;
+    udivmod(wp.tile, 3, t, c);
+    const int e = t * (int)blockDim.x + (int)threadIdx.x;
+    switch (c) {
+        case 0: emf_edge<REC, 0>(G, a, wp.q, e); break;
+        case 1: emf_edge<REC, 1>(G, a, wp.q, e); break;
+        default: emf_edge<REC, 2>(G, a, wp.q, e); break;
     }
 }
 
@@ -1428,14 +1482,14 @@ struct grmhd_ctx {
     DevStats* noalloc_part = nullptr;         // device address of `scratch` on this context's device
     unsigned long long* fatal_d = nullptr;    // fatal c2p cells since the last sync point (Opts::fatal_count)
     double* dt_scalar = nullptr;              // dt of the host-dt entry points
-    // ring faces written by the neighbouring block's face threads: per block
-    // the face neighbours (-1 beyond an outflow face) and the mask of block
-    // faces beyond which k_flux computes the ring itself; null when off
+    // ring faces taken from the neighbouring block's interior faces: per
+    // block the face neighbours (-1 beyond an outflow face) and the mask of
+    // block faces beyond which k_flux computes the ring itself; null when off
     int32_t* ring_nbr = nullptr;
     uint8_t* ring_own = nullptr;
     bool ring_any = false;                    // some block has such a face
     // set by the RK3 step around the flux launches of its second and third
-    // stages: their ring faces come from the neighbours' pushes and their
+    // stages: their ring faces are the neighbours' interior faces and their
     // full faces read the cells beyond a block face from the neighbour's
     // interior, so the gathers between stages leave the face slabs alone
     // (the first stage and grmhd_advance_substep read the caller's ghosts and
@@ -2122,7 +2176,7 @@ static void launch_flux(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s,
     const bool uct = c->P.emf != GRMHD_EMF_GS;
     static const char* fam[3] = {"flux_x", "flux_y", "flux_z"};
     f.ring_own = c->ring_copy_now ? c->ring_own : nullptr;
-    f.push_nbr = f.ring_own ? c->ring_nbr : nullptr;
+    f.nbr = f.ring_own ? c->ring_nbr : nullptr;
     f.ndir = c->timing ? 1 : 3;
     for (f.dir0 = 0; f.dir0 < 3; f.dir0 += f.ndir) {
         Scope sc(c, fam[f.dir0], s);
@@ -2178,7 +2232,7 @@ static void site_launch(const DevGrid& G, int bs, F&& f) {
     const int wpb = (int)nblk_bs(sites, bs);
     f(dim3((unsigned)(wpb * G.nq)), wpb);
 }
-static void launch_emf(grmhd_ctx* c, const double* const B[3], hipStream_t s) {
+static void launch_emf(grmhd_ctx* c, const double* const B[3], bool share, hipStream_t s) {
     Scope sc(c, "emf", s);
     const DevGrid& G = c->G;
     if (c->P.emf == GRMHD_EMF_GS) {
@@ -2190,14 +2244,20 @@ static void launch_emf(grmhd_ctx* c, const double* const B[3], hipStream_t s) {
                                                                    nullptr, wide);
         return;
     }
-    site_launch(G, c->tune.emf, [&](dim3 g, int wpb) {
-        switch (c->P.recon) {
-            case 0: k_emf_uct<0><<<g, c->tune.emf, 0, s>>>(G, B[0], B[1], B[2], c->vbar[0], c->vbar[1], c->vbar[2], c->emf, wpb); break;
-            case 1: k_emf_uct<1><<<g, c->tune.emf, 0, s>>>(G, B[0], B[1], B[2], c->vbar[0], c->vbar[1], c->vbar[2], c->emf, wpb); break;
-            case 2: k_emf_uct<2><<<g, c->tune.emf, 0, s>>>(G, B[0], B[1], B[2], c->vbar[0], c->vbar[1], c->vbar[2], c->emf, wpb); break;
-            default: k_emf_uct<3><<<g, c->tune.emf, 0, s>>>(G, B[0], B[1], B[2], c->vbar[0], c->vbar[1], c->vbar[2], c->emf, wpb); break;
-        }
-    });
+    EmfArgs a{};
+    for (int d = 0; d < 3; ++d) { a.B[d] = B[d]; a.V[d] = c->vbar[d]; }
+    a.emf = c->emf;
+    a.nbr = share && c->ring_own ? c->ring_nbr : nullptr;
+    const int64_t n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
+    const int64_t edges = std::max(n0 * (n1 + 1) * (n2 + 1), std::max((n0 + 1) * n1 * (n2 + 1), (n0 + 1) * (n1 + 1) * n2));
+    a.tiles = (int)nblk_bs(edges, c->tune.emf);
+    const dim3 grid((unsigned)(a.tiles * 3 * G.nq));
+    switch (c->P.recon) {
+        case 0: k_emf_uct<0><<<grid, c->tune.emf, 0, s>>>(G, a); break;
+        case 1: k_emf_uct<1><<<grid, c->tune.emf, 0, s>>>(G, a); break;
+        case 2: k_emf_uct<2><<<grid, c->tune.emf, 0, s>>>(G, a); break;
+        default: k_emf_uct<3><<<grid, c->tune.emf, 0, s>>>(G, a); break;
+    }
 }
 static void launch_update(grmhd_ctx* c, UpdArgs& a, hipStream_t s) {
     Scope sc(c, "update", s);
@@ -2391,7 +2451,7 @@ extern "C" grmhd_status grmhd_advance_substep(grmhd_ctx* c, const double* dt_dev
     if (!c || !dt_dev || !new_state || !old_state || !new_B || !old_B || !aux) { set_err("null argument"); return GRMHD_ERR_INVALID; }
     hipStream_t s = (hipStream_t)stream;
     launch_fluxes(c, aux, old_state, NSTATE, old_B, s);
-    launch_emf(c, old_B, s);
+    launch_emf(c, old_B, false, s);
     if (c->P.fofc)
         launch_fofc(c, new_state, NSTATE, nullptr, 0, 1.0, 0.0, old_state, old_B, aux, dt_dev, dtfact, s);
     launch_reflux(c, s);
@@ -2844,7 +2904,7 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
             fork(6, s, c->side);
             launch_reflux(c, c->side, 1);
         }
-        launch_emf(c, S.oB, s);
+        launch_emf(c, S.oB, sidx > 0, s);
         if (c->P.fofc)
             launch_fofc(c, S.ast, S.anv, S.bst, S.bnv, S.ca, S.cb, state, S.oB, aux, dt_dev, S.dtf, s);
         launch_reflux(c, s, split_update ? 2 : 0);
@@ -3048,7 +3108,7 @@ extern "C" grmhd_status grmhd_autotune(grmhd_ctx* c, const double* state, const 
     grmhd_tuning keep = c->tune;
     const bool conc = stage_conc(c);
     // the flux launch in the form of the second and third RK stages (ring
-    // faces pushed, reads across block faces) when the context shares ring
+    // faces left to their blocks, reads across block faces) when the context shares ring
     // faces; one workgroup size for its three directions
     {
         int v = c->tune.flux[0];
@@ -3075,13 +3135,13 @@ extern "C" grmhd_status grmhd_autotune(grmhd_ctx* c, const double* state, const 
             UpdArgs uc = u;
             uc.part = 1;
             launch_update(c, uc, c->side);
-            launch_emf(c, Bc, s);
+            launch_emf(c, Bc, true, s);
             u.part = 2;
             launch_update(c, u, s);
             (void)hipEventRecord(c->fev[1], c->side);
             (void)hipStreamWaitEvent(s, c->fev[1], 0);
         } else {
-            launch_emf(c, Bc, s);
+            launch_emf(c, Bc, true, s);
             launch_update(c, u, s);
         }
     };

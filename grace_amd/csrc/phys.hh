@@ -1085,58 +1085,12 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
 
 // ---- reconstruction ----------------------------------------------------------
 // u0..u5 = u(i-3..i+2); uL at i-1/2-eps, uR at i-1/2+eps
-// WENO-Z (weno_reconstruction.hh:172-278).  Per side, the three ratios
-// t5/(b_k+eps) come from one reciprocal of d0 d1 d2 (d_k >= 1e-42, so the
-// product cannot underflow), and the two sides of a face share their
-// reciprocals: 1/(P_R P_L) gives 1/P_R and 1/P_L, 1/(S_R S_L) the two
-// normalisations (guarded against overflow of the products, which falls back
-// to separate divisions).  This differs from the reference's three divisions
-// per weight by a few ulp.
-struct WenoSide { double q0, q1, q2; double P; };
-GHD void weno_betas(double b0, double b1, double b2, double& d0, double& d1, double& d2, double& t5) {
-    const double eps = 1.0e-42;
-    d0 = b0 + eps; d1 = b1 + eps; d2 = b2 + eps;
-    t5 = fabs(b0 - b2);
-}
-GHD void wenoz(double um3, double um2, double um1, double u0, double up1, double up2, double& uL, double& uR) {
-    const double c0 = 13.0 / 12.0, c1 = 0.25;
-    // right state (cell i stencils; a0 pairs with i2, a2 with i0 on this side)
-    const double rb0 = c0 * sq(um2 + u0 - 2.0 * um1) + c1 * sq(um2 + 3.0 * u0 - 4.0 * um1);
-    const double rb1 = c0 * sq(um1 + up1 - 2.0 * u0) + c1 * sq(um1 - up1);
-    const double rb2 = c0 * sq(up2 + u0 - 2.0 * up1) + c1 * sq(up2 + 3.0 * u0 - 4.0 * up1);
-    // left state (cell i-1 stencils)
-    const double lb0 = c0 * sq(um3 + um1 - 2.0 * um2) + c1 * sq(um3 + 3.0 * um1 - 4.0 * um2);
-    const double lb1 = c0 * sq(um2 + u0 - 2.0 * um1) + c1 * sq(um2 - u0);
-    const double lb2 = c0 * sq(up1 + um1 - 2.0 * u0) + c1 * sq(up1 + 3.0 * um1 - 4.0 * u0);
-    double rd0, rd1, rd2, rt, ld0, ld1, ld2, lt;
-    weno_betas(rb2, rb1, rb0, rd0, rd1, rd2, rt);
-    weno_betas(lb0, lb1, lb2, ld0, ld1, ld2, lt);
-    const double rP01 = rd0 * rd1, rP = rP01 * rd2, lP01 = ld0 * ld1, lP = lP01 * ld2;
-    double rr, lr;
-    const double PP = rP * lP;
-    // PP >= 1e-252 (every d >= 1e-42): a normal, finite reciprocal
-    if (PP < 1e300) { const double inv = nr_rcp(PP); rr = rt * lP * inv; lr = lt * rP * inv; }
-    else { rr = rt / rP; lr = lt / lP; }
-    const double rq0 = rd1 * rd2 * rr, rq1 = rd0 * rd2 * rr, rq2 = rP01 * rr;
-    const double lq0 = ld1 * ld2 * lr, lq1 = ld0 * ld2 * lr, lq2 = lP01 * lr;
-    const double ra0 = 0.1 * (1.0 + rq0 * rq0), ra1 = 0.6 * (1.0 + rq1 * rq1), ra2 = 0.3 * (1.0 + rq2 * rq2);
-    const double la0 = 0.1 * (1.0 + lq0 * lq0), la1 = 0.6 * (1.0 + lq1 * lq1), la2 = 0.3 * (1.0 + lq2 * lq2);
-    const double rn = (2.0 * up2 - 7.0 * up1 + 11.0 * u0) * ra0 + (-1.0 * up1 + 5.0 * u0 + 2.0 * um1) * ra1 +
-                      (2.0 * u0 + 5.0 * um1 - um2) * ra2;
-    const double ln = (2.0 * um3 - 7.0 * um2 + 11.0 * um1) * la0 + (-1.0 * um2 + 5.0 * um1 + 2.0 * u0) * la1 +
-                      (2.0 * um1 + 5.0 * u0 - up1) * la2;
-    const double rS = 6.0 * (ra0 + ra1 + ra2), lS = 6.0 * (la0 + la1 + la2);
-    const double SS = rS * lS;
-    // SS >= 36 (every a >= its linear weight)
-    if (SS < 1e300) { const double inv = nr_rcp(SS); uR = rn * lS * inv; uL = ln * rS * inv; }
-    else { uR = rn / rS; uL = ln / lS; }
-}
-// WENO-Z from the cell's side: both face values of the cell of u0 (its lower
-// face's right state and its upper face's left state) from um2..up2.  The
-// candidates pair with the linear weights in opposite order.  Everything is
-// formed from the four differences of neighbours, and a face value is u0 plus
-// a correction, so that smooth data lose no digits to the candidates' large
-// coefficients.  The multiply-adds are written out: a value that two blocks
+// WENO-Z (weno_reconstruction.hh:172-278) from the cell's side: both face
+// values of the cell of u0 (its lower face's right state and its upper face's
+// left state) from um2..up2.  The candidates pair with the linear weights in
+// opposite order.  Everything is formed from the four differences of
+// neighbours, and a face value is u0 plus a correction, so that smooth data
+// lose no digits to the candidates' large coefficients.  The multiply-adds are written out: a value that two blocks
 // form (a face on their common boundary) then has the same bits wherever this
 // is inlined.  Here every ratio is divided by itself (values of any size):
 // the wide form, taken where wenoz_face says so.
@@ -1211,11 +1165,11 @@ GHD double mc2(double sL, double sR) {
 GHD double minmod(double sL, double sR) {
     return 0.5 * (copysign(1.0, sL) + copysign(1.0, sR)) * fmin(fabs(sL), fabs(sR));
 }
+// MC2, minmod, donor cell: both states of the face between um1 and u0
 template <int REC>
-GHD void recon(double um3, double um2, double um1, double u0, double up1, double up2, double& uL, double& uR) {
-    if constexpr (REC == 0) {
-        wenoz(um3, um2, um1, u0, up1, up2, uL, uR);
-    } else if constexpr (REC == 3) {
+GHD void recon(double um2, double um1, double u0, double up1, double& uL, double& uR) {
+    static_assert(REC >= 1 && REC <= 3, "WENO-Z is wenoz_face");
+    if constexpr (REC == 3) {
         uL = um1; uR = u0;
     } else {
         double sL = u0 - um1, sR = up1 - u0;
