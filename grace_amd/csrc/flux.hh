@@ -281,7 +281,7 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
     const double Bf = ld_off(f.B[D] + q * nf, (uint32_t)fidx<D>(G, i, j, k) * 8u);
     // (scalar registers; -1: none)
     int32_t nl = -1, nh = -1;
-    if (FLAT && !ring && f.nbr) {
+    if (!ring && f.nbr) {
         nl = __builtin_amdgcn_readfirstlane(f.nbr[q * 6 + 2 * D]);
         nh = __builtin_amdgcn_readfirstlane(f.nbr[q * 6 + 2 * D + 1]);
     }

@@ -1488,6 +1488,8 @@ struct grmhd_ctx {
     int32_t* ring_nbr = nullptr;
     uint8_t* ring_own = nullptr;
     bool ring_any = false;                    // some block has such a face
+    int32_t* metric_diff = nullptr;           // device flag of k_metric_diff
+    bool metric_same = false;                 // its outcome for mder_src
     // set by the RK3 step around the flux launches of its second and third
     // stages: their ring faces are the neighbours' interior faces and their
     // full faces read the cells beyond a block face from the neighbour's
@@ -1631,7 +1633,7 @@ static void free_ctx(grmhd_ctx* c) {
     F(c->ftag[0]); F(c->ftag[1]); F(c->ftag[2]); F(c->etag); F(c->mder);
     F(c->fmet[0]); F(c->fmet[1]); F(c->fmet[2]);
     F(c->cmap_d); F(c->fblk_d); F(c->amr_cells); F(c->amr_faces); F(c->amr_faces_mid); F(c->rflux); F(c->remf);
-    F(c->vcm); F(c->fatal_d); F(c->dt_scalar); F(c->ring_nbr); F(c->ring_own);
+    F(c->vcm); F(c->fatal_d); F(c->dt_scalar); F(c->ring_nbr); F(c->ring_own); F(c->metric_diff);
     for (int d = 0; d < 3; ++d) { F(c->flux[d]); F(c->vbar[d]); F(c->B1[d]); F(c->B2[d]); }
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
     if (c->graph) (void)hipGraphDestroy(c->graph);
@@ -1806,12 +1808,11 @@ static grmhd_status ctx_create_impl(const grmhd_params* p, const grmhd_grid* g, 
     // 2-D c2p grids with workgroups down to 64 threads, plus per-launch rounding
     c->n_part_cap = nblk_bs(G.ncell * G.nq, 64) + 2 * G.nq + 2;
     if ((e = hipMalloc(&c->stats_part, sizeof(DevStats) * c->n_part_cap)) != hipSuccess) return fail("stats part", e);
-    if (!fin && p->emf == GRMHD_EMF_UCT && !p->fofc && p->flat_metric && G.n[0] >= G.ng && G.n[1] >= G.ng &&
-        G.n[2] >= G.ng) {
+    if (!fin && p->emf == GRMHD_EMF_UCT && !p->fofc && G.n[0] >= G.ng && G.n[1] >= G.ng && G.n[2] >= G.ng) {
         // Ring faces whose ghost side has a neighbouring block are that
-        // block's interior faces; with a flat metric every input of those
-        // faces is a copy on both sides (ghost metric values from the caller
-        // could differ in the last bit from the neighbour's, hence flat only).
+        // block's interior faces: every input of those faces is a copy on
+        // both sides, with a curved metric where the caller's ghost values are
+        // the neighbours' to the last bit (see ring_shared).
         std::vector<int32_t> nbr((size_t)g->nq * 6, -1);
         std::vector<uint8_t> own((size_t)g->nq, 0);
         for (int64_t q = 0; q < g->nq; ++q) {
@@ -2247,7 +2248,7 @@ static void launch_emf(grmhd_ctx* c, const double* const B[3], bool share, hipSt
     EmfArgs a{};
     for (int d = 0; d < 3; ++d) { a.B[d] = B[d]; a.V[d] = c->vbar[d]; }
     a.emf = c->emf;
-    a.nbr = share && c->ring_own ? c->ring_nbr : nullptr;
+    a.nbr = share ? c->ring_nbr : nullptr;
     const int64_t n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
     const int64_t edges = std::max(n0 * (n1 + 1) * (n2 + 1), std::max((n0 + 1) * n1 * (n2 + 1), (n0 + 1) * (n1 + 1) * n2));
     a.tiles = (int)nblk_bs(edges, c->tune.emf);
@@ -2689,6 +2690,32 @@ extern "C" grmhd_status grmhd_mlp_fit_cells(grmhd_ctx* c, grmhd_mlp* mlp, const 
     return st;
 }
 
+// Compares the metric of every cell beyond a block face that has a neighbour
+// (ng layers, all transverse indices) with the neighbour's cell at the same
+// position, bit by bit; *diff becomes 1 where one differs.
+__global__ __launch_bounds__(256) void k_metric_diff(DevGrid G, const double* __restrict__ state, int nv,
+                                                     const int32_t* __restrict__ nbr, int per, int32_t* diff) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t qs = t / per, q = qs / 6;
+    const int side = (int)(qs - q * 6), d = side >> 1, e = (int)(t - qs * per);
+    if (q >= G.nq) return;
+    const int32_t qn = nbr[q * 6 + side];
+    const int E0 = d == 0 ? G.ng : G.N[0], E1 = d == 1 ? G.ng : G.N[1], E2 = d == 2 ? G.ng : G.N[2];
+    if (qn < 0 || e >= E0 * E1 * E2) return;
+    int r, x[3];
+    udivmod(e, E0, r, x[0]);
+    udivmod(r, E1, x[2], x[1]);
+    if (side & 1) x[d] += G.n[d] + G.ng;
+    const int64_t st = d == 0 ? 1 : (d == 1 ? G.N[0] : (int64_t)G.N[0] * G.N[1]);
+    const int64_t c = cidx(G, x[0], x[1], x[2]), o = c + ((side & 1) ? -G.n[d] : G.n[d]) * st;
+    const double* A = state + q * nv * G.ncell + c;
+    const double* B = state + qn * nv * G.ncell + o;
+    bool bad = false;
+    for (int v = GXX_; v <= BETAZ_; ++v)
+        bad |= __double_as_longlong(A[v * G.ncell]) != __double_as_longlong(B[v * G.ncell]);
+    if (bad) *diff = 1;
+}
+
 extern "C" grmhd_status grmhd_set_static_metric(grmhd_ctx* c, const double* state, int32_t enable,
                                                 grmhd_stream_t stream) {
     if (!c || (enable && !state)) { set_err("invalid set_static_metric arguments"); return GRMHD_ERR_INVALID; }
@@ -2715,6 +2742,19 @@ extern "C" grmhd_status grmhd_set_static_metric(grmhd_ctx* c, const double* stat
         else k_face_metric<2><<<grid, 256, 0, s>>>(G, state, NSTATE, c->O.ex.alp_ex, c->fmet[2], wpb);
     }
     c->mder_src = state;
+    c->metric_same = false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (c->ring_own && hipStreamIsCapturing((hipStream_t)stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+        const hipStream_t s = (hipStream_t)stream;
+        if (!c->metric_diff) HIP_TRY(hipMalloc(&c->metric_diff, sizeof(int32_t)));
+        const int per = G.ng * (int)std::max((int64_t)G.N[0] * G.N[1], std::max((int64_t)G.N[0] * G.N[2], (int64_t)G.N[1] * G.N[2]));
+        int32_t diff = 0;
+        HIP_TRY(hipMemsetAsync(c->metric_diff, 0, sizeof(int32_t), s));
+        k_metric_diff<<<nblk((int64_t)per * 6 * G.nq), 256, 0, s>>>(G, state, NSTATE, c->ring_nbr, per, c->metric_diff);
+        HIP_TRY(hipMemcpyAsync(&diff, c->metric_diff, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        c->metric_same = diff == 0;
+    }
     return launch_check("metric_der");
 }
 
@@ -2838,6 +2878,15 @@ static grmhd_status ensure_stage_buffers(grmhd_ctx* c) {
     return GRMHD_OK;
 }
 
+// Whether the second and third RK stages take ring faces, and cells beyond
+// block faces, from the neighbouring blocks.  With a curved metric only for
+// the array whose cached metric (grmhd_set_static_metric) was found to agree
+// with itself across block faces: the ring faces are 43% of the faces of 16^3
+// blocks, and the gathers between stages fall away with them.
+static bool ring_shared(const grmhd_ctx* c, const double* state) {
+    return c->ring_own && (c->P.flat_metric || (c->metric_same && state == c->mder_src));
+}
+
 // Whether the independent launches of a stage run on a side stream beside the
 // main one, from 2^18 interior cells on.  Below, a launch does not fill the
 // card for longer than a fork and a join cost, and one stream also lets
@@ -2885,14 +2934,14 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
     // Ordering by events, so the same sequence is captured into the step's
     // graph.  (Small grids, see stage_conc, grmhd_params.stage_streams = 0 or
     // per-family timing: every launch on s.)
-    const bool conc = stage_conc(c) && !c->timing;
+    const bool conc = stage_conc(c) && !c->timing, share = ring_shared(c, state);
     auto fork = [&](int k, hipStream_t from, hipStream_t to) {
         (void)hipEventRecord(c->fev[k], from);
         (void)hipStreamWaitEvent(to, c->fev[k], 0);
     };
     for (int sidx = 0; sidx < 3; ++sidx) {
         Stage& S = st[sidx];
-        c->ring_copy_now = sidx > 0;
+        c->ring_copy_now = share && sidx > 0;
         launch_fluxes(c, aux, state, NSTATE, S.oB, s);
         c->ring_copy_now = false;
         // the cell part of the update needs only the fluxes (on a forest
@@ -2904,7 +2953,7 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
             fork(6, s, c->side);
             launch_reflux(c, c->side, 1);
         }
-        launch_emf(c, S.oB, sidx > 0, s);
+        launch_emf(c, S.oB, share && sidx > 0, s);
         if (c->P.fofc)
             launch_fofc(c, S.ast, S.anv, S.bst, S.bnv, S.ca, S.cb, state, S.oB, aux, dt_dev, S.dtf, s);
         launch_reflux(c, s, split_update ? 2 : 0);
@@ -2928,7 +2977,7 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
         // shared ring faces the next edge EMFs and the ring faces beyond
         // outflow faces read only the face slabs, the ghost cells beyond
         // outflow faces their own faces
-        const bool faces_slab = sidx < 2 && c->ring_own != nullptr;
+        const bool faces_slab = sidx < 2 && share;
         if (conc) {
             // side: ghost faces, then (after the conserved fills on s) the
             // c2p of the ghosts that run their own; s: conserved fills,
@@ -2977,7 +3026,7 @@ static void rk3_launches(grmhd_ctx* c, const double* dt_dev, double* state, doub
             // block face from the neighbour's interior: of the ghost
             // primitives it reads only those beyond outflow faces, which
             // run their own c2p or copy a first-layer ghost
-            g.copies_only = !last && c->ring_own != nullptr;
+            g.copies_only = !last && share;
             launch_gather(c, g, s);
         }
     }
@@ -3114,7 +3163,7 @@ extern "C" grmhd_status grmhd_autotune(grmhd_ctx* c, const double* state, const 
         int v = c->tune.flux[0];
         pick(&v, [&] {
             for (int d = 0; d < 3; ++d) c->tune.flux[d] = v;
-            c->ring_copy_now = c->ring_own != nullptr;
+            c->ring_copy_now = ring_shared(c, state);
             launch_fluxes(c, aux, state, NSTATE, Bc, s);
             c->ring_copy_now = false;
         });
@@ -3135,13 +3184,13 @@ extern "C" grmhd_status grmhd_autotune(grmhd_ctx* c, const double* state, const 
             UpdArgs uc = u;
             uc.part = 1;
             launch_update(c, uc, c->side);
-            launch_emf(c, Bc, true, s);
+            launch_emf(c, Bc, ring_shared(c, state), s);
             u.part = 2;
             launch_update(c, u, s);
             (void)hipEventRecord(c->fev[1], c->side);
             (void)hipStreamWaitEvent(s, c->fev[1], 0);
         } else {
-            launch_emf(c, Bc, true, s);
+            launch_emf(c, Bc, ring_shared(c, state), s);
             launch_update(c, u, s);
         }
     };

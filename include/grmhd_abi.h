@@ -329,7 +329,11 @@ grmhd_status grmhd_rk3_step_graph(grmhd_ctx* ctx, const double* dt_dev, double* 
  * z face), and the update and flux kernels of calls whose metric
  * source is that same array then read them instead (results
  * bit-identical).  The cache is not refreshed automatically: call again
- * after changing the metric in that array, or enable = 0 to drop it.
+ * after changing the metric in that array, or enable = 0 to drop it.  On a
+ * uniform grid with UCT the call also compares the metric in the ghost cells
+ * between blocks with the neighbours' interior (and waits for the stream to
+ * do so, unless it is capturing): where they agree to the last bit, the later
+ * stages of an RK3 step take those faces from the neighbouring blocks.
  * No effect for flat_metric.  Invalidates a captured RK3 graph. */
 grmhd_status grmhd_set_static_metric(grmhd_ctx* ctx, const double* state, int32_t enable, grmhd_stream_t stream);
 

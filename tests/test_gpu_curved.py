@@ -76,6 +76,34 @@ def test_gpu_static_metric_cache_bit_identical(dev):
         assert np.array_equal(res[0][1][d], res[1][1][d])
 
 
+@pytest.mark.parametrize("n,ngz,nb", [(16, 3, (2, 2, 2)), (7, 3, (3, 3, 3)), (5, 4, (2, 2, 2))])
+@pytest.mark.parametrize("ghost", ["agrees", "differs"])
+def test_gpu_static_metric_shared_faces(dev, n, ngz, nb, ghost):
+    """With a cached metric the later stages take ring faces and cells beyond
+    block faces from the neighbouring blocks, if the ghost metric agrees with
+    theirs; a single ghost value one bit off keeps the block's own.  Either
+    way the bits of the step without the cache."""
+    import torch
+    wl = W.blast_ks(nb=nb, n=n, ngz=ngz)
+    if ghost == "differs":
+        g = wl.state[0, ga.ALP]
+        at = (ngz + 1, ngz + 1, ngz + n)           # a ghost cell shared with block 1
+        g[at] = np.nextafter(g[at], 2.0)
+    dt = torch.tensor([0.2 * wl.extra["dx"]], dtype=torch.float64, device=dev)
+    res = []
+    for cache in (False, True):
+        ctx = ga.Context(wl.params, wl.grid, wl.instances)
+        sg, Bg, ag = dev_arrays(wl, dev)
+        if cache:
+            ctx.set_static_metric(sg)
+        for _ in range(2):
+            ctx.rk3_step(dt, sg, Bg, ag)
+        torch.cuda.synchronize()
+        res.append([sg, *Bg, ag])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
 def test_gpu_torus_rk3(dev):
     """Fishbone-Moncrief torus around a spin-0.9375 hole (the hole, its
     excised ring region, the atmosphere and the magnetised torus all on a
