@@ -392,8 +392,9 @@ __global__ __launch_bounds__(256, FLAT ? 3 : 2) void k_flux(DevGrid G, EOS eos, 
 
 // FOFC correction (evolve.cpp:646-702): the tagged faces of the normal range
 // [ng, n + ng], every transverse index, from donor cells with the options o
-// (LLF); one thread per face, x across the lanes.
-template <typename EOS, bool FLAT, int D>
+// (LLF); one thread per face, x across the lanes.  Flat metric; a curved one
+// takes k_flux_gs_curved.
+template <typename EOS, int D>
 __global__ __launch_bounds__(256) void k_flux_tagged(DevGrid G, EOS eos, Opts o, FluxArgs f, const uint8_t* __restrict__ only) {
     const WgPos wp = wg_pos(f.tiles);
     const int64_t q = wp.q;
@@ -412,7 +413,7 @@ __global__ __launch_bounds__(256) void k_flux_tagged(DevGrid G, EOS eos, Opts o,
     const int64_t st = D == 0 ? 1 : (D == 1 ? G.N[0] : (int64_t)G.N[0] * G.N[1]);
     Met mf;
     bool excise;
-    face_met<FLAT, D>(G, f, o.ex.alp_ex, q, i, j, k, st, mf, excise);
+    face_met<true, D>(G, f, o.ex.alp_ex, q, i, j, k, st, mf, excise);
     const double* A = f.aux + q * NAUX * nc + cidx(G, i, j, k);
     double L[FQ_N], R[FQ_N], V[4], F[7];
 #pragma unroll
@@ -420,11 +421,172 @@ __global__ __launch_bounds__(256) void k_flux_tagged(DevGrid G, EOS eos, Opts o,
         const double* P = A + fq_aux<D>(v, o.thermo) * nc;
         L[v] = P[-st]; R[v] = P[0];
     }
-    face_solve<EOS, FLAT, D>(eos, o, mf, L, R, f.B[D][q * nf + fo] / mf.sqrtg, false, V, F);
+    face_solve<EOS, true, D>(eos, o, mf, L, R, f.B[D][q * nf + fo] / mf.sqrtg, false, V, F);
     const int64_t so = sidx(G, i, j, k);
     double* V0 = f.vbar[D] + q * 4 * G.ns + so;
     V0[0] = V[0]; V0[G.ns] = V[1];
     double* F0 = f.flux[D] + q * NHRSC * G.ns + so;
 #pragma unroll
     for (int v = 0; v < NHRSC; ++v) F0[v * G.ns] = F[v];
+}
+
+// Fluxes and face EMFs for GS on a curved metric, one thread per face of
+// direction D, every face (FOFC widens the normal range by one face on each
+// side; only: its correction pass, the tagged faces).  Every quotient is an
+// IEEE division and the wave speeds are get_cm_cp's, for the sign of the mass
+// flux (see c2p), which is why this path is not k_flux's.
+template <typename EOS, int REC, int D>
+__global__ __launch_bounds__(256) void k_flux_gs_curved(DevGrid G, EOS eos, Opts o, FluxArgs f,
+                                                        const uint8_t* __restrict__ only) {
+    const WgPos wp = wg_pos(f.tiles);
+    const int64_t q = wp.q;
+    const int e = wp.tile * (int)blockDim.x + (int)threadIdx.x;
+    constexpr int T0 = D == 0 ? 1 : 0, T1 = D == 2 ? 1 : 2;
+    const int N0 = G.N[T0], N1 = G.N[T1], Rg = G.n[D] + 1 + 2 * o.fofc;
+    if (e >= Rg * N0 * N1) return;
+    int a, b, c, r;
+    if (D == 0) { udivmod(e, Rg, r, a); udivmod(r, N0, c, b); }
+    else if (D == 1) { udivmod(e, N0, r, b); udivmod(r, Rg, c, a); }
+    else { udivmod(e, N0, r, b); udivmod(r, N1, a, c); }
+    a += G.ng - o.fofc;
+    const int i = D == 0 ? a : b, j = D == 1 ? a : (D == 0 ? b : c), k = D == 2 ? a : c;
+    if (only && (a < G.ng || a > G.ng + G.n[D] || !only[q * G.nface[D] + fidx<D>(G, i, j, k)])) return;
+    const int64_t nc = G.ncell;
+    const int64_t c0 = cidx(G, i, j, k);
+    const int64_t st = D == 0 ? 1 : (D == 1 ? G.N[0] : (int64_t)G.N[0] * G.N[1]);
+    const double* A = f.aux + q * NAUX * nc;
+    Met mf;
+    bool excise_override = false;
+    if (f.fmc[D]) {
+        // the face-metric cache: only the inverse component this direction
+        // uses (cmcp, the LLF speed limit) is kept
+        const int64_t nfd = G.nface[D];
+        const double* FM = f.fmc[D] + q * FMC * nfd + fidx<D>(G, i, j, k);
+        for (int a = 0; a < 6; ++a) { mf.g[a] = FM[a * nfd]; mf.gi[a] = 0.0; }
+        mf.gi[D == 0 ? 0 : (D == 1 ? 3 : 5)] = FM[6 * nfd];
+        for (int a = 0; a < 3; ++a) mf.beta[a] = FM[(7 + a) * nfd];
+        mf.alp = FM[10 * nfd];
+        mf.sqrtg = FM[11 * nfd];
+        excise_override = FM[12 * nfd] != 0.0;
+    } else {
+        face_metric(f.mstate + q * (int64_t)f.mnv * nc, nc, c0, st, o.ex.alp_ex, mf, excise_override);
+    }
+    // reconstruction of RHO Z(3) YE THERMO ENT B(3)
+    const int th_aux = o.thermo ? PRESS_ : TEMP_;
+    const int ridx[10] = {RHO_, ZVECX_, ZVECY_, ZVECZ_, YE_, th_aux, ENTROPY_, BX_, BY_, BZ_};
+    const int rloc[10] = {RHOL, ZXL, ZYL, ZZL, YEL, o.thermo ? PRESSL : TEMPL, ENTL, BXL, BYL, BZL};
+    double pL[NPRIM], pR[NPRIM];
+#pragma unroll
+    for (int v = 0; v < 10; ++v) {
+        // (the normal B component is replaced by the face value below)
+        if (v == 7 + D) { pL[rloc[v]] = 0.0; pR[rloc[v]] = 0.0; continue; }
+        double uL, uR;
+        const double* P = A + ridx[v] * nc + c0;
+        if (excise_override) { uL = P[-st]; uR = P[0]; }
+        else if constexpr (REC == 0) wenoz(P[-3 * st], P[-2 * st], P[-st], P[0], P[st], P[2 * st], uL, uR);
+        else recon<REC>(P[-2 * st], P[-st], P[0], P[st], uL, uR);
+        pL[rloc[v]] = uL; pR[rloc[v]] = uR;
+    }
+    double Bn = f.B[D][q * G.nface[D] + fidx<D>(G, i, j, k)] / mf.sqrtg;
+    pL[BXL + D] = Bn; pR[BXL + D] = Bn;
+    unsigned ee = 0;
+    if (o.thermo) {
+        double h, s;
+        pL[EPSL] = eos.eps_from_press(h, pL[CS2L], pL[TEMPL], s, pL[PRESSL], pL[RHOL], ee);
+        pR[EPSL] = eos.eps_from_press(h, pR[CS2L], pR[TEMPL], s, pR[PRESSL], pR[RHOL], ee);
+    } else {
+        pL[PRESSL] = eos.press_from_temp(pL[EPSL], pL[CS2L], pL[TEMPL], pL[RHOL], ee);
+        pR[PRESSL] = eos.press_from_temp(pR[EPSL], pR[CS2L], pR[TEMPL], pR[RHOL], ee);
+    }
+    // compute_mhd_fluxes (grmhd.hh:774-970)
+    const double *zl = &pL[ZXL], *zr = &pR[ZXL], *Bl = &pL[BXL], *Br = &pR[BXL];
+    double wl = lorentz<false>(mf.g, zl), wr = lorentz<false>(mf.g, zr);
+    double bl[4], br[4], b2l, b2r;
+    smallb<false>(mf, Bl, zl, wl, bl, b2l);
+    smallb<false>(mf, Br, zr, wr, br, b2r);
+    double vtl[3], vtr[3];
+    vtilde(mf, zl, wl, vtl);
+    vtilde(mf, zr, wr, vtr);
+    double cml, cpl, cmr, cpr, cmin, cmax;
+    cmcp<false>(mf, pL[RHOL], pL[PRESSL], pL[EPSL], pL[CS2L], wl, b2l, vtl, D, cml, cpl);
+    cmcp<false>(mf, pR[RHOL], pR[PRESSL], pR[EPSL], pR[CS2L], wr, b2r, vtr, D, cmr, cpr);
+    if (o.riemann == 1) {
+        cmax = fmax(fmax(fabs(cml), fabs(cmr)), fmax(fabs(cpl), fabs(cpr)));
+        if (fmin(pL[RHOL], pR[RHOL]) < o.c_limit) {
+            double gdd = D == 0 ? mf.gi[0] : (D == 1 ? mf.gi[3] : mf.gi[5]);
+            cmax = fmax(cmax, mf.alp * sqrt(gdd) + fabs(mf.beta[D]));
+        }
+        cmin = cmax;
+    } else {
+        cmin = -fmin(0., fmin(cml, cmr));
+        cmax = fmax(0., fmax(cpl, cpr));
+    }
+    if (cmin < 1e-12 && cmax < 1e-12) { cmin = 1; cmax = 1; }
+    const double ihll = 1.0 / (cmax + cmin);   // shared by the HLL fluxes of this face
+    const int64_t so = sidx(G, i, j, k), ns = G.ns;
+    double* V = f.vbar[D] + q * 4 * ns + so;
+    double Dl, taul, Sl[3], Esl, Dr, taur, Sr[3], Esr;
+    conserved<false>(mf, pL[RHOL], pL[PRESSL], pL[EPSL], zl, pL[ENTL], wl, b2l, bl, Dl, taul, Sl, Esl);
+    conserved<false>(mf, pR[RHOL], pR[PRESSL], pR[EPSL], zr, pR[ENTL], wr, b2r, br, Dr, taur, Sr, Esr);
+    // fluxes along D (grmhd_subexpressions.hh:97-156)
+    double bsh[3]; lower3(mf.g, mf.beta[0], mf.beta[1], mf.beta[2], bsh);
+    double ia2 = 1. / (mf.alp * mf.alp);
+    double Fl[7], Fr[7];
+    {
+        double rhoh = b2l + pL[EPSL] * pL[RHOL] + pL[PRESSL] + pL[RHOL];
+        double ps = 0.5 * b2l + pL[PRESSL];
+        double W2rh = wl * wl * rhoh;
+        double fD = vtl[D] * Dl;
+        Fl[0] = fD;
+        double blo[3]; lower3<false>(mf.g, bl[1], bl[2], bl[3], blo);
+        double vlo[3]; lower3<false>(mf.g, vtl[0], vtl[1], vtl[2], vlo);
+        Fl[4] = W2rh * vtl[D] + ps * mf.beta[D] - mf.alp * mf.alp * bl[0] * bl[1 + D] - fD;
+        const double c = vtl[D] * W2rh * ia2;
+        for (int a = 0; a < 3; ++a)
+            Fl[1 + a] = mf.alp * (-bl[1 + D] * (blo[a] + bl[0] * bsh[a]) + (a == D ? ps : 0.0) + c * (vlo[a] + bsh[a]));
+        Fl[6] = vtl[D] * Esl;
+        Fl[5] = pL[YEL] * fD;
+    }
+    {
+        double rhoh = b2r + pR[EPSL] * pR[RHOL] + pR[PRESSL] + pR[RHOL];
+        double ps = 0.5 * b2r + pR[PRESSL];
+        double W2rh = wr * wr * rhoh;
+        double fD = vtr[D] * Dr;
+        Fr[0] = fD;
+        double blo[3]; lower3<false>(mf.g, br[1], br[2], br[3], blo);
+        double vlo[3]; lower3<false>(mf.g, vtr[0], vtr[1], vtr[2], vlo);
+        Fr[4] = W2rh * vtr[D] + ps * mf.beta[D] - mf.alp * mf.alp * br[0] * br[1 + D] - fD;
+        const double c = vtr[D] * W2rh * ia2;
+        for (int a = 0; a < 3; ++a)
+            Fr[1 + a] = mf.alp * (-br[1 + D] * (blo[a] + br[0] * bsh[a]) + (a == D ? ps : 0.0) + c * (vlo[a] + bsh[a]));
+        Fr[6] = vtr[D] * Esr;
+        Fr[5] = pR[YEL] * fD;
+    }
+    double* F = f.flux[D] + q * NHRSC * ns + so;
+    const double sg = mf.sqrtg;
+    F[DENS_ * ns] = sg * hll_r(Fl[0], Fr[0], Dl, Dr, cmin, cmax, ihll);
+    F[ENTROPYSTAR_ * ns] = sg * hll_r(Fl[6], Fr[6], Esl, Esr, cmin, cmax, ihll);
+    F[TAU_ * ns] = sg * hll_r(Fl[4], Fr[4], taul, taur, cmin, cmax, ihll);
+    F[SX_ * ns] = sg * hll_r(Fl[1], Fr[1], Sl[0], Sr[0], cmin, cmax, ihll);
+    F[SY_ * ns] = sg * hll_r(Fl[2], Fr[2], Sl[1], Sr[1], cmin, cmax, ihll);
+    F[SZ_ * ns] = sg * hll_r(Fl[3], Fr[3], Sl[2], Sr[2], cmin, cmax, ihll);
+    F[YESTAR_ * ns] = sg * hll_r(Fl[5], Fr[5], pL[YEL] * Dl, pR[YEL] * Dr, cmin, cmax, ihll);
+    {  // face EMFs (grmhd.hh:937-969)
+        if (D == 0) {
+            double a = -Bl[0] * vtl[2] + Bl[2] * vtl[0], b = -Br[0] * vtr[2] + Br[2] * vtr[0];
+            V[0] = sg * hll_r(a, b, Bl[2], Br[2], cmin, cmax, ihll);
+            a = -Bl[0] * vtl[1] + Bl[1] * vtl[0]; b = -Br[0] * vtr[1] + Br[1] * vtr[0];
+            V[ns] = -sg * hll_r(a, b, Bl[1], Br[1], cmin, cmax, ihll);
+        } else if (D == 1) {
+            double a = -Bl[1] * vtl[2] + Bl[2] * vtl[1], b = -Br[1] * vtr[2] + Br[2] * vtr[1];
+            V[0] = -sg * hll_r(a, b, Bl[2], Br[2], cmin, cmax, ihll);
+            a = Bl[0] * vtl[1] - Bl[1] * vtl[0]; b = Br[0] * vtr[1] - Br[1] * vtr[0];
+            V[ns] = sg * hll_r(a, b, Bl[0], Br[0], cmin, cmax, ihll);
+        } else {
+            double a = Bl[1] * vtl[2] - Bl[2] * vtl[1], b = Br[1] * vtr[2] - Br[2] * vtr[1];
+            V[0] = sg * hll_r(a, b, Bl[1], Br[1], cmin, cmax, ihll);
+            a = Bl[0] * vtl[2] - Bl[2] * vtl[0]; b = Br[0] * vtr[2] - Br[2] * vtr[0];
+            V[ns] = -sg * hll_r(a, b, Bl[0], Br[0], cmin, cmax, ihll);
+        }
+    }
 }

@@ -850,7 +850,7 @@ __global__ __launch_bounds__(256) void k_fofc_flag(DevGrid G, EOS eos, Opts o, F
     C2PGuess gs{0, 0, 0, 0, 0, 0};
     C2PRoots rt{-1, -1, -1, -1};
     const double rad = o.ex.by_radius ? cell_radius(o.ex, I, a.blk[q].b, G.n, G.ng, i, j, k) : 1e300;
-    const C2POut out = c2p<FLAT>(cons, pr, m, eos, o.atmo, o.ex, cp, rad, err, true, cnt, gs, rt);
+    const C2POut out = c2p<FLAT, !FLAT>(cons, pr, m, eos, o.atmo, o.ex, cp, rad, err, true, cnt, gs, rt);
     if (!(out.floored || dmp)) return;
     for (int t = 0; t < 2; ++t) {
         a.ftag[0][q * nf0 + fidx<0>(G, i + t, j, k)] = 1;
@@ -1148,7 +1148,8 @@ enum { CS_INTERIOR = 0, CS_SHELL = 1, CS_LIST = 2, CS_STAGE = 3 };
 // previous primitives in aux, mu = 1/(h W) of the last c2p of this cell
 // (the previous RK stage, or the caller's data), at most warm_newton
 // evaluations before the plain path.
-template <typename EOS, bool FLAT, int GUESS = 0>
+// X: see c2p (GS on a curved metric).
+template <typename EOS, bool FLAT, int GUESS = 0, bool X = false>
 __global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_cells(DevGrid G, EOS eos, Opts o, const DevInst* __restrict__ inst,
                                                    const DevBlk* __restrict__ blk, double* st, int snv,
                                                    const double* __restrict__ mstate, int mnv,
@@ -1265,7 +1266,7 @@ __global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_cells(DevGrid G, EO
         A[BX_ * nc] = Bc0 / m.sqrtg; A[BY_ * nc] = Bc1 / m.sqrtg; A[BZ_ * nc] = Bc2 / m.sqrtg;
         C2PRoots rt{-1, -1, -1, -1};
         const double rad = o.ex.by_radius ? cell_radius(o.ex, inst[blk[q].inst], blk[q].b, G.n, G.ng, i, j, k) : 1e300;
-        out = c2p<FLAT>(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad, err, false, cnt, gs, rt);
+        out = c2p<FLAT, X>(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad, err, false, cnt, gs, rt);
         if (out.fatal && o.fatal_count) atomicAdd(o.fatal_count, 1ull);
         A[RHO_ * nc] = pr[RHOL]; A[EPS_ * nc] = pr[EPSL]; A[PRESS_ * nc] = pr[PRESSL];
         A[TEMP_ * nc] = pr[TEMPL]; A[ENTROPY_ * nc] = pr[ENTL]; A[YE_ * nc] = pr[YEL];
@@ -1356,7 +1357,7 @@ __global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_batch(int64_t n, EO
     C2PCount cnt;
     C2POut out{false, false};
     if (active) {
-        out = c2p<false>(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad ? rad[s] : 1e300, err, dry_run != 0, cnt, gs, rt);
+        out = c2p<false, false>(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad ? rad[s] : 1e300, err, dry_run != 0, cnt, gs, rt);
         if (out.fatal && o.fatal_count) atomicAdd(o.fatal_count, 1ull);
         if (roots) { roots[s] = rt.x_e; roots[n + s] = rt.x_s; roots[2 * n + s] = rt.m_e; roots[3 * n + s] = rt.m_s; }
         for (int v = 0; v < NPRIM; ++v) prims[v * n + s] = pr[v];
@@ -2155,7 +2156,7 @@ static FluxArgs flux_args(grmhd_ctx* c, const double* aux, const double* ms, int
     }
     return f;
 }
-template <typename EOS, bool FLAT>
+template <typename EOS>
 static void launch_flux_tagged(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O,
                                uint8_t* const* only) {
     const DevGrid& G = c->G;
@@ -2165,9 +2166,27 @@ static void launch_flux_tagged(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStre
         const int bs = c->tune.flux[d];
         f.tiles = (int)nblk_bs(n, bs);
         const dim3 grid((unsigned)(f.tiles * G.nq));
-        if (d == 0) k_flux_tagged<EOS, FLAT, 0><<<grid, bs, 0, s>>>(G, eos, O, f, only[0]);
-        else if (d == 1) k_flux_tagged<EOS, FLAT, 1><<<grid, bs, 0, s>>>(G, eos, O, f, only[1]);
-        else k_flux_tagged<EOS, FLAT, 2><<<grid, bs, 0, s>>>(G, eos, O, f, only[2]);
+        if (d == 0) k_flux_tagged<EOS, 0><<<grid, bs, 0, s>>>(G, eos, O, f, only[0]);
+        else if (d == 1) k_flux_tagged<EOS, 1><<<grid, bs, 0, s>>>(G, eos, O, f, only[1]);
+        else k_flux_tagged<EOS, 2><<<grid, bs, 0, s>>>(G, eos, O, f, only[2]);
+    }
+}
+// GS on a curved metric: one launch per direction (only: the FOFC pass).
+template <typename EOS, int REC>
+static void launch_flux_gs_curved(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O,
+                                  uint8_t* const* only) {
+    const DevGrid& G = c->G;
+    static const char* fam[3] = {"flux_x", "flux_y", "flux_z"};
+    for (int d = 0; d < 3; ++d) {
+        Scope sc(c, only ? "fofc" : fam[d], s);
+        const int64_t n = (int64_t)(G.n[d] + 1 + 2 * O.fofc) * G.N[(d + 1) % 3] * G.N[(d + 2) % 3];
+        const int bs = c->tune.flux[d];
+        f.tiles = (int)nblk_bs(n, bs);
+        const dim3 grid((unsigned)(f.tiles * G.nq));
+        const uint8_t* od = only ? only[d] : nullptr;
+        if (d == 0) k_flux_gs_curved<EOS, REC, 0><<<grid, bs, 0, s>>>(G, eos, O, f, od);
+        else if (d == 1) k_flux_gs_curved<EOS, REC, 1><<<grid, bs, 0, s>>>(G, eos, O, f, od);
+        else k_flux_gs_curved<EOS, REC, 2><<<grid, bs, 0, s>>>(G, eos, O, f, od);
     }
 }
 // The three directions in one launch; one by one where each is timed.
@@ -2198,7 +2217,17 @@ template <typename EOS, bool FLAT>
 static void flux_rec(grmhd_ctx* c, const EOS& eos, const double* aux, const double* ms, int mnv,
                      const double* const B[3], hipStream_t s, int recon, const Opts& O, uint8_t* const* only) {
     const FluxArgs f = flux_args(c, aux, ms, mnv, B);
-    if (only) { launch_flux_tagged<EOS, FLAT>(c, eos, f, s, O, only); return; }
+    if constexpr (!FLAT) {
+        if (c->P.emf == GRMHD_EMF_GS) {
+            switch (recon) {
+                case 0: launch_flux_gs_curved<EOS, 0>(c, eos, f, s, O, only); break;
+                case 1: launch_flux_gs_curved<EOS, 1>(c, eos, f, s, O, only); break;
+                case 2: launch_flux_gs_curved<EOS, 2>(c, eos, f, s, O, only); break;
+                default: launch_flux_gs_curved<EOS, 3>(c, eos, f, s, O, only); break;
+            }
+            return;
+        }
+    } else if (only) { launch_flux_tagged<EOS>(c, eos, f, s, O, only); return; }
     switch (recon) {
         case 0: launch_flux<EOS, 0, FLAT>(c, eos, f, s, O); break;
         case 1: launch_flux<EOS, 1, FLAT>(c, eos, f, s, O); break;
@@ -2380,15 +2409,19 @@ static void launch_c2p_cells(grmhd_ctx* c, double* st, int snv, const double* ms
         DevStats* part = with_stats ? c->stats_part + npart : nullptr;
         npart += grid;
         const hipStream_t ls = cset == CS_LIST ? sl : s;
-#define C2PL(EOSV, FL, LR) k_c2p_cells<decltype(EOSV), FL, LR><<<grid, bs, 0, ls>>>(G, EOSV, c->O, c->inst_d, c->blk_d, st, snv, ms, mnv, B[0], B[1], B[2], aux, ec, part, cset, nint, fresh, c->ghost_list, c->own_cells, ne, nlist, wpb, md)
+#define C2PL(EOSV, FL, ...) k_c2p_cells<decltype(EOSV), FL, __VA_ARGS__><<<grid, bs, 0, ls>>>(G, EOSV, c->O, c->inst_d, c->blk_d, st, snv, ms, mnv, B[0], B[1], B[2], aux, ec, part, cset, nint, fresh, c->ghost_list, c->own_cells, ne, nlist, wpb, md)
         if (warm) {
             if (flat) C2PL(c->ideal, true, 2); else C2PL(c->ideal, false, 2);
         } else if (c->mlp) {
             if (c->P.eos_kind == GRMHD_EOS_IDEAL_GAS) { if (flat) C2PL(c->ideal, true, 1); else C2PL(c->ideal, false, 1); }
             else { if (flat) C2PL(c->hybrid, true, 1); else C2PL(c->hybrid, false, 1); }
         } else {
-            if (c->P.eos_kind == GRMHD_EOS_IDEAL_GAS) { if (flat) C2PL(c->ideal, true, 0); else C2PL(c->ideal, false, 0); }
-            else { if (flat) C2PL(c->hybrid, true, 0); else C2PL(c->hybrid, false, 0); }
+            const bool x = !flat && c->P.emf == GRMHD_EMF_GS;
+            if (c->P.eos_kind == GRMHD_EOS_IDEAL_GAS) {
+                if (flat) C2PL(c->ideal, true, 0); else if (x) C2PL(c->ideal, false, 0, true); else C2PL(c->ideal, false, 0);
+            } else {
+                if (flat) C2PL(c->hybrid, true, 0); else if (x) C2PL(c->hybrid, false, 0, true); else C2PL(c->hybrid, false, 0);
+            }
         }
 #undef C2PL
     };

@@ -93,6 +93,15 @@ GHD void nr_sqrt(double x, double& g, double& ig) {
     ig = 1.0 / g;
 #endif
 }
+// The same with a choice: X, the IEEE operation (see c2p).
+template <bool X>
+GHD double rcp(double b) { if constexpr (X) return 1.0 / b; else return nr_rcp(b); }
+template <bool X>
+GHD double quot(double a, double b, double ib) { if constexpr (X) return a / b; else return quot(a, b, ib); }
+template <bool X>
+GHD void root(double x, double& g, double& ig) {
+    if constexpr (X) { g = sqrt(x); ig = 1.0 / g; } else nr_sqrt(x, g, ig);
+}
 // ---- 3-metric -------------------------------------------------------------
 struct Met {
     double g[6], gi[6], beta[3], alp, sqrtg;
@@ -192,6 +201,21 @@ struct EosIdeal {
         const double p = gm1 * eps * rho;
         a2 = gamma * p;
         return p;
+    }
+    // the face states' EOS with sound speed, for GS EMFs on a curved metric
+    GHD double press_from_temp(double& eps, double& cs2, double& temp, double rho, unsigned& e) const {
+        limit_temp(temp, e);
+        eps = temp / gm1;
+        double p = gm1 * eps * rho;
+        double h = 1.0 + gamma * eps;
+        cs2 = ggm1 * eps / h;
+        return p;
+    }
+    GHD double eps_from_press(double& h, double& cs2, double& temp, double& ent, double& press, double rho,
+                              unsigned&) const {
+        double eps = press / (gm1 * rho);
+        h = 1.0 + gamma * eps; cs2 = ggm1 * eps / h; ent = ent_of(eps, rho); temp = eps * gm1;
+        return eps;
     }
     GHD double face_from_press(double& eps, double& a2, double press, double rho) const {
         eps = press / (gm1 * rho);
@@ -310,6 +334,27 @@ struct EosHybrid {
         a2 = a2_of(rho, eth);
         return pc + eth * rho * gth_m1;
     }
+    // the face states' EOS with sound speed, for GS EMFs on a curved metric
+    GHD double press_from_temp(double& eps, double& cs2, double& temp, double rho, unsigned& e) const {
+        chk_rho(rho, e); chk_temp(temp, e);
+        double ec; double pc = pcold(ec, rho);
+        double eth = eth_of_t(temp);
+        double p = pc + eth * rho * gth_m1;
+        eps = ec + eth;
+        double h = 1. + eps + p / rho;
+        cs2 = cs2_of(rho, eth, h);
+        return p;
+    }
+    GHD double eps_from_press(double& h, double& cs2, double& temp, double& ent, double& press, double rho,
+                              unsigned& e) const {
+        chk_rho(rho, e);
+        double ec; double pc = pcold(ec, rho);
+        press = fmax(press, pc);
+        double eth = fmax(0, (press - pc) / (rho * gth_m1));
+        double eps = eth + ec;
+        h = 1. + eps + press / rho; cs2 = cs2_of(rho, eth, h); ent = ent_of(eth, rho); temp = t_of(eth);
+        return eps;
+    }
     GHD double face_from_press(double& eps, double& a2, double press, double rho) const {
         unsigned e = 0;
         chk_rho(rho, e);
@@ -373,27 +418,27 @@ GHD double norm_low(const Met& m, double x, double y, double z) {
     if constexpr (FL) return x * x + y * y + z * z;
     else return m.sqcov(x, y, z);
 }
-template <bool FL = false>
+template <bool FL = false, bool X = true>
 GHD double lorentz(const double g[6], const double z[3]) {
     double zl[3], W, iW; lower3<FL>(g, z[0], z[1], z[2], zl);
-    nr_sqrt(z[0] * zl[0] + z[1] * zl[1] + z[2] * zl[2] + 1, W, iW);
+    root<X>(z[0] * zl[0] + z[1] * zl[1] + z[2] * zl[2] + 1, W, iW);
     return W;
 }
-template <bool FL = false>
+template <bool FL = false, bool X = true>
 GHD void smallb(const Met& m, const double B[3], const double z[3], double W, double b[4], double& b2) {
     double zl[3]; lower3<FL>(m.g, z[0], z[1], z[2], zl);
     double Bz = B[0] * zl[0] + B[1] * zl[1] + B[2] * zl[2];
-    const double iW = nr_rcp(W);
+    const double iW = rcp<X>(W);
     if constexpr (FL) {
         b[0] = Bz;
         for (int i = 0; i < 3; ++i) b[1 + i] = iW * (B[i] + Bz * z[i]);
     } else {
-        const double ia = nr_rcp(m.alp);
-        b[0] = quot(Bz, m.alp, ia);
-        for (int i = 0; i < 3; ++i) b[1 + i] = iW * (B[i] + Bz * (z[i] - quot(W * m.beta[i], m.alp, ia)));
+        const double ia = rcp<X>(m.alp);
+        b[0] = quot<X>(Bz, m.alp, ia);
+        for (int i = 0; i < 3; ++i) b[1 + i] = iW * (B[i] + Bz * (z[i] - quot<X>(W * m.beta[i], m.alp, ia)));
     }
     double Bl[3]; lower3<FL>(m.g, B[0], B[1], B[2], Bl);
-    b2 = quot(B[0] * Bl[0] + B[1] * Bl[1] + B[2] * Bl[2] + Bz * Bz, W * W, iW * iW);
+    b2 = quot<X>(B[0] * Bl[0] + B[1] * Bl[1] + B[2] * Bl[2] + Bz * Bz, W * W, iW * iW);
 }
 GHD void vtilde(const Met& m, const double z[3], double W, double vt[3]) {
     double iW = 1. / W;
@@ -440,7 +485,7 @@ GHD void conserved(const Met& m, double rho, double press, double eps, const dou
 // ---- roots --------------------------------------------------------------------
 // Brent's zero-in (Brent 1973, ch. 4): same step sequence as rootfinding.hh:73-231.
 constexpr int BRENT_MAX_ITER = 1000;
-template <typename F>
+template <bool X, typename F>
 __host__ __device__ inline double brent_fab(F& f, double a, double b, double fa, double fb, double t) {
     double sa = a, sb = b;
     double c = sa, fc = fa, e = sb - sa, d = e;
@@ -455,18 +500,18 @@ __host__ __device__ inline double brent_fab(F& f, double a, double b, double fa,
         if (fabs(e) < tol || fabs(fa) <= fabs(fb)) { e = mm; d = e; }
         else {
             // (fa, fc: non-zero here; the quotients only shape the step)
-            const double iac = nr_rcp(fa * fc);
-            double s = fb * (fc * iac), p, q;
+            const double iac = X ? 0.0 : nr_rcp(fa * fc);
+            double s = X ? fb / fa : fb * (fc * iac), p, q;
             if (sa == c) { p = 2.0 * mm * s; q = 1.0 - s; }
             else {
                 const double ic = fa * iac;
-                double qq = fa * ic, r = fb * ic;
+                double qq = X ? fa / fc : fa * ic, r = X ? fb / fc : fb * ic;
                 p = s * (2.0 * mm * qq * (qq - r) - (sb - sa) * (r - 1.0));
                 q = (qq - 1.0) * (r - 1.0) * (s - 1.0);
             }
             if (0.0 < p) q = -q; else p = -p;
             s = e; e = d;
-            if (2.0 * p < 3.0 * mm * q - fabs(tol * q) && p < fabs(0.5 * s * q)) d = p * nr_rcp(q);
+            if (2.0 * p < 3.0 * mm * q - fabs(tol * q) && p < fabs(0.5 * s * q)) d = X ? p / q : p * nr_rcp(q);
             else { e = mm; d = e; }
         }
         sa = sb; fa = fb;
@@ -476,12 +521,12 @@ __host__ __device__ inline double brent_fab(F& f, double a, double b, double fa,
     }
     return sb;
 }
-template <typename F>
+template <bool X, typename F>
 __host__ __device__ inline double brent(F& f, double a, double b, double t) {
     double fa = f(a), fb = f(b);
-    return brent_fab(f, a, b, fa, fb, t);
+    return brent_fab<X>(f, a, b, fa, fb, t);
 }
-template <typename F>
+template <bool X, typename F>
 __host__ __device__ inline double newton_br(double sa, double sb, F& f, int maxiter, double tol, int& err) {
     const double macheps = 2.220446049250313e-16;
     double a = sa, b = sb, fa, fb, dd;
@@ -495,7 +540,7 @@ __host__ __device__ inline double newton_br(double sa, double sb, F& f, int maxi
     do {
         xold = x; f(x, fx, dfx);
         if (fx * fb > 0) { fb = fx; b = x; } else if (fx * fa > 0) { fa = fx; a = x; }
-        x -= fx * nr_rcp(dfx);
+        x -= X ? fx / dfx : fx * nr_rcp(dfx);
         t = 2. * macheps * fabs(x) + tol;
         if (fabs(x - xold) < t || fx == 0) { err = 0; return x; }
         if (x > b || x < a) x = 0.5 * (b + a);
@@ -506,22 +551,23 @@ __host__ __device__ inline double newton_br(double sa, double sb, F& f, int maxi
 }
 
 // ---- Kastaun master functions ----------------------------------------------------
+template <bool X>
 struct FBr {
     double rsqr, bsqr, rbsqr, h0sqr; int* cnt;
-    GHD double xm(double mu) const { return nr_rcp(1. + mu * bsqr); }
+    GHD double xm(double mu) const { return rcp<X>(1. + mu * bsqr); }
     GHD double rb(double mu, double x) const { return x * (rsqr * x + mu * (x + 1.0) * rbsqr); }
     GHD void operator()(double mu, double& f, double& df) {
         (*cnt)++;
         double x = xm(mu), x2 = x * x;
         double hw, ihw;
-        nr_sqrt(h0sqr + rb(mu, x), hw, ihw);
+        root<X>(h0sqr + rb(mu, x), hw, ihw);
         double bb = x * (x2 * rsqr + mu * (1 + x + x2) * rbsqr);
-        f = mu * hw - 1.; df = (h0sqr + bb) * ihw;
+        f = mu * hw - 1.; df = X ? (h0sqr + bb) / hw : (h0sqr + bb) * ihw;
     }
     GHD double operator()(double mu) {
         (*cnt)++;
         double hw, ihw;
-        nr_sqrt(h0sqr + rb(mu, xm(mu)), hw, ihw);
+        root<X>(h0sqr + rb(mu, xm(mu)), hw, ihw);
         return mu * hw - 1.;
     }
     GHD void bracket(double& lo, double& hi) const {
@@ -533,17 +579,17 @@ struct FBr {
     }
 };
 
-template <typename EOS>
+template <bool X, typename EOS>
 struct FMu {
     const EOS& eos;
     double d, qtot, rsqr, bsqr, rbsqr, brosqr, vsqrmax, wmax, iwmax; int* cnt;
     GHD FMu(const EOS& e, double d_, double q_, double r2, double rb2, double b2, double h0, int* c)
         : eos(e), d(d_), qtot(q_), rsqr(r2), bsqr(b2), rbsqr(rb2), brosqr(r2 * b2 - rb2), cnt(c) {
         double zs = rsqr / (h0 * h0), ws = 1 + zs;
-        nr_sqrt(ws, wmax, iwmax);
+        root<X>(ws, wmax, iwmax);
         vsqrmax = zs / ws;
     }
-    GHD double xm(double mu) const { return nr_rcp(1. + mu * bsqr); }
+    GHD double xm(double mu) const { return rcp<X>(1. + mu * bsqr); }
     GHD double rf(double mu, double x) const { return x * (rsqr * x + mu * (x + 1.0) * rbsqr); }
     GHD double qf(double mu, double x) const { double mx = mu * x; return qtot - 0.5 * (bsqr + mx * mx * brosqr); }
     GHD double epsraw(double mu, double q, double r, double w) const { return w * (q - mu * r * (1.0 - mu * w / (1 + w))); }
@@ -556,7 +602,7 @@ struct FMu {
         (*cnt)++;
         double x = xm(mu), r = rf(mu, x), q = qf(mu, x);
         double vs = r * mu * mu, w;
-        if constexpr (EOS::is_ideal) {
+        if constexpr (EOS::is_ideal && !X) {
             double iw;
             nr_sqrt(fmax(1 - vs, 1e-280), iw, w);
             if (vs > vsqrmax) { w = wmax; iw = iwmax; }
@@ -632,26 +678,31 @@ struct FMu {
     }
 };
 
-template <typename EOS>
+template <bool X, typename EOS>
 struct FMuEnt {
     const EOS& eos;
     double d, s, rsqr, bsqr, rbsqr, vsqrmax, wmax, iwmax; int* cnt;
     GHD FMuEnt(const EOS& e, double d_, double r2, double rb2, double b2, double s_, double h0, int* c)
         : eos(e), d(d_), s(s_), rsqr(r2), bsqr(b2), rbsqr(rb2), cnt(c) {
         double zs = rsqr / (h0 * h0), ws = 1 + zs;
-        nr_sqrt(ws, wmax, iwmax);
+        root<X>(ws, wmax, iwmax);
         vsqrmax = zs / ws;
     }
-    GHD double xm(double mu) const { return nr_rcp(1. + mu * bsqr); }
+    GHD double xm(double mu) const { return rcp<X>(1. + mu * bsqr); }
     GHD double rf(double mu, double x) const { return x * (rsqr * x + mu * (x + 1.0) * rbsqr); }
     GHD double operator()(double mu) {
         (*cnt)++;
         double x = xm(mu), r = rf(mu, x);
-        double vs = r * mu * mu, w, iw;
-        nr_sqrt(fmax(1 - vs, 1e-280), iw, w);
-        if (vs > vsqrmax) { w = wmax; iw = iwmax; }
-        double rho = fmin(eos.rhomax(), fmax(eos.rhomin(), d * iw));
-        if constexpr (EOS::is_ideal) {
+        double vs = r * mu * mu, w, iw = 0.0;
+        if constexpr (X) {
+            w = 1 / sqrt(1 - vs);
+            if (vs > vsqrmax) w = wmax;
+        } else {
+            nr_sqrt(fmax(1 - vs, 1e-280), iw, w);
+            if (vs > vsqrmax) { w = wmax; iw = iwmax; }
+        }
+        double rho = fmin(eos.rhomax(), fmax(eos.rhomin(), X ? d / w : d * iw));
+        if constexpr (EOS::is_ideal && !X) {
             const double h = 1 + eos.gamma * eos.eps_from_ent(s, rho), den = h * iw + r * mu;
             return mu - quot(1.0, den, nr_rcp(den));
         }
@@ -709,16 +760,16 @@ struct C2PIn {
     double D, q, s, r2, Bt2, rBt, rBt2, h0;
     double r[3], Bt[3], B[3];
 };
-template <bool FL, typename EOS>
+template <bool FL, bool X, typename EOS>
 GHD void c2p_setup(const EOS& eos, const Met& m, double cons[NCONS], C2PIn& c) {
     c.h0 = eos.hmin();
     cons[DENSL] = fmax(0., cons[DENSL]);
     c.D = cons[DENSL];
-    const double iD = nr_rcp(c.D), sD = sqrt(c.D), isD = nr_rcp(sD);
-    c.q = quot(cons[TAUL], c.D, iD);
-    c.s = quot(cons[ENTSL], c.D, iD);
-    const double rl0 = quot(cons[STXL], c.D, iD), rl1 = quot(cons[STYL], c.D, iD), rl2 = quot(cons[STZL], c.D, iD);
-    for (int i = 0; i < 3; ++i) { c.Bt[i] = quot(cons[BSXL + i], sD, isD); c.B[i] = cons[BSXL + i]; }
+    const double iD = rcp<X>(c.D), sD = sqrt(c.D), isD = rcp<X>(sD);
+    c.q = quot<X>(cons[TAUL], c.D, iD);
+    c.s = quot<X>(cons[ENTSL], c.D, iD);
+    const double rl0 = quot<X>(cons[STXL], c.D, iD), rl1 = quot<X>(cons[STYL], c.D, iD), rl2 = quot<X>(cons[STZL], c.D, iD);
+    for (int i = 0; i < 3; ++i) { c.Bt[i] = quot<X>(cons[BSXL + i], sD, isD); c.B[i] = cons[BSXL + i]; }
     c.r2 = norm_low<FL>(m, rl0, rl1, rl2);
     c.Bt2 = norm_up<FL>(m, c.Bt[0], c.Bt[1], c.Bt[2]);
     c.rBt = rl0 * c.Bt[0] + rl1 * c.Bt[1] + rl2 * c.Bt[2];
@@ -812,11 +863,11 @@ GHD bool newton_guess(F& f, double x, double umax, int maxit, double acc, double
     return false;
 }
 
-template <typename EOS>
+template <bool X, typename EOS>
 GHD double kastaun(const EOS& eos, const C2PIn& c, double pr[NPRIM], unsigned& sig, C2PCount& cnt,
                    const C2PGuess& gs, C2PRoots& rt) {
     double h0 = c.h0;
-    FMu<EOS> f(eos, c.D, c.q, c.r2, c.rBt2, c.Bt2, h0, &cnt.root);
+    FMu<X, EOS> f(eos, c.D, c.q, c.r2, c.rBt2, c.Bt2, h0, &cnt.root);
     double mu = -1.0;
     if constexpr (EOS::is_ideal) {
         double r;
@@ -828,7 +879,7 @@ GHD double kastaun(const EOS& eos, const C2PIn& c, double pr[NPRIM], unsigned& s
     if (mu < 0.0 && guess_ok(gs.e_lo, gs.e_hi)) {
         double a, b, fa, fb;
         if (guess_bracket(f, gs.e_lo / h0, gs.e_hi / h0, 1.0 / h0, gs.nexp, a, b, fa, fb)) {
-            mu = brent_fab(f, a, b, fa, fb, 1e-15);
+            mu = brent_fab<X>(f, a, b, fa, fb, 1e-15);
             cnt.guess_used |= 1;
         }
     }
@@ -836,13 +887,13 @@ GHD double kastaun(const EOS& eos, const C2PIn& c, double pr[NPRIM], unsigned& s
     if (mu < 0.0) {
         double mu0 = 1 / h0;
         if (c.r2 >= h0 * h0) {
-            FBr g{c.r2, c.Bt2, c.rBt2, h0 * h0, &cnt.bracket};
+            FBr<X> g{c.r2, c.Bt2, c.rBt2, h0 * h0, &cnt.bracket};
             double lo, hi; g.bracket(lo, hi);
             int rerr;
-            mu0 = newton_br(lo, hi, g, 30, 1e-10, rerr);
+            mu0 = newton_br<X>(lo, hi, g, 30, 1e-10, rerr);
             if (rerr == 0) mu0 *= 1 + 1e-10; else mu0 = 1.0 / h0;
         }
-        mu = brent(f, 0., mu0, 1e-15);
+        mu = brent<X>(f, 0., mu0, 1e-15);
         rt.m_e = mu0 * h0;
     }
     rt.x_e = mu * h0;
@@ -854,11 +905,11 @@ GHD double kastaun(const EOS& eos, const C2PIn& c, double pr[NPRIM], unsigned& s
     return fabs(res);
 }
 
-template <typename EOS>
+template <bool X, typename EOS>
 GHD double kastaun_ent(const EOS& eos, const C2PIn& c, double pr[NPRIM], unsigned& sig, C2PCount& cnt,
                        const C2PGuess& gs, C2PRoots& rt) {
     double h0 = c.h0;
-    FMuEnt<EOS> f(eos, c.D, c.r2, c.rBt2, c.Bt2, c.s, h0, &cnt.root);
+    FMuEnt<X, EOS> f(eos, c.D, c.r2, c.rBt2, c.Bt2, c.s, h0, &cnt.root);
     double mu = -1.0;
     if constexpr (EOS::is_ideal) {
         double r;
@@ -870,7 +921,7 @@ GHD double kastaun_ent(const EOS& eos, const C2PIn& c, double pr[NPRIM], unsigne
     if (mu < 0.0 && guess_ok(gs.s_lo, gs.s_hi)) {
         double a, b, fa, fb;
         if (guess_bracket(f, gs.s_lo / h0, gs.s_hi / h0, 1.0 / h0, gs.nexp, a, b, fa, fb)) {
-            mu = brent_fab(f, a, b, fa, fb, 1e-15);
+            mu = brent_fab<X>(f, a, b, fa, fb, 1e-15);
             cnt.guess_used |= 2;
         }
     }
@@ -878,12 +929,12 @@ GHD double kastaun_ent(const EOS& eos, const C2PIn& c, double pr[NPRIM], unsigne
     if (mu < 0.0) {
         double mu0 = 1 / h0;
         if (c.r2 >= h0 * h0) {
-            FBr g{c.r2, c.Bt2, c.rBt2, h0 * h0, &cnt.bracket};
+            FBr<X> g{c.r2, c.Bt2, c.rBt2, h0 * h0, &cnt.bracket};
             int rerr;
-            mu0 = newton_br(0., 1. / h0, g, 30, 1e-10, rerr);
-            if (rerr == 0) mu0 *= 1 + 1e-10; else mu0 = brent(g, 0., 1. / h0, 1e-10) * (1 + 1e-10);
+            mu0 = newton_br<X>(0., 1. / h0, g, 30, 1e-10, rerr);
+            if (rerr == 0) mu0 *= 1 + 1e-10; else mu0 = brent<X>(g, 0., 1. / h0, 1e-10) * (1 + 1e-10);
         }
-        mu = brent(f, 0., mu0, 1e-15);
+        mu = brent<X>(f, 0., mu0, 1e-15);
         rt.m_s = mu0 * h0;
     }
     rt.x_s = mu * h0;
@@ -953,20 +1004,20 @@ GHD void p2c_wb(const double pr[NPRIM], double cons[NCONS], const Met& m, double
     cons[TAUL] = m.sqrtg * tau; cons[ENTSL] = m.sqrtg * Ss;
     cons[YESL] = cons[DENSL] * pr[YEL];
 }
-template <bool FL = false>
+template <bool FL = false, bool X = true>
 GHD void p2c(const double pr[NPRIM], double cons[NCONS], const Met& m) {
-    double W = lorentz<FL>(m.g, &pr[ZXL]);
-    double b[4], b2; smallb<FL>(m, &pr[BXL], &pr[ZXL], W, b, b2);
+    double W = lorentz<FL, X>(m.g, &pr[ZXL]);
+    double b[4], b2; smallb<FL, X>(m, &pr[BXL], &pr[ZXL], W, b, b2);
     p2c_wb<FL>(pr, cons, m, W, b, b2);
 }
 
-template <bool FL, typename EOS>
+template <bool FL, bool X, typename EOS>
 GHD void atmo_reset(double cons[NCONS], double pr[NPRIM], const Met& m, const Atmo& at, const EOS& eos, uint64_t& err) {
     pr[RHOL] = at.rho_fl; pr[YEL] = at.ye_fl; pr[TEMPL] = at.temp_fl;
     pr[ZXL] = pr[ZYL] = pr[ZZL] = 0.;
     unsigned ee = 0; double cs2;
     pr[PRESSL] = eos.press_from_temp_ent(pr[EPSL], cs2, pr[ENTL], pr[TEMPL], pr[RHOL], ee);
-    p2c<FL>(pr, cons, m);
+    p2c<FL, X>(pr, cons, m);
     set_all_resets(err);
     err |= BIT(E_ATMO_RESET);
 }
@@ -974,7 +1025,14 @@ GHD void atmo_reset(double cons[NCONS], double pr[NPRIM], const Met& m, const At
 struct C2POut { bool floored, fatal; };
 
 // conservs_to_prims (c2p.cpp:188-414).  cons densitised in, re-densitised out.
-template <bool FL, typename EOS>
+// X: every quotient and root an IEEE operation, the master functions in the
+// general form.  For GS EMFs on a curved metric: they choose a side by the
+// sign of the mass flux, which in a stationary flow (a torus: no poloidal
+// velocity) is rounding at many faces, and primitives that differ in the last
+// bit move the field by 1e-6 of its largest value in one step.  The other
+// form is as accurate (2.8e-11 against 64-bit bisection either way) and takes
+// 0.7 of the time.
+template <bool FL, bool X, typename EOS>
 GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eos, const Atmo& at,
                const ExcPar& ex, const C2PPar& cp, double radius, uint64_t& err, bool dry_run, C2PCount& cnt,
                const C2PGuess& gs, C2PRoots& rt) {
@@ -983,24 +1041,24 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
     unsigned ret = 0;
     err = BIT(E_RESET_ENTROPY);
     if constexpr (!FL) {
-        const double isg = nr_rcp(m.sqrtg);
-        for (int i = 0; i < NCONS; ++i) cons[i] = quot(cons[i], m.sqrtg, isg);
+        const double isg = rcp<X>(m.sqrtg);
+        for (int i = 0; i < NCONS; ++i) cons[i] = quot<X>(cons[i], m.sqrtg, isg);
     }
     pr[BXL] = cons[BSXL]; pr[BYL] = cons[BSYL]; pr[BZL] = cons[BSZL];
-    if (cons[DENSL] < 0) { atmo_reset<FL>(cons, pr, m, at, eos, err); out.floored = true; return out; }
-    const double iD = nr_rcp(cons[DENSL]);
-    pr[YEL] = quot(cons[YESL], cons[DENSL], iD);
+    if (cons[DENSL] < 0) { atmo_reset<FL, X>(cons, pr, m, at, eos, err); out.floored = true; return out; }
+    const double iD = rcp<X>(cons[DENSL]);
+    pr[YEL] = quot<X>(cons[YESL], cons[DENSL], iD);
     if (pr[YEL] > eos.yemax()) { pr[YEL] = eos.yemax(); err |= BIT(E_RESET_YE); }
     if (pr[YEL] < eos.yemin()) { pr[YEL] = eos.yemin(); err |= BIT(E_RESET_YE); }
     bool lenient = m.alp < cp.alp_bh_thresh;
     {   // limit_conservatives (c2p.cpp:117-157)
         double emin, emax; eos.eps_range(emin, emax, cons[DENSL]);
         double B2 = norm_up<FL>(m, cons[BSXL], cons[BSYL], cons[BSZL]);
-        if (quot(cons[TAUL], cons[DENSL], iD) - quot(0.5 * B2, cons[DENSL], iD) < fmin(0.0, emin)) {
+        if (quot<X>(cons[TAUL], cons[DENSL], iD) - quot<X>(0.5 * B2, cons[DENSL], iD) < fmin(0.0, emin)) {
             cons[TAUL] = emin * cons[DENSL] + 0.5 * B2;
             err |= BIT(E_RESET_TAU); floored = true;
         }
-        double st2max = sq(quot(cons[TAUL], cons[DENSL], iD) + 1);
+        double st2max = sq(quot<X>(cons[TAUL], cons[DENSL], iD) + 1);
         double st2 = norm_low<FL>(m, cons[STXL], cons[STYL], cons[STZL]) / sq(cons[DENSL]);
         if (st2 > st2max) {
             double f = sqrt(st2max / st2);
@@ -1012,13 +1070,13 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
     if (cons[DENSL] >= at.rho_fl * (1 + at.atmo_tol)) {
         // both inversions start from the same invariants of the (limited)
         // conserved state, so they are formed once
-        C2PIn ci; c2p_setup<FL>(eos, m, cons, ci);
-        double res = kastaun(eos, ci, pr, ret, cnt, gs, rt);
+        C2PIn ci; c2p_setup<FL, X>(eos, m, cons, ci);
+        double res = kastaun<X>(eos, ci, pr, ret, cnt, gs, rt);
         failed = (fabs(res) > cp.tol) || (ret & BIT(SIG_RHO_TOO_HIGH)) || (ret & BIT(SIG_EPS_TOO_HIGH)) || !isfinite(res);
         double beta;
         {
-            double W = lorentz<FL>(m.g, &pr[ZXL]);
-            double b[4], b2; smallb<FL>(m, &pr[BXL], &pr[ZXL], W, b, b2);
+            double W = lorentz<FL, X>(m.g, &pr[ZXL]);
+            double b[4], b2; smallb<FL, X>(m, &pr[BXL], &pr[ZXL], W, b, b2);
             beta = 2.0 * pr[PRESSL] / fmax(b2, 1e-50);
         }
         bool distrust = failed || (ret & BIT(SIG_EPS_TOO_LOW)) || (beta <= cp.beta_fallback);
@@ -1031,7 +1089,7 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
                 gse.s_lo = gs.s_lo * rt.x_e; gse.s_hi = fmin(gs.s_hi * rt.x_e, 1.0);
                 gse.s_c = gs.s_c * rt.x_e;
             }
-            double rb = kastaun_ent(eos, ci, pr, bret, cnt, gse, rt);
+            double rb = kastaun_ent<X>(eos, ci, pr, bret, cnt, gse, rt);
             bool ok = (fabs(rb) <= cp.tol) && isfinite(rb) && (pr[EPSL] < eos.eps_max);
             if (ok) { ret = bret; failed = false; err |= BIT(E_ENT_BACKUP_USED); }
             else if (!failed) { for (int i = 0; i < NPRIM; ++i) pr[i] = save[i]; }
@@ -1044,7 +1102,7 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
     }
     bool excise = ex.by_radius ? (radius <= ex.r_ex) : (m.alp <= ex.alp_ex);
     if ((pr[RHOL] < (1. + at.atmo_tol) * at.rho_fl) || failed || excise) {
-        atmo_reset<FL>(cons, pr, m, at, eos, err);
+        atmo_reset<FL, X>(cons, pr, m, at, eos, err);
         floored = true;
     } else if (pr[TEMPL] < at.temp_fl) {
         pr[TEMPL] = at.temp_fl;
@@ -1062,8 +1120,8 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
             pr[ZXL] *= zn; pr[ZYL] *= zn; pr[ZZL] *= zn;
             sg |= BIT(SIG_VEL_TOO_HIGH);
         }
-        const double W = lorentz<FL>(m.g, &pr[ZXL]);
-        double b[4], b2; smallb<FL>(m, &pr[BXL], &pr[ZXL], W, b, b2);
+        const double W = lorentz<FL, X>(m.g, &pr[ZXL]);
+        double b[4], b2; smallb<FL, X>(m, &pr[BXL], &pr[ZXL], W, b, b2);
         double sigma = b2 / pr[RHOL];
         if (sigma >= cp.max_sigma) {
             pr[RHOL] *= 1.001 * sigma / cp.max_sigma;
@@ -1078,7 +1136,7 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
         out.floored = floored;
         return out;
     }
-    p2c<FL>(pr, cons, m);
+    p2c<FL, X>(pr, cons, m);
     out.floored = floored;
     return out;
 }
@@ -1164,6 +1222,54 @@ GHD double mc2(double sL, double sR) {
 }
 GHD double minmod(double sL, double sR) {
     return 0.5 * (copysign(1.0, sL) + copysign(1.0, sR)) * fmin(fabs(sL), fabs(sR));
+}
+// The candidates' form of WENO-Z, kept for GS EMFs on a curved metric (see
+// c2p): the same values up to rounding.
+// Per side, the three ratios
+// t5/(b_k+eps) come from one reciprocal of d0 d1 d2 (d_k >= 1e-42, so the
+// product cannot underflow), and the two sides of a face share their
+// reciprocals: 1/(P_R P_L) gives 1/P_R and 1/P_L, 1/(S_R S_L) the two
+// normalisations (guarded against overflow of the products, which falls back
+// to separate divisions).  This differs from the reference's three divisions
+// per weight by a few ulp.
+struct WenoSide { double q0, q1, q2; double P; };
+GHD void weno_betas(double b0, double b1, double b2, double& d0, double& d1, double& d2, double& t5) {
+    const double eps = 1.0e-42;
+    d0 = b0 + eps; d1 = b1 + eps; d2 = b2 + eps;
+    t5 = fabs(b0 - b2);
+}
+GHD void wenoz(double um3, double um2, double um1, double u0, double up1, double up2, double& uL, double& uR) {
+    const double c0 = 13.0 / 12.0, c1 = 0.25;
+    // right state (cell i stencils; a0 pairs with i2, a2 with i0 on this side)
+    const double rb0 = c0 * sq(um2 + u0 - 2.0 * um1) + c1 * sq(um2 + 3.0 * u0 - 4.0 * um1);
+    const double rb1 = c0 * sq(um1 + up1 - 2.0 * u0) + c1 * sq(um1 - up1);
+    const double rb2 = c0 * sq(up2 + u0 - 2.0 * up1) + c1 * sq(up2 + 3.0 * u0 - 4.0 * up1);
+    // left state (cell i-1 stencils)
+    const double lb0 = c0 * sq(um3 + um1 - 2.0 * um2) + c1 * sq(um3 + 3.0 * um1 - 4.0 * um2);
+    const double lb1 = c0 * sq(um2 + u0 - 2.0 * um1) + c1 * sq(um2 - u0);
+    const double lb2 = c0 * sq(up1 + um1 - 2.0 * u0) + c1 * sq(up1 + 3.0 * um1 - 4.0 * u0);
+    double rd0, rd1, rd2, rt, ld0, ld1, ld2, lt;
+    weno_betas(rb2, rb1, rb0, rd0, rd1, rd2, rt);
+    weno_betas(lb0, lb1, lb2, ld0, ld1, ld2, lt);
+    const double rP01 = rd0 * rd1, rP = rP01 * rd2, lP01 = ld0 * ld1, lP = lP01 * ld2;
+    double rr, lr;
+    const double PP = rP * lP;
+    // PP >= 1e-252 (every d >= 1e-42): a normal, finite reciprocal
+    if (PP < 1e300) { const double inv = nr_rcp(PP); rr = rt * lP * inv; lr = lt * rP * inv; }
+    else { rr = rt / rP; lr = lt / lP; }
+    const double rq0 = rd1 * rd2 * rr, rq1 = rd0 * rd2 * rr, rq2 = rP01 * rr;
+    const double lq0 = ld1 * ld2 * lr, lq1 = ld0 * ld2 * lr, lq2 = lP01 * lr;
+    const double ra0 = 0.1 * (1.0 + rq0 * rq0), ra1 = 0.6 * (1.0 + rq1 * rq1), ra2 = 0.3 * (1.0 + rq2 * rq2);
+    const double la0 = 0.1 * (1.0 + lq0 * lq0), la1 = 0.6 * (1.0 + lq1 * lq1), la2 = 0.3 * (1.0 + lq2 * lq2);
+    const double rn = (2.0 * up2 - 7.0 * up1 + 11.0 * u0) * ra0 + (-1.0 * up1 + 5.0 * u0 + 2.0 * um1) * ra1 +
+                      (2.0 * u0 + 5.0 * um1 - um2) * ra2;
+    const double ln = (2.0 * um3 - 7.0 * um2 + 11.0 * um1) * la0 + (-1.0 * um2 + 5.0 * um1 + 2.0 * u0) * la1 +
+                      (2.0 * um1 + 5.0 * u0 - up1) * la2;
+    const double rS = 6.0 * (ra0 + ra1 + ra2), lS = 6.0 * (la0 + la1 + la2);
+    const double SS = rS * lS;
+    // SS >= 36 (every a >= its linear weight)
+    if (SS < 1e300) { const double inv = nr_rcp(SS); uR = rn * lS * inv; uL = ln * rS * inv; }
+    else { uR = rn / rS; uL = ln / lS; }
 }
 // MC2, minmod, donor cell: both states of the face between um1 and u0
 template <int REC>

@@ -78,3 +78,14 @@ def test_gpu_flux_faces_overflowing_products(dev, where):
     assert linf_rel(gn[:, ga.YESTAR], new_o[:, ga.YESTAR]) < 1e-12
     for v in (ga.DENS, ga.TAU, ga.SX, ga.SY, ga.SZ, ga.ENTROPYSTAR):
         assert linf_rel(gn[:, v], new_o[:, v]) < 1e-12, v
+
+
+@pytest.mark.parametrize("n,recon,riemann,thermo", [(5, 0, 0, 1), (6, 1, 1, 0), (7, 2, 1, 1), (16, 3, 0, 0)])
+def test_gpu_flux_faces_gs_curved(dev, n, recon, riemann, thermo):
+    """GS on a curved metric has a face kernel (and an inversion) of its own:
+    two RK3 steps against the oracle."""
+    wl = W.blast_ks(nb=(2, 2, 2), n=n, emf=ga.EMF_GS)
+    wl.params.recon, wl.params.riemann, wl.params.thermo_recon = recon, riemann, thermo
+    ref, got, _ = run_rk3_pair(wl, dev, steps=2)
+    check_close(wl, ref, got, 1e-12)
+    assert np.array_equal(got[2][:, ga.C2P_ERR], ref[2][:, ga.C2P_ERR])
