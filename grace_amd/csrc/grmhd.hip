@@ -1130,11 +1130,14 @@ static __device__ __align__(256) DevStats scratch[GRMHD_NOALLOC_MAX_STATES / 256
 // ---------------------------------------------------------------------------
 // c2p over cells (compute_auxiliaries)
 // ---------------------------------------------------------------------------
-// Minimum resident 256-thread blocks per CU for the c2p kernels (caps their
-// registers: 2 -> 256 VGPRs, 3 -> 168, 4 -> 128 per lane).
-#ifndef GRMHD_C2P_MINB
-#define GRMHD_C2P_MINB 3
-#endif
+// Resident 256-thread blocks per CU that the c2p kernels are built for: 3
+// (168 VGPRs) where little spills, 2 (256 VGPRs, no spills) where the metric
+// or the network's fragments stay alive across the root solves.  With 3 / 2:
+// flat cells (128^3 step) 4300 / 4295 us, curved cells 80^3 1548 / 1503 and
+// the torus forest 2074 / 2014, learned batch of 1M 201 / 193; plain batch of
+// 4M 860 / 935.  With 4 every one is slower (spills of 200 bytes and more).
+constexpr int c2p_cells_blocks(bool flat) { return flat ? 3 : 2; }
+constexpr int c2p_batch_blocks(bool learned) { return learned ? 2 : 3; }
 // Cell sets: CS_INTERIOR (the interior cells of every block, wpb workgroups
 // per block, see wg_pos), CS_SHELL (the ghost-shell cells of every block),
 // CS_LIST (explicit {block, cell} pairs), CS_STAGE (the interior cells in the
@@ -1150,7 +1153,7 @@ enum { CS_INTERIOR = 0, CS_SHELL = 1, CS_LIST = 2, CS_STAGE = 3 };
 // evaluations before the plain path.
 // X: see c2p (GS on a curved metric).
 template <typename EOS, bool FLAT, int GUESS = 0, bool X = false>
-__global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_cells(DevGrid G, EOS eos, Opts o, const DevInst* __restrict__ inst,
+__global__ __launch_bounds__(256, c2p_cells_blocks(FLAT)) void k_c2p_cells(DevGrid G, EOS eos, Opts o, const DevInst* __restrict__ inst,
                                                    const DevBlk* __restrict__ blk, double* st, int snv,
                                                    const double* __restrict__ mstate, int mnv,
                                                    const double* __restrict__ Bx, const double* __restrict__ By,
@@ -1306,7 +1309,7 @@ __global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_cells(DevGrid G, EO
 // (ideal gas): the predicted roots start Newton iterations, and where those
 // do not converge the plain path runs (no bracket code in this variant).
 template <typename EOS, bool LEARNED, bool NEWTON = false>
-__global__ __launch_bounds__(256, GRMHD_C2P_MINB) void k_c2p_batch(int64_t n, EOS eos, Opts o, double* cons_soa,
+__global__ __launch_bounds__(256, c2p_batch_blocks(LEARNED)) void k_c2p_batch(int64_t n, EOS eos, Opts o, double* cons_soa,
                                                    const double* __restrict__ met, double* prims,
                                                    uint64_t* errb, uint8_t* floored, int dry_run,
                                                    const double* __restrict__ rad, const double* __restrict__ guess,
