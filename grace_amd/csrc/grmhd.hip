@@ -2179,22 +2179,24 @@ static void launch_flux_tagged(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStre
         else k_flux_tagged<EOS, 2><<<grid, bs, 0, s>>>(G, eos, O, f, only[2]);
     }
 }
-// GS on a curved metric: one launch per direction (only: the FOFC pass).
+// GS on a curved metric (only: the FOFC pass).
 template <typename EOS, int REC>
 static void launch_flux_gs_curved(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O,
                                   uint8_t* const* only) {
     const DevGrid& G = c->G;
     static const char* fam[3] = {"flux_x", "flux_y", "flux_z"};
-    for (int d = 0; d < 3; ++d) {
-        Scope sc(c, only ? "fofc" : fam[d], s);
-        const int64_t n = (int64_t)(G.n[d] + 1 + 2 * O.fofc) * G.N[(d + 1) % 3] * G.N[(d + 2) % 3];
-        const int bs = c->tune.flux[d];
-        f.tiles = (int)nblk_bs(n, bs);
-        const dim3 grid((unsigned)(f.tiles * G.nq));
-        const uint8_t* od = only ? only[d] : nullptr;
-        if (d == 0) k_flux_gs_curved<EOS, REC, 0><<<grid, bs, 0, s>>>(G, eos, O, f, od);
-        else if (d == 1) k_flux_gs_curved<EOS, REC, 1><<<grid, bs, 0, s>>>(G, eos, O, f, od);
-        else k_flux_gs_curved<EOS, REC, 2><<<grid, bs, 0, s>>>(G, eos, O, f, od);
+    FaceTags tags{};
+    if (only) for (int d = 0; d < 3; ++d) tags.d[d] = only[d];
+    f.ndir = c->timing && !only ? 1 : 3;
+    for (f.dir0 = 0; f.dir0 < 3; f.dir0 += f.ndir) {
+        Scope sc(c, only ? "fofc" : fam[f.dir0], s);
+        const int bs = c->tune.flux[f.dir0];
+        f.tiles = 0;
+        for (int d = f.dir0; d < f.dir0 + f.ndir; ++d) {
+            const int64_t n = (int64_t)(G.n[d] + 1 + 2 * O.fofc) * G.N[(d + 1) % 3] * G.N[(d + 2) % 3];
+            f.tiles = std::max(f.tiles, (int)nblk_bs(n, bs));
+        }
+        k_flux_gs_curved<EOS, REC><<<dim3((unsigned)(f.tiles * f.ndir * G.nq)), bs, 0, s>>>(G, eos, O, f, tags);
     }
 }
 // The three directions in one launch; one by one where each is timed.
