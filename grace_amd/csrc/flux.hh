@@ -317,6 +317,10 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
             else recon<REC>(w[1], w[2], w[3], w[4], L[v], R[v]);
             settle(L[v], R[v]);
         }
+        // Some variable's products are out of range: each such variable takes
+        // the other form, by itself.  (All of them at once would give a full
+        // face another rounding than the ring face that the neighbour forms of
+        // it without Y_e and entropy, and the blocks' face B would part.)
         if constexpr (REC == 0)
             if (!ok) {
                 uint32_t again = 0;
@@ -325,7 +329,9 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
                 for (int v = 0; v < FQ_N; ++v) {
                     if (ring && (v == FQ_YE || v == FQ_ENT)) continue;
                     load(v, u[0], again);
-                    wenoz_face_wide(u[0][0], u[0][1], u[0][2], u[0][3], u[0][4], u[0][5], L[v], R[v]);
+                    double lo, hi;
+                    if (!wenoz_face(u[0][0], u[0][1], u[0][2], u[0][3], u[0][4], u[0][5], lo, hi))
+                        wenoz_face_wide(u[0][0], u[0][1], u[0][2], u[0][3], u[0][4], u[0][5], L[v], R[v]);
                     settle(L[v], R[v]);
                 }
             }
