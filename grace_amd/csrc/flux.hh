@@ -381,7 +381,7 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
 // stages against 0.67 and 0.64 here; with the stencil read again at each step
 // 1.1 and 1.0.
 template <typename EOS, int REC, bool FLAT>
-__global__ __launch_bounds__(256, FLAT ? 3 : 2) void k_flux(DevGrid G, EOS eos, Opts o, FluxArgs f) {
+__global__ __launch_bounds__(256, 3) void k_flux(DevGrid G, EOS eos, Opts o, FluxArgs f) {
     const uint32_t nfull = (uint32_t)(f.tiles * f.ndir) * (uint32_t)G.nq;
     const bool ring = blockIdx.x >= nfull;
     const WgPos wp = ring ? wg_pos_in(blockIdx.x - nfull, gridDim.x - nfull, f.tilesr * f.ndir)

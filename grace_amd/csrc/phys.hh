@@ -324,15 +324,25 @@ struct EosHybrid {
         cs2 = cs2_of(rho, eth, h); ent = ent_of(eth, rho);
         return p;
     }
-    GHD double a2_of(double rho, double eth) const { return rho * (dpcold(rho) + gth_m1 * (gth_m1 + 1) * eth); }
-    GHD double face_from_temp(double& eps, double& a2, double temp, double rho) const {
+    // rho h c_s^2 of a face of density rho_f, whose EOS density is rho: the
+    // enthalpy of c_s^2 = (h c_s^2) / h is the EOS's, that of rho h the face's,
+    // and the two cancel unless the EOS has clamped the density (a
+    // reconstruction may leave it at or below zero).
+    GHD double a2_of(double rho_f, double rho, double eth, double eps, double p) const {
+        const double hc2 = dpcold(rho) + gth_m1 * (gth_m1 + 1) * eth;
+        if (rho == rho_f) return rho * hc2;
+        return hc2 / (1. + eps + p / rho) * (rho_f + eps * rho_f + p);
+    }
+    GHD double face_from_temp(double& eps, double& a2, double temp, double rho_f) const {
         unsigned e = 0;
+        double rho = rho_f;
         chk_rho(rho, e); chk_temp(temp, e);
         double ec; double pc = pcold(ec, rho);
         double eth = eth_of_t(temp);
         eps = ec + eth;
-        a2 = a2_of(rho, eth);
-        return pc + eth * rho * gth_m1;
+        const double p = pc + eth * rho * gth_m1;
+        a2 = a2_of(rho_f, rho, eth, eps, p);
+        return p;
     }
     // the face states' EOS with sound speed, for GS EMFs on a curved metric
     GHD double press_from_temp(double& eps, double& cs2, double& temp, double rho, unsigned& e) const {
@@ -355,14 +365,15 @@ struct EosHybrid {
         h = 1. + eps + press / rho; cs2 = cs2_of(rho, eth, h); ent = ent_of(eth, rho); temp = t_of(eth);
         return eps;
     }
-    GHD double face_from_press(double& eps, double& a2, double press, double rho) const {
+    GHD double face_from_press(double& eps, double& a2, double press, double rho_f) const {
         unsigned e = 0;
+        double rho = rho_f;
         chk_rho(rho, e);
         double ec; double pc = pcold(ec, rho);
         press = fmax(press, pc);
         double eth = fmax(0, (press - pc) / (rho * gth_m1));
         eps = eth + ec;
-        a2 = a2_of(rho, eth);
+        a2 = a2_of(rho_f, rho, eth, eps, press);
         return press;
     }
     GHD double press_h_cs2_from_temp(double& h, double& cs2, double& temp, double rho, unsigned& e) const {
