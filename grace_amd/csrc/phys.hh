@@ -601,6 +601,11 @@ struct FMu {
         vsqrmax = zs / ws;
     }
     GHD double xm(double mu) const { return rcp<X>(1. + mu * bsqr); }
+    // the same for the final state, also where B^2 / D is infinite
+    GHD double xm_any(double mu) const {
+        const double b = 1. + mu * bsqr;
+        return __builtin_isinf(b) ? 0. : rcp<X>(b);
+    }
     GHD double rf(double mu, double x) const { return x * (rsqr * x + mu * (x + 1.0) * rbsqr); }
     GHD double qf(double mu, double x) const { double mx = mu * x; return qtot - 0.5 * (bsqr + mx * mx * brosqr); }
     GHD double epsraw(double mu, double q, double r, double w) const { return w * (q - mu * r * (1.0 - mu * w / (1 + w))); }
@@ -668,7 +673,7 @@ struct FMu {
     }
     GHD double prims(double mu, unsigned& sig, double& x, double& w, double& rho, double& press, double& eps,
                      double& temp, double& ent) {
-        x = xm(mu);
+        x = xm_any(mu);
         double r = rf(mu, x), q = qf(mu, x);
         double vs = r * mu * mu;
         if (vs > vsqrmax) { w = wmax; sig |= BIT(SIG_VEL_TOO_HIGH); } else w = 1 / sqrt(1 - vs);
@@ -700,6 +705,11 @@ struct FMuEnt {
         vsqrmax = zs / ws;
     }
     GHD double xm(double mu) const { return rcp<X>(1. + mu * bsqr); }
+    // see FMu
+    GHD double xm_any(double mu) const {
+        const double b = 1. + mu * bsqr;
+        return __builtin_isinf(b) ? 0. : rcp<X>(b);
+    }
     GHD double rf(double mu, double x) const { return x * (rsqr * x + mu * (x + 1.0) * rbsqr); }
     GHD double operator()(double mu) {
         (*cnt)++;
@@ -748,7 +758,7 @@ struct FMuEnt {
     GHD double prims(double mu, unsigned& sig, double& x, double& w, double& rho, double& press, double& eps,
                      double& temp, double& ent) {
         ent = s;
-        x = xm(mu);
+        x = xm_any(mu);
         double r = rf(mu, x);
         double vs = r * mu * mu;
         w = 1 / sqrt(1 - vs);
