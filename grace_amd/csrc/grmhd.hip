@@ -1499,6 +1499,10 @@ struct grmhd_ctx {
     bool ring_any = false;                    // some block has such a face
     int32_t* metric_diff = nullptr;           // device flag of k_metric_diff
     bool metric_same = false;                 // its outcome for mder_src
+    // grmhd_set_static_metric was captured: replays of that graph change the
+    // cached metric without a comparison
+    bool metric_in_graph = false;
+    bool caller_captures = false;             // this RK3 step goes into a graph of the caller's
     // set by the RK3 step around the flux launches of its second and third
     // stages: their ring faces are the neighbours' interior faces and their
     // full faces read the cells beyond a block face from the neighbour's
@@ -2759,6 +2763,12 @@ __global__ __launch_bounds__(256) void k_metric_diff(DevGrid G, const double* __
     if (bad) *diff = 1;
 }
 
+// Whether launches on s go into a graph that is being captured.
+static bool is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 extern "C" grmhd_status grmhd_set_static_metric(grmhd_ctx* c, const double* state, int32_t enable,
                                                 grmhd_stream_t stream) {
     if (!c || (enable && !state)) { set_err("invalid set_static_metric arguments"); return GRMHD_ERR_INVALID; }
@@ -2766,13 +2776,13 @@ extern "C" grmhd_status grmhd_set_static_metric(grmhd_ctx* c, const double* stat
     if (!enable) { c->mder_src = nullptr; return GRMHD_OK; }
     if (c->P.flat_metric) { c->mder_src = nullptr; return GRMHD_OK; }   // flat kernels take no derivatives
     const DevGrid& G = c->G;
+    const hipStream_t s = (hipStream_t)stream;
     const int64_t n = (int64_t)G.n[0] * G.n[1] * G.n[2] * G.nq;
     if (!c->mder) {
         hipError_t e = hipMalloc(&c->mder, sizeof(double) * 30 * n);
         if (e != hipSuccess) { c->mder = nullptr; set_err("static metric cache: %s", hipGetErrorString(e)); return GRMHD_ERR_ALLOC; }
     }
-    k_metric_der<<<nblk(n), 256, 0, (hipStream_t)stream>>>(G, c->inst_d, c->blk_d, state, NSTATE, c->P.fd_order,
-                                                            c->mder);
+    k_metric_der<<<nblk(n), 256, 0, s>>>(G, c->inst_d, c->blk_d, state, NSTATE, c->P.fd_order, c->mder);
     for (int d = 1; d < 3; ++d) {
         if (!c->fmet[d]) {
             hipError_t e = hipMalloc(&c->fmet[d], sizeof(double) * FMC * G.nface[d] * G.nq);
@@ -2780,15 +2790,13 @@ extern "C" grmhd_status grmhd_set_static_metric(grmhd_ctx* c, const double* stat
         }
         const int wpb = (int)nblk(G.nface[d]);
         const dim3 grid((unsigned)(wpb * G.nq));
-        hipStream_t s = (hipStream_t)stream;
         if (d == 1) k_face_metric<1><<<grid, 256, 0, s>>>(G, state, NSTATE, c->O.ex.alp_ex, c->fmet[1], wpb);
         else k_face_metric<2><<<grid, 256, 0, s>>>(G, state, NSTATE, c->O.ex.alp_ex, c->fmet[2], wpb);
     }
     c->mder_src = state;
     c->metric_same = false;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (c->ring_own && hipStreamIsCapturing((hipStream_t)stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
-        const hipStream_t s = (hipStream_t)stream;
+    if (c->ring_own && is_capturing(s)) c->metric_in_graph = true;
+    if (c->ring_own && !c->metric_in_graph) {
         if (!c->metric_diff) HIP_TRY(hipMalloc(&c->metric_diff, sizeof(int32_t)));
         const int per = G.ng * (int)std::max((int64_t)G.N[0] * G.N[1], std::max((int64_t)G.N[0] * G.N[2], (int64_t)G.N[1] * G.N[2]));
         int32_t diff = 0;
@@ -2925,9 +2933,12 @@ static grmhd_status ensure_stage_buffers(grmhd_ctx* c) {
 // block faces, from the neighbouring blocks.  With a curved metric only for
 // the array whose cached metric (grmhd_set_static_metric) was found to agree
 // with itself across block faces: the ring faces are 43% of the faces of 16^3
-// blocks, and the gathers between stages fall away with them.
+// blocks, and the gathers between stages fall away with them.  Not in a graph
+// of the caller's, whose replays outlast the outcome of the comparison: the
+// metric may be another one by then, cached by a later call.  (The context's
+// own graph is dropped by that call.)
 static bool ring_shared(const grmhd_ctx* c, const double* state) {
-    return c->ring_own && (c->P.flat_metric || (c->metric_same && state == c->mder_src));
+    return c->ring_own && (c->P.flat_metric || (c->metric_same && !c->caller_captures && state == c->mder_src));
 }
 
 // Whether the independent launches of a stage run on a side stream beside the
@@ -3081,10 +3092,12 @@ extern "C" grmhd_status grmhd_rk3_step(grmhd_ctx* c, const double* dt_dev, doubl
     grmhd_status r = ensure_stage_buffers(c);
     if (r != GRMHD_OK) return r;
     hipStream_t s = (hipStream_t)stream;
+    c->caller_captures = !c->P.flat_metric && c->metric_same && is_capturing(s);
     {
         Scope sc(c, "step", s);
         rk3_launches(c, dt_dev, state, B, aux, s);
     }
+    c->caller_captures = false;
     return launch_check("rk3_step");
 }
 

@@ -332,8 +332,11 @@ grmhd_status grmhd_rk3_step_graph(grmhd_ctx* ctx, const double* dt_dev, double* 
  * after changing the metric in that array, or enable = 0 to drop it.  On a
  * uniform grid with UCT the call also compares the metric in the ghost cells
  * between blocks with the neighbours' interior (and waits for the stream to
- * do so, unless it is capturing): where they agree to the last bit, the later
- * stages of an RK3 step take those faces from the neighbouring blocks.
+ * do so): where they agree to the last bit, the later stages of an RK3 step
+ * take those faces from the neighbouring blocks.  Not in a graph that the
+ * caller captures (only in that of grmhd_rk3_step_graph), and not in a context
+ * whose call of this function was itself captured: their replays may meet a
+ * metric that was not compared.
  * No effect for flat_metric.  Invalidates a captured RK3 graph. */
 grmhd_status grmhd_set_static_metric(grmhd_ctx* ctx, const double* state, int32_t enable, grmhd_stream_t stream);
 
