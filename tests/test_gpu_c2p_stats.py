@@ -41,3 +41,38 @@ def test_gpu_c2p_stats_sums(n):
     assert s["n_ent_backup"] == int(np.sum((e >> np.uint64(ENT_BACKUP)) & np.uint64(1)))
     assert s["n_atmo_reset"] == int(np.sum((e >> np.uint64(ATMO_RESET)) & np.uint64(1))) >= 1
     assert s["max_root_evals"] <= c.max() and s["n_guess_used"] == 0
+
+
+@pytest.mark.parametrize("n,at", [(1, 0), (257, 256), (777_777, 777_776), (777_777, 0), (2048 * 256 + 1, 2048 * 256),
+                                  (2048 * 256 + 1, 131_071)])
+def test_gpu_c2p_stats_maximum(n, at):
+    """The largest number of root evaluations is that of the one state that
+    takes more than the others, wherever it stands: alone, in the last, partly
+    filled workgroup, in the first, and among records that two launches sum."""
+    import torch
+    dev = torch.device("cuda:0")
+    st = W.c2p_states(4000, seed=3)
+    inst = ga.make_instances([dict(nb=(1, 1, 1), q0=0, bc=(0,) * 6, idx=(1.0, 1.0, 1.0))])
+    ctx = ga.Context(st["params"], ga.Grid(1, 1, 1, 3, 1), inst)
+    cons0 = torch.from_numpy(st["cons"]).to(dev)
+    met0 = torch.from_numpy(st["met"]).to(dev)
+
+    def stats(pick):
+        m = pick.numel()
+        prims = torch.zeros((13, m), dtype=torch.float64, device=dev)
+        err = torch.zeros(m, dtype=torch.int64, device=dev)
+        fl = torch.zeros(m, dtype=torch.uint8, device=dev)
+        ctx.c2p_batch(m, cons0[:, pick].contiguous(), met0[:, pick].contiguous(), prims, err, fl)
+        torch.cuda.synchronize()
+        return ctx.c2p_stats()
+
+    one = [stats(torch.tensor([k], device=dev)) for k in range(40)]
+    roots = [s["n_root_evals"] for s in one]
+    assert all(s["max_root_evals"] == s["n_root_evals"] > 0 for s in one)
+    few, many = int(np.argmin(roots)), int(np.argmax(roots))
+    assert roots[many] > roots[few]
+    pick = torch.full((n,), few, dtype=torch.int64, device=dev)
+    pick[at] = many
+    s = stats(pick)
+    assert s["max_root_evals"] == roots[many]
+    assert s["n_root_evals"] == roots[many] + (n - 1) * roots[few]

@@ -89,3 +89,37 @@ def test_gpu_flux_faces_gs_curved(dev, n, recon, riemann, thermo):
     ref, got, _ = run_rk3_pair(wl, dev, steps=2)
     check_close(wl, ref, got, 1e-12)
     assert np.array_equal(got[2][:, ga.C2P_ERR], ref[2][:, ga.C2P_ERR])
+
+
+@pytest.mark.parametrize("recon_field", ["everywhere", "beside small values"])
+def test_gpu_edge_emfs_overflowing_products(dev, recon_field):
+    """Face B of 1e27: the indicator products of the edge EMFs' transverse
+    reconstructions overflow as well, and the edge takes its other form."""
+    import torch
+    wl = blast_of((2, 1, 2), (6, 7, 6), 3, (_O,) * 6, 0, 0, 0, 0)
+    rng = np.random.default_rng(5)
+    size = 1e27
+    for d, b in enumerate(wl.B):
+        b[...] = size * (0.5 + 0.3 * rng.uniform(-1, 1, b.shape))
+        if recon_field == "beside small values":
+            b[rng.uniform(size=b.shape) < 0.5] *= 1e-30
+    O.Stepper(wl).ghosts(wl.state, wl.B)
+    a = wl.aux
+    a[:, ga.BX] = 0.5 * (wl.B[0][:, 0, :, :, :-1] + wl.B[0][:, 0, :, :, 1:])
+    a[:, ga.BY] = 0.5 * (wl.B[1][:, 0, :, :-1] + wl.B[1][:, 0, :, 1:])
+    a[:, ga.BZ] = 0.5 * (wl.B[2][:, 0, :-1] + wl.B[2][:, 0, 1:])
+    for v in (ga.ZVECX, ga.ZVECY, ga.ZVECZ):
+        a[:, v] = 0.3 * rng.uniform(-1, 1, a[:, v].shape)
+    st, B, aux = wl.copy_arrays()
+    dt = 0.25 * wl.extra["dx"]
+    new_o, nB_o = st.copy(), [b.copy() for b in B]
+    O.Stepper(wl).substep(dt, 1.0, new_o, st, nB_o, B, aux)
+    ctx = ga.Context(wl.params, wl.grid, wl.instances)
+    sg, Bg, ag = dev_arrays(wl, dev)
+    ng, nBg = sg.clone(), [b.clone() for b in Bg]
+    ctx.advance_substep(torch.tensor([dt], dtype=torch.float64, device=dev), 1.0, ng, sg, nBg, Bg, ag)
+    torch.cuda.synchronize()
+    for d in range(3):
+        got = to_host(nBg[d])
+        assert np.isfinite(got).all() and np.max(np.abs(nB_o[d] - B[d])) > 1e-3 * size
+        assert linf_rel(got, nB_o[d]) < 1e-12, d
