@@ -70,7 +70,8 @@ struct DevGrid {
     // doubles, N[1] + 1 rows to a plane, element i of a row at so + i.  sp
     // and so put the first interior element of every row on a 128-byte
     // boundary: a row of 16 faces is then one whole line, written and read
-    // with one request.  (With the rows of the boundary's arrays, 22 doubles
+    // with one request (rows without gaps where memory is scarce, see the
+    // context's creation).  (With the rows of the boundary's arrays, 22 doubles
     // from byte 24 on, each row shares both its lines with the next rows, and
     // a kernel that walks along y writes every line twice, in parts: y faces
     // 314 us against 258 us, z 277 against 224, 512 blocks of 16^3.)
@@ -1764,9 +1765,20 @@ static grmhd_status ctx_create_impl(const grmhd_params* p, const grmhd_grid* g, 
     G.ncell = (int64_t)G.N[0] * G.N[1] * G.N[2];
     for (int d = 0; d < 3; ++d) G.nface[d] = (int64_t)(G.N[0] + (d == 0)) * (G.N[1] + (d == 1)) * (G.N[2] + (d == 2));
     G.nedge = (int64_t)(G.N[0] + 1) * (G.N[1] + 1) * (G.N[2] + 1);
-    G.sp = (G.N[0] + 1 + 15) / 16 * 16;
-    G.so = (16 - G.ng % 16) % 16;
-    G.ns = (G.so + (int64_t)G.sp * (G.N[1] + 1) * (G.N[2] + 1) + 15) / 16 * 16;
+    // Rows on whole lines (see DevGrid), unless the 3 (7 + 4) + 3 components of
+    // the face and edge arrays would take more than a third of the free memory
+    // with them: 1.4 times as much for blocks of 16^3 as without gaps.  The
+    // stage buffers, the metric caches and the caller's arrays need up to twice
+    // as much again, and a grid that fits only without the gaps has to fit.
+    // (128^3 blast step 4.61 ms with whole lines, 5.05 without gaps.)
+    size_t free_bytes = 0, all_bytes = 0;
+    hipError_t e = hipMemGetInfo(&free_bytes, &all_bytes);
+    for (int whole = 1; whole >= 0; --whole) {
+        G.sp = whole ? (G.N[0] + 1 + 15) / 16 * 16 : G.N[0] + 1;
+        G.so = whole ? (16 - G.ng % 16) % 16 : 0;
+        G.ns = (G.so + (int64_t)G.sp * (G.N[1] + 1) * (G.N[2] + 1) + 15) / 16 * 16;
+        if (e != hipSuccess || 3. * 36. * sizeof(double) * (double)(G.ns * G.nq) <= (double)free_bytes) break;
+    }
     Opts& O = c->O;
     O.atmo = Atmo{p->rho_fl, p->temp_fl, p->ye_fl, p->atmo_tol};
     O.cp = C2PPar{p->c2p_tol, p->max_lorentz, p->max_sigma, p->beta_fallback, p->bh_alp_thresh, p->use_entropy_backup};
@@ -1789,7 +1801,6 @@ static grmhd_status ctx_create_impl(const grmhd_params* p, const grmhd_grid* g, 
         free_ctx(c); delete c;
         return GRMHD_ERR_ALLOC;
     };
-    hipError_t e;
     if (n_inst > 0) {
         if ((e = hipMalloc(&c->inst_d, sizeof(DevInst) * n_inst)) != hipSuccess) return fail("inst", e);
         if ((e = hipMemcpy(c->inst_d, c->inst_h.data(), sizeof(DevInst) * n_inst, hipMemcpyHostToDevice)) != hipSuccess) return fail("inst copy", e);
