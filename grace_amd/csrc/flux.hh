@@ -365,17 +365,20 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
 // workgroups of a block follow each other direction by direction, plane by
 // plane along z, on one XCD (wg_pos_in), then the next block's: the three
 // directions read the same nine primitives, and the second and third find
-// them in that XCD's L2.  Ring faces (only the first RK stage has many) come
-// behind the full faces of all blocks: their threads are shorter.
+// them in that XCD's L2.  Ring faces (many in the first RK stage, and in every
+// stage of a forest and of a curved grid without a cached metric that agrees
+// across block faces) come behind the full faces of all blocks: their threads
+// are shorter.
 //
 // Bound by the FP64 units (about 350 us of arithmetic for 512 blocks of
-// 16^3) beside the stores of fluxes and face values: 500 us per launch there
-// in the RK stages that share ring faces, 430 without the flux stores; one
-// launch per direction over rows in the boundary's layout, which also copied
-// its outer face values into the neighbours' ring slots, took 3 x 245.  (The
-// edge EMFs read them from the neighbour instead: 130 MB less to write.)  A
-// thread per face with nine variables one after another needs 126 VGPRs (4
-// waves per SIMD; curved 165, 3 waves).  A thread that walks along a line of
+// 16^3) beside the stores of fluxes and face values: 535 us per launch there
+// in the RK stages that share ring faces, 725 with them (500 and 430, the
+// latter without the flux stores, on a card with faster memory); one launch
+// per direction over rows in the boundary's layout, which also copied its
+// outer face values into the neighbours' ring slots, took 3 x 245.  (The edge
+// EMFs read them from the neighbour instead: 130 MB less to write.)  A thread
+// per face with nine variables one after another needs 126 VGPRs (4 waves per
+// SIMD; curved 167, 3 waves: the bound of 3 keeps the hybrid EOS from 169).  A thread that walks along a line of
 // faces saves the shared half of the reconstruction but keeps the stencils of
 // nine variables: 230 VGPRs, 2 waves, 1.0 ms for y and 0.9 for z per three
 // stages against 0.67 and 0.64 here; with the stencil read again at each step

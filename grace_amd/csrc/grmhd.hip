@@ -884,9 +884,6 @@ GHD int map_fc(int f, int N, int lo, int hi) {
 // from any interior cell: it needs its own c2p.  Every other ghost cell (same
 // level neighbour or periodic image) has the exact inputs of its source cell,
 // so its c2p outputs are copies of the source's.
-GHD bool cell_is_interior(const DevGrid& G, int i, int j, int k) {
-    return i >= G.ng && i < G.n[0] + G.ng && j >= G.ng && j < G.n[1] + G.ng && k >= G.ng && k < G.n[2] + G.ng;
-}
 GHD bool ghost_needs_own_c2p(const DevGrid& G, const DevInst& I, const DevBlk& b, int i, int j, int k) {
     int loc[3] = {i, j, k};
     for (int d = 0; d < 3; ++d) {
@@ -1134,9 +1131,10 @@ static __device__ __align__(256) DevStats scratch[GRMHD_NOALLOC_MAX_STATES / 256
 // Resident 256-thread blocks per CU that the c2p kernels are built for: 3
 // (168 VGPRs) where little spills, 2 (256 VGPRs, no spills) where the metric
 // or the network's fragments stay alive across the root solves.  With 3 / 2:
-// flat cells (128^3 step) 4300 / 4295 us, curved cells 80^3 1548 / 1503 and
-// the torus forest 2074 / 2014, learned batch of 1M 201 / 193; plain batch of
-// 4M 860 / 935.  With 4 every one is slower (spills of 200 bytes and more).
+// flat cells (128^3 blast step) 4768 / 4779 us, cells with a metric (curved
+// 80^3 step 1642 / 1598, torus forest 2212 / 2165), learned batch of 1M
+// 189 / 177; plain batch of 4M 844 / 931.  With 4 every one is slower (spills
+// of 200 bytes and more).
 constexpr int c2p_cells_blocks(bool flat) { return flat ? 3 : 2; }
 constexpr int c2p_batch_blocks(bool learned) { return learned ? 2 : 3; }
 // Cell sets: CS_INTERIOR (the interior cells of every block, wpb workgroups
@@ -2166,8 +2164,6 @@ static grmhd_status launch_check(const char* what) {
 }
 
 // ---- dispatch helpers -------------------------------------------------------
-// only != null: FOFC correction pass over the tagged faces with the options O
-// (donor cell + LLF); otherwise every face the later passes read.
 static FluxArgs flux_args(grmhd_ctx* c, const double* aux, const double* ms, int mnv, const double* const B[3]) {
     FluxArgs f{};
     f.aux = aux; f.mstate = ms; f.mnv = mnv;
@@ -2179,6 +2175,8 @@ static FluxArgs flux_args(grmhd_ctx* c, const double* aux, const double* ms, int
     }
     return f;
 }
+// FOFC correction pass over the tagged faces (only) with the options O (donor
+// cell + LLF).
 template <typename EOS>
 static void launch_flux_tagged(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O,
                                uint8_t* const* only) {
@@ -2956,12 +2954,21 @@ static bool ring_shared(const grmhd_ctx* c, const double* state) {
 // main one, from 2^18 interior cells on.  Below, a launch does not fill the
 // card for longer than a fork and a join cost, and one stream also lets
 // launches merge (update cells with faces, ghost faces with conserved, interior
-// c2p with that of the ghosts: six launches a stage).  RK3 steps with / without
-// the side stream, 16^3 blocks, us eager and as a graph: 8 blocks 335 / 187
-// and 224 / 195, 27 blocks 401 / 333 and 354 / 346, 48 blocks 564 / 506 and
-// 521 / 518, 64 blocks 692 / 680 and 658 / 684, 100 blocks 980 / 1009 and
-// 945 / 1012; curved, 27 blocks 609 / 519 and 532 / 532, 64 blocks
-// 1110 / 1074 and 1068 / 1070.
+// c2p with that of the ghosts: six launches a stage).  RK3 steps of 16^3 blocks
+// in us:
+//             side stream          one stream
+//             eager    graph       eager    graph
+//     8       335      187         224      195
+//    27       401      333         354      346     curved 609 519 / 532 532
+//    48       564      506         521      518
+//    64       692      680         658      684     curved 1110 1074 / 1068 1070
+//   100       980     1009         945     1012
+// A graph, in which a fork costs little, gains up to 4% from the side stream
+// below the line too; eager steps, and curved ones, still lose up to 5% at 64
+// blocks, which is the line, and 4% at 100.  The line is where both are within
+// 5% of the better order; the larger grids that it is for run the update's
+// cell part, bound by memory, beside the edge EMFs, bound by their
+// instructions.
 constexpr int64_t CONC_MIN_CELLS = 1 << 18;
 static bool stage_conc(const grmhd_ctx* c) {
     const DevGrid& G = c->G;

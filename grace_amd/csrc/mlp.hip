@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void k_mlp_forward(int64_t n, MlpDev w, const 
 // entry: loss).
 //
 // Bound by latency: a chunk is some 5000 cycles of matrix instructions per
-// SIMD between five barriers.  With k_mlp_reduce 12.6 us for 4096 states,
+// SIMD between six barriers.  With k_mlp_reduce 12.6 us for 4096 states,
 // against 66.8 with one wave per chunk that kept a row of every product per
 // lane, and one thread per column of the sum.
 // ---------------------------------------------------------------------------

@@ -49,7 +49,7 @@ GHD double sq(double x) { return x * x; }
 // 1/b for a normal, finite b: the hardware reciprocal refined by two
 // Newton-Raphson steps r <- r + r (1 - b r) (within 1 ulp of 1/b; about half
 // the instructions of an IEEE division, which also handles zero, infinity and
-// denormal operands).  Host builds divide.
+// denormal operands: here they give NaN).  Host builds divide.
 GHD double nr_rcp(double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
     double r = __builtin_amdgcn_rcp(b);
@@ -74,9 +74,10 @@ GHD double quot(double a, double b, double ib) {
 #endif
 }
 // sqrt(x) and 1/sqrt(x) for a normal, finite x > 0: the hardware's reciprocal
-// root (about 24 bits) and two coupled Newton steps, the last one on the
-// residual x - g^2; half the instructions of the library's root and a
-// division.  Host builds use those.
+// root (about 24 bits), one step of Goldschmidt's coupled iteration for g and
+// 1/(2g) and a correction by the residual x - g^2 (Markstein); half the
+// instructions of the library's root and a division.  Host builds use those.
+// (An infinite x gives NaN, not infinity.)
 GHD void nr_sqrt(double x, double& g, double& ig) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const double y = __builtin_amdgcn_rsq(x);
@@ -1047,12 +1048,16 @@ struct C2POut { bool floored, fatal; };
 
 // conservs_to_prims (c2p.cpp:188-414).  cons densitised in, re-densitised out.
 // X: every quotient and root an IEEE operation, the master functions in the
-// general form.  For GS EMFs on a curved metric: they choose a side by the
-// sign of the mass flux, which in a stationary flow (a torus: no poloidal
-// velocity) is rounding at many faces, and primitives that differ in the last
-// bit move the field by 1e-6 of its largest value in one step.  The other
-// form is as accurate (2.8e-11 against 64-bit bisection either way) and takes
-// 0.7 of the time.
+// general form.  For GS EMFs on a curved metric with the plain solve: they
+// choose a side by the sign of the mass flux, which in a stationary flow (a
+// torus: no poloidal velocity) is rounding at many faces, and one ulp in the
+// primitives was seen to move single faces of the field by 5e-6 of its largest
+// value in one step.  (The Newton finish of the learned and the warm-started
+// guess has another root in the last digits anyway and takes the other form:
+// over tori on grids and forests the field stays within 7e-16 of the one with
+// divisions, the conserved within 6e-15.)  The other form is as accurate
+// (against 128-bit solves of 720 000 states 0.998 +- 0.012 of the error with
+// divisions) and takes 0.7 of the time.
 template <bool FL, bool X, typename EOS>
 GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eos, const Atmo& at,
                const ExcPar& ex, const C2PPar& cp, double radius, uint64_t& err, bool dry_run, C2PCount& cnt,
@@ -1169,10 +1174,12 @@ GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eo
 // left state) from um2..up2.  The candidates pair with the linear weights in
 // opposite order.  Everything is formed from the four differences of
 // neighbours, and a face value is u0 plus a correction, so that smooth data
-// lose no digits to the candidates' large coefficients.  The multiply-adds are written out: a value that two blocks
-// form (a face on their common boundary) then has the same bits wherever this
-// is inlined.  Here every ratio is divided by itself (values of any size):
-// the wide form, taken where wenoz_face says so.
+// lose no digits to the candidates' large coefficients.  The multiply-adds are
+// written out: a value that two blocks form (a face on their common boundary)
+// then has the same bits wherever this is inlined, in the same form (which is
+// why each variable of a face chooses its form by itself).  Here every ratio
+// is divided by itself (values of any size): the wide form, taken where
+// wenoz_face says so.
 struct WenoCell { double d0, d1, d2, cl[3], ch[3]; };
 GHD void weno_cell_parts(double um2, double um1, double u0, double up1, double up2, WenoCell& w) {
 #pragma clang fp contract(off)
@@ -1305,10 +1312,7 @@ GHD void recon(double um2, double um1, double u0, double up1, double& uL, double
         uL = um1 + 0.5 * (REC == 1 ? mc2(sL, sR) : minmod(sL, sR));
     }
 }
-GHD double hll(double fL, double fR, double uL, double uR, double cmin, double cmax) {
-    return (cmax * fL + cmin * fR - cmax * cmin * (uR - uL)) / (cmax + cmin);
-}
-// hll with the reciprocal of cmax + cmin shared by the fluxes of one face
+// HLL with the reciprocal inv of cmax + cmin, which the fluxes of a face share
 GHD double hll_r(double fL, double fR, double uL, double uR, double cmin, double cmax, double inv) {
     return (cmax * fL + cmin * fR - cmax * cmin * (uR - uL)) * inv;
 }
