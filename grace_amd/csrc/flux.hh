@@ -2,9 +2,8 @@
 // evolve.cpp:813-1068, grmhd.hh:551-970).
 //
 // Included by grmhd.hip after the block geometry (DevGrid, Opts, wg_pos,
-// face_metric).  k_flux solves the faces of all three directions in one
-// launch, one thread per face; k_flux_tagged redoes the faces that the
-// first-order correction tagged.
+// face_metric).  k_flux (UCT) and k_flux_gs (Gardiner-Stone EMFs) solve the
+// faces of all three directions in one launch, one thread per face.
 #pragma once
 
 // The reconstructed variables of a face (the normal B is the face value).
@@ -28,9 +27,9 @@ GHD int fq_aux(int v, int thermo) {
 }
 
 // Fluxes of one face of direction D from the states below (L) and above (R)
-// it (compute_mhd_fluxes, grmhd.hh:774-970).  V: UCT (emf 0) the HLL-averaged
-// transverse transport velocities and the wave speeds; GS (emf 1) the two
-// face EMFs in V[0], V[1].  A ring face returns after V.
+// it for UCT (compute_mhd_fluxes, grmhd.hh:774-970).  V: the HLL-averaged
+// transverse transport velocities and the wave speeds.  A ring face returns
+// after V.
 template <typename EOS, bool FLAT, int D>
 GHD void face_solve(const EOS& eos, const Opts& o, const Met& mf, const double L[FQ_N], const double R[FQ_N], double Bn,
                     bool ring, double V[4], double F[7]) {
@@ -100,20 +99,10 @@ GHD void face_solve(const EOS& eos, const Opts& o, const Met& mf, const double L
     if (cmin < 1e-12 && cmax < 1e-12) { cmin = 1; cmax = 1; }
     const double ihll = nr_rcp(cmax + cmin);   // shared by the HLL fluxes of this face
     const double sg = mf.sqrtg;
-    if (o.emf == 0) {
-        V[0] = hll_r(vtl[J0], vtr[J0], 0, 0, cmin, cmax, ihll);
-        V[1] = hll_r(vtl[J1], vtr[J1], 0, 0, cmin, cmax, ihll);
-        V[2] = cmin; V[3] = cmax;
-        if (ring) return;
-    } else {
-        // induction fluxes v_D B_c - v_c B_D of the transverse components
-        // (grmhd.hh:937-969)
-        constexpr double s = D == 1 ? -1.0 : 1.0;
-        V[0] = s * sg * hll_r(-Bl[D] * vtl[J1] + Bl[J1] * vtl[D], -Br[D] * vtr[J1] + Br[J1] * vtr[D], Bl[J1], Br[J1],
-                              cmin, cmax, ihll);
-        V[1] = -s * sg * hll_r(-Bl[D] * vtl[J0] + Bl[J0] * vtl[D], -Br[D] * vtr[J0] + Br[J0] * vtr[D], Bl[J0], Br[J0],
-                               cmin, cmax, ihll);
-    }
+    V[0] = hll_r(vtl[J0], vtr[J0], 0, 0, cmin, cmax, ihll);
+    V[1] = hll_r(vtl[J1], vtr[J1], 0, 0, cmin, cmax, ihll);
+    V[2] = cmin; V[3] = cmax;
+    if (ring) return;
     // conserved and fluxes along D (grmhd_subexpressions.hh:97-156)
     double bsh[3];
     lower3(mf.g, mf.beta[0], mf.beta[1], mf.beta[2], bsh);
@@ -196,17 +185,13 @@ __device__ __forceinline__ void settle(double& lo, double& hi) {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// The transverse indices (ghosts included) of line p of direction D: UCT the
+// The transverse indices (ghosts included) of line p of direction D: the
 // n0 n1 lines with both interior, or (ring) the lines with exactly one in
 // the ghost layers (they feed only the transverse reconstructions of the
-// edge EMFs; lines with both in the ghost layers are never read); GS every
-// line.  False where there is none or another block writes it.
-GHD bool line_pos(const DevGrid& G, int T0, int T1, bool uct, bool ring, int p, uint8_t own, bool use_own, int& b, int& c) {
+// edge EMFs; lines with both in the ghost layers are never read).  False where
+// there is none or another block writes it.
+GHD bool line_pos(const DevGrid& G, int T0, int T1, bool ring, int p, uint8_t own, bool use_own, int& b, int& c) {
     const int ng = G.ng, n0 = G.n[T0], n1 = G.n[T1];
-    if (!uct) {
-        udivmod(p, G.N[T0], c, b);
-        return c < G.N[T1];
-    }
     if (!ring) {
         udivmod(p, n0, c, b);
         b += ng; c += ng;
@@ -258,22 +243,19 @@ template <typename EOS, int REC, bool FLAT, int D>
 __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, const Opts& o, const FluxArgs& f, int64_t q,
                                           int e, bool ring) {
     constexpr int T0 = D == 0 ? 1 : 0, T1 = D == 2 ? 1 : 2;
-    const bool uct = o.emf == 0;
-    const int wide = uct ? 0 : o.fofc, Rn = G.n[D] + 1 + 2 * wide, ng = G.ng, nD = G.n[D];
+    const int Rn = G.n[D] + 1, ng = G.ng, nD = G.n[D];
     int a, b, c, r;
     if (D == 1 && !ring) {
         // x, then the normal, then z
-        const int n0 = uct ? G.n[T0] : G.N[T0], n1 = uct ? G.n[T1] : G.N[T1];
-        udivmod(e, n0, r, b); udivmod(r, Rn, c, a);
-        if (c >= n1) return;
-        if (uct) { b += ng; c += ng; }
+        udivmod(e, G.n[T0], r, b); udivmod(r, Rn, c, a);
+        if (c >= G.n[T1]) return;
+        b += ng; c += ng;
     } else {
-        const int per = ring ? 2 * ng * (G.n[T0] + G.n[T1]) : (uct ? G.n[T0] * G.n[T1] : G.N[T0] * G.N[T1]);
+        const int per = ring ? 2 * ng * (G.n[T0] + G.n[T1]) : G.n[T0] * G.n[T1];
         int p;
         if (D == 0) udivmod(e, Rn, p, a); else udivmod(e, per, a, p);
-        if (a >= Rn || !line_pos(G, T0, T1, uct, ring, p, (ring && f.ring_own) ? f.ring_own[q] : 0, f.ring_own != nullptr, b, c)) return;
+        if (a >= Rn || !line_pos(G, T0, T1, ring, p, (ring && f.ring_own) ? f.ring_own[q] : 0, f.ring_own != nullptr, b, c)) return;
     }
-    a -= wide;
     const int m0 = ng + a;
     const int i = D == 0 ? m0 : b, j = D == 1 ? m0 : (D == 0 ? b : c), k = D == 2 ? m0 : c;
     const int64_t nc = G.ncell, nf = G.nface[D];
@@ -352,9 +334,8 @@ __device__ __forceinline__ void flux_face(const DevGrid& G, const EOS& eos, cons
     const int64_t ns = G.ns;
     const uint32_t so = (uint32_t)sidx(G, i, j, k) * 8u;
     double* V0 = f.vbar[D] + q * 4 * ns;
-    st_off(V0, so, V[0]);
-    st_off(V0 + ns, so, V[1]);
-    if (uct) { st_off(V0 + 2 * ns, so, V[2]); st_off(V0 + 3 * ns, so, V[3]); }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) st_off(V0 + v * ns, so, V[v]);
     if (ring) return;
     double* F0 = f.flux[D] + q * NHRSC * ns;
 #pragma unroll
@@ -399,54 +380,18 @@ __global__ __launch_bounds__(256, 3) void k_flux(DevGrid G, EOS eos, Opts o, Flu
     }
 }
 
-// FOFC correction (evolve.cpp:646-702): the tagged faces of the normal range
-// [ng, n + ng], every transverse index, from donor cells with the options o
-// (LLF); one thread per face, x across the lanes.  Flat metric; a curved one
-// takes k_flux_gs_curved.
-template <typename EOS, int D>
-__global__ __launch_bounds__(256) void k_flux_tagged(DevGrid G, EOS eos, Opts o, FluxArgs f, const uint8_t* __restrict__ only) {
-    const WgPos wp = wg_pos(f.tiles);
-    const int64_t q = wp.q;
-    const int e = wp.tile * (int)blockDim.x + (int)threadIdx.x;
-    const int E0 = D == 0 ? G.n[0] + 1 : G.N[0], E1 = D == 1 ? G.n[1] + 1 : G.N[1], E2 = D == 2 ? G.n[2] + 1 : G.N[2];
-    if (e >= E0 * E1 * E2) return;
-    int r, i, j, k;
-    udivmod(e, E0, r, i);
-    udivmod(r, E1, k, j);
-    if (D == 0) i += G.ng;
-    else if (D == 1) j += G.ng;
-    else k += G.ng;
-    const int64_t nf = G.nface[D], fo = fidx<D>(G, i, j, k);
-    if (!only[q * nf + fo]) return;
-    const int64_t nc = G.ncell;
-    const int64_t st = D == 0 ? 1 : (D == 1 ? G.N[0] : (int64_t)G.N[0] * G.N[1]);
-    Met mf;
-    bool excise;
-    face_met<true, D>(G, f, o.ex.alp_ex, q, i, j, k, st, mf, excise);
-    const double* A = f.aux + q * NAUX * nc + cidx(G, i, j, k);
-    double L[FQ_N], R[FQ_N], V[4], F[7];
-#pragma unroll
-    for (int v = 0; v < FQ_N; ++v) {
-        const double* P = A + fq_aux<D>(v, o.thermo) * nc;
-        L[v] = P[-st]; R[v] = P[0];
-    }
-    face_solve<EOS, true, D>(eos, o, mf, L, R, f.B[D][q * nf + fo] / mf.sqrtg, false, V, F);
-    const int64_t so = sidx(G, i, j, k);
-    double* V0 = f.vbar[D] + q * 4 * G.ns + so;
-    V0[0] = V[0]; V0[G.ns] = V[1];
-    double* F0 = f.flux[D] + q * NHRSC * G.ns + so;
-#pragma unroll
-    for (int v = 0; v < NHRSC; ++v) F0[v * G.ns] = F[v];
-}
-
-// Fluxes and face EMFs for GS on a curved metric: face e of direction D of
-// block q, of every face (FOFC widens the normal range by one face on each
-// side; only: its correction pass, the tagged faces).  Every quotient is an
-// IEEE division and the wave speeds are get_cm_cp's, for the sign of the mass
-// flux (see c2p), which is why this path is not k_flux's.
-template <typename EOS, int REC, int D>
-__device__ __forceinline__ void gs_curved_face(const DevGrid& G, const EOS& eos, const Opts& o, const FluxArgs& f,
-                                               const uint8_t* only, int64_t q, int e) {
+// Fluxes and face EMFs for GS: face e of direction D of block q, of every face
+// (FOFC widens the normal range by one face on each side; only: its correction
+// pass, evolve.cpp:646-702, the tagged faces of the normal range [ng, n + ng]).
+// WENO-Z is formed from the candidates, every quotient is an IEEE division and
+// the wave speeds are get_cm_cp's, for the sign of the mass flux: the edge EMF
+// takes a side by it, and where nothing flows (between two cells reset to the
+// floor, in a stationary flow) that sign is rounding.  With k_flux's forms B
+// is off by 0.2 of its largest value at single faces beside floored cells,
+// which is why this path is not k_flux's.
+template <typename EOS, int REC, bool FLAT, int D>
+__device__ __forceinline__ void gs_face(const DevGrid& G, const EOS& eos, const Opts& o, const FluxArgs& f,
+                                        const uint8_t* only, int64_t q, int e) {
     constexpr int T0 = D == 0 ? 1 : 0, T1 = D == 2 ? 1 : 2;
     const int N0 = G.N[T0], N1 = G.N[T1], Rg = G.n[D] + 1 + 2 * o.fofc;
     if (e >= Rg * N0 * N1) return;
@@ -462,21 +407,8 @@ __device__ __forceinline__ void gs_curved_face(const DevGrid& G, const EOS& eos,
     const int64_t st = D == 0 ? 1 : (D == 1 ? G.N[0] : (int64_t)G.N[0] * G.N[1]);
     const double* A = f.aux + q * NAUX * nc;
     Met mf;
-    bool excise_override = false;
-    if (f.fmc[D]) {
-        // the face-metric cache: only the inverse component this direction
-        // uses (cmcp, the LLF speed limit) is kept
-        const int64_t nfd = G.nface[D];
-        const double* FM = f.fmc[D] + q * FMC * nfd + fidx<D>(G, i, j, k);
-        for (int a = 0; a < 6; ++a) { mf.g[a] = FM[a * nfd]; mf.gi[a] = 0.0; }
-        mf.gi[D == 0 ? 0 : (D == 1 ? 3 : 5)] = FM[6 * nfd];
-        for (int a = 0; a < 3; ++a) mf.beta[a] = FM[(7 + a) * nfd];
-        mf.alp = FM[10 * nfd];
-        mf.sqrtg = FM[11 * nfd];
-        excise_override = FM[12 * nfd] != 0.0;
-    } else {
-        face_metric(f.mstate + q * (int64_t)f.mnv * nc, nc, c0, st, o.ex.alp_ex, mf, excise_override);
-    }
+    bool excise = false;
+    face_met<FLAT, D>(G, f, o.ex.alp_ex, q, i, j, k, st, mf, excise);
     // reconstruction of RHO Z(3) YE THERMO ENT B(3)
     const int th_aux = o.thermo ? PRESS_ : TEMP_;
     const int ridx[10] = {RHO_, ZVECX_, ZVECY_, ZVECZ_, YE_, th_aux, ENTROPY_, BX_, BY_, BZ_};
@@ -488,7 +420,7 @@ __device__ __forceinline__ void gs_curved_face(const DevGrid& G, const EOS& eos,
         if (v == 7 + D) { pL[rloc[v]] = 0.0; pR[rloc[v]] = 0.0; continue; }
         double uL, uR;
         const double* P = A + ridx[v] * nc + c0;
-        if (excise_override) { uL = P[-st]; uR = P[0]; }
+        if (!FLAT && excise) { uL = P[-st]; uR = P[0]; }
         else if constexpr (REC == 0) wenoz(P[-3 * st], P[-2 * st], P[-st], P[0], P[st], P[2 * st], uL, uR);
         else recon<REC>(P[-2 * st], P[-st], P[0], P[st], uL, uR);
         pL[rloc[v]] = uL; pR[rloc[v]] = uR;
@@ -506,16 +438,16 @@ __device__ __forceinline__ void gs_curved_face(const DevGrid& G, const EOS& eos,
     }
     // compute_mhd_fluxes (grmhd.hh:774-970)
     const double *zl = &pL[ZXL], *zr = &pR[ZXL], *Bl = &pL[BXL], *Br = &pR[BXL];
-    double wl = lorentz<false>(mf.g, zl), wr = lorentz<false>(mf.g, zr);
+    double wl = lorentz<FLAT>(mf.g, zl), wr = lorentz<FLAT>(mf.g, zr);
     double bl[4], br[4], b2l, b2r;
-    smallb<false>(mf, Bl, zl, wl, bl, b2l);
-    smallb<false>(mf, Br, zr, wr, br, b2r);
+    smallb<FLAT>(mf, Bl, zl, wl, bl, b2l);
+    smallb<FLAT>(mf, Br, zr, wr, br, b2r);
     double vtl[3], vtr[3];
     vtilde(mf, zl, wl, vtl);
     vtilde(mf, zr, wr, vtr);
     double cml, cpl, cmr, cpr, cmin, cmax;
-    cmcp<false>(mf, pL[RHOL], pL[PRESSL], pL[EPSL], pL[CS2L], wl, b2l, vtl, D, cml, cpl);
-    cmcp<false>(mf, pR[RHOL], pR[PRESSL], pR[EPSL], pR[CS2L], wr, b2r, vtr, D, cmr, cpr);
+    cmcp<FLAT>(mf, pL[RHOL], pL[PRESSL], pL[EPSL], pL[CS2L], wl, b2l, vtl, D, cml, cpl);
+    cmcp<FLAT>(mf, pR[RHOL], pR[PRESSL], pR[EPSL], pR[CS2L], wr, b2r, vtr, D, cmr, cpr);
     if (o.riemann == 1) {
         cmax = fmax(fmax(fabs(cml), fabs(cmr)), fmax(fabs(cpl), fabs(cpr)));
         if (fmin(pL[RHOL], pR[RHOL]) < o.c_limit) {
@@ -532,8 +464,8 @@ __device__ __forceinline__ void gs_curved_face(const DevGrid& G, const EOS& eos,
     const int64_t so = sidx(G, i, j, k), ns = G.ns;
     double* V = f.vbar[D] + q * 4 * ns + so;
     double Dl, taul, Sl[3], Esl, Dr, taur, Sr[3], Esr;
-    conserved<false>(mf, pL[RHOL], pL[PRESSL], pL[EPSL], zl, pL[ENTL], wl, b2l, bl, Dl, taul, Sl, Esl);
-    conserved<false>(mf, pR[RHOL], pR[PRESSL], pR[EPSL], zr, pR[ENTL], wr, b2r, br, Dr, taur, Sr, Esr);
+    conserved<FLAT>(mf, pL[RHOL], pL[PRESSL], pL[EPSL], zl, pL[ENTL], wl, b2l, bl, Dl, taul, Sl, Esl);
+    conserved<FLAT>(mf, pR[RHOL], pR[PRESSL], pR[EPSL], zr, pR[ENTL], wr, b2r, br, Dr, taur, Sr, Esr);
     // fluxes along D (grmhd_subexpressions.hh:97-156)
     double bsh[3]; lower3(mf.g, mf.beta[0], mf.beta[1], mf.beta[2], bsh);
     double ia2 = 1. / (mf.alp * mf.alp);
@@ -544,12 +476,19 @@ __device__ __forceinline__ void gs_curved_face(const DevGrid& G, const EOS& eos,
         double W2rh = wl * wl * rhoh;
         double fD = vtl[D] * Dl;
         Fl[0] = fD;
-        double blo[3]; lower3<false>(mf.g, bl[1], bl[2], bl[3], blo);
-        double vlo[3]; lower3<false>(mf.g, vtl[0], vtl[1], vtl[2], vlo);
-        Fl[4] = W2rh * vtl[D] + ps * mf.beta[D] - mf.alp * mf.alp * bl[0] * bl[1 + D] - fD;
-        const double c = vtl[D] * W2rh * ia2;
-        for (int a = 0; a < 3; ++a)
-            Fl[1 + a] = mf.alp * (-bl[1 + D] * (blo[a] + bl[0] * bsh[a]) + (a == D ? ps : 0.0) + c * (vlo[a] + bsh[a]));
+        double blo[3]; lower3<FLAT>(mf.g, bl[1], bl[2], bl[3], blo);
+        double vlo[3]; lower3<FLAT>(mf.g, vtl[0], vtl[1], vtl[2], vlo);
+        if constexpr (FLAT) {
+            Fl[4] = W2rh * vtl[D] - bl[0] * bl[1 + D] - fD;
+            const double c = vtl[D] * W2rh;
+            for (int a = 0; a < 3; ++a)
+                Fl[1 + a] = a == D ? -bl[1 + D] * blo[a] + ps + c * vlo[a] : -bl[1 + D] * blo[a] + c * vlo[a];
+        } else {
+            Fl[4] = W2rh * vtl[D] + ps * mf.beta[D] - mf.alp * mf.alp * bl[0] * bl[1 + D] - fD;
+            const double c = vtl[D] * W2rh * ia2;
+            for (int a = 0; a < 3; ++a)
+                Fl[1 + a] = mf.alp * (-bl[1 + D] * (blo[a] + bl[0] * bsh[a]) + (a == D ? ps : 0.0) + c * (vlo[a] + bsh[a]));
+        }
         Fl[6] = vtl[D] * Esl;
         Fl[5] = pL[YEL] * fD;
     }
@@ -559,12 +498,19 @@ __device__ __forceinline__ void gs_curved_face(const DevGrid& G, const EOS& eos,
         double W2rh = wr * wr * rhoh;
         double fD = vtr[D] * Dr;
         Fr[0] = fD;
-        double blo[3]; lower3<false>(mf.g, br[1], br[2], br[3], blo);
-        double vlo[3]; lower3<false>(mf.g, vtr[0], vtr[1], vtr[2], vlo);
-        Fr[4] = W2rh * vtr[D] + ps * mf.beta[D] - mf.alp * mf.alp * br[0] * br[1 + D] - fD;
-        const double c = vtr[D] * W2rh * ia2;
-        for (int a = 0; a < 3; ++a)
-            Fr[1 + a] = mf.alp * (-br[1 + D] * (blo[a] + br[0] * bsh[a]) + (a == D ? ps : 0.0) + c * (vlo[a] + bsh[a]));
+        double blo[3]; lower3<FLAT>(mf.g, br[1], br[2], br[3], blo);
+        double vlo[3]; lower3<FLAT>(mf.g, vtr[0], vtr[1], vtr[2], vlo);
+        if constexpr (FLAT) {
+            Fr[4] = W2rh * vtr[D] - br[0] * br[1 + D] - fD;
+            const double c = vtr[D] * W2rh;
+            for (int a = 0; a < 3; ++a)
+                Fr[1 + a] = a == D ? -br[1 + D] * blo[a] + ps + c * vlo[a] : -br[1 + D] * blo[a] + c * vlo[a];
+        } else {
+            Fr[4] = W2rh * vtr[D] + ps * mf.beta[D] - mf.alp * mf.alp * br[0] * br[1 + D] - fD;
+            const double c = vtr[D] * W2rh * ia2;
+            for (int a = 0; a < 3; ++a)
+                Fr[1 + a] = mf.alp * (-br[1 + D] * (blo[a] + br[0] * bsh[a]) + (a == D ? ps : 0.0) + c * (vlo[a] + bsh[a]));
+        }
         Fr[6] = vtr[D] * Esr;
         Fr[5] = pR[YEL] * fD;
     }
@@ -602,15 +548,15 @@ __device__ __forceinline__ void gs_curved_face(const DevGrid& G, const EOS& eos,
 // 24^3 209 -> 172 against a launch per direction (2523, 2037 and 499 with
 // those on three streams).
 struct FaceTags { const uint8_t* d[3]; };
-template <typename EOS, int REC>
-__global__ __launch_bounds__(256) void k_flux_gs_curved(DevGrid G, EOS eos, Opts o, FluxArgs f, FaceTags only) {
+template <typename EOS, int REC, bool FLAT>
+__global__ __launch_bounds__(256) void k_flux_gs(DevGrid G, EOS eos, Opts o, FluxArgs f, FaceTags only) {
     const WgPos wp = wg_pos(f.tiles * f.ndir);
     int t, d;
     udivmod(wp.tile, f.ndir, t, d);
     const int e = t * (int)blockDim.x + (int)threadIdx.x;
     switch (f.dir0 + d) {
-        case 0: gs_curved_face<EOS, REC, 0>(G, eos, o, f, only.d[0], wp.q, e); break;
-        case 1: gs_curved_face<EOS, REC, 1>(G, eos, o, f, only.d[1], wp.q, e); break;
-        default: gs_curved_face<EOS, REC, 2>(G, eos, o, f, only.d[2], wp.q, e); break;
+        case 0: gs_face<EOS, REC, FLAT, 0>(G, eos, o, f, only.d[0], wp.q, e); break;
+        case 1: gs_face<EOS, REC, FLAT, 1>(G, eos, o, f, only.d[1], wp.q, e); break;
+        default: gs_face<EOS, REC, FLAT, 2>(G, eos, o, f, only.d[2], wp.q, e); break;
     }
 }

@@ -851,7 +851,7 @@ __global__ __launch_bounds__(256) void k_fofc_flag(DevGrid G, EOS eos, Opts o, F
     C2PGuess gs{0, 0, 0, 0, 0, 0};
     C2PRoots rt{-1, -1, -1, -1};
     const double rad = o.ex.by_radius ? cell_radius(o.ex, I, a.blk[q].b, G.n, G.ng, i, j, k) : 1e300;
-    const C2POut out = c2p<FLAT, !FLAT>(cons, pr, m, eos, o.atmo, o.ex, cp, rad, err, true, cnt, gs, rt);
+    const C2POut out = c2p<false, true>(cons, pr, m, eos, o.atmo, o.ex, cp, rad, err, true, cnt, gs, rt);
     if (!(out.floored || dmp)) return;
     for (int t = 0; t < 2; ++t) {
         a.ftag[0][q * nf0 + fidx<0>(G, i + t, j, k)] = 1;
@@ -1150,7 +1150,7 @@ enum { CS_INTERIOR = 0, CS_SHELL = 1, CS_LIST = 2, CS_STAGE = 3 };
 // previous primitives in aux, mu = 1/(h W) of the last c2p of this cell
 // (the previous RK stage, or the caller's data), at most warm_newton
 // evaluations before the plain path.
-// X: see c2p (GS on a curved metric).
+// X: see c2p (GS).
 template <typename EOS, bool FLAT, int GUESS = 0, bool X = false>
 __global__ __launch_bounds__(256, c2p_cells_blocks(FLAT)) void k_c2p_cells(DevGrid G, EOS eos, Opts o, const DevInst* __restrict__ inst,
                                                    const DevBlk* __restrict__ blk, double* st, int snv,
@@ -1268,7 +1268,7 @@ __global__ __launch_bounds__(256, c2p_cells_blocks(FLAT)) void k_c2p_cells(DevGr
         A[BX_ * nc] = Bc0 / m.sqrtg; A[BY_ * nc] = Bc1 / m.sqrtg; A[BZ_ * nc] = Bc2 / m.sqrtg;
         C2PRoots rt{-1, -1, -1, -1};
         const double rad = o.ex.by_radius ? cell_radius(o.ex, inst[blk[q].inst], blk[q].b, G.n, G.ng, i, j, k) : 1e300;
-        out = c2p<FLAT, X>(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad, err, false, cnt, gs, rt);
+        out = c2p<FLAT && !X, X>(cons, pr, m, eos, o.atmo, o.ex, o.cp, rad, err, false, cnt, gs, rt);
         if (out.fatal && o.fatal_count) atomicAdd(o.fatal_count, 1ull);
         A[RHO_ * nc] = pr[RHOL]; A[EPS_ * nc] = pr[EPSL]; A[PRESS_ * nc] = pr[PRESSL];
         A[TEMP_ * nc] = pr[TEMPL]; A[ENTROPY_ * nc] = pr[ENTL]; A[YE_ * nc] = pr[YEL];
@@ -2175,27 +2175,11 @@ static FluxArgs flux_args(grmhd_ctx* c, const double* aux, const double* ms, int
     }
     return f;
 }
-// FOFC correction pass over the tagged faces (only) with the options O (donor
-// cell + LLF).
-template <typename EOS>
-static void launch_flux_tagged(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O,
-                               uint8_t* const* only) {
-    const DevGrid& G = c->G;
-    for (int d = 0; d < 3; ++d) {
-        Scope sc(c, "fofc", s);
-        const int64_t n = (int64_t)(G.n[d] + 1) * G.N[(d + 1) % 3] * G.N[(d + 2) % 3];
-        const int bs = c->tune.flux[d];
-        f.tiles = (int)nblk_bs(n, bs);
-        const dim3 grid((unsigned)(f.tiles * G.nq));
-        if (d == 0) k_flux_tagged<EOS, 0><<<grid, bs, 0, s>>>(G, eos, O, f, only[0]);
-        else if (d == 1) k_flux_tagged<EOS, 1><<<grid, bs, 0, s>>>(G, eos, O, f, only[1]);
-        else k_flux_tagged<EOS, 2><<<grid, bs, 0, s>>>(G, eos, O, f, only[2]);
-    }
-}
-// GS on a curved metric (only: the FOFC pass).
-template <typename EOS, int REC>
-static void launch_flux_gs_curved(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O,
-                                  uint8_t* const* only) {
+// Gardiner-Stone: every face, or (only) the FOFC correction pass over the
+// tagged faces with the options O (donor cell + LLF).
+template <typename EOS, int REC, bool FLAT>
+static void launch_flux_gs(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O,
+                           uint8_t* const* only) {
     const DevGrid& G = c->G;
     static const char* fam[3] = {"flux_x", "flux_y", "flux_z"};
     FaceTags tags{};
@@ -2209,14 +2193,13 @@ static void launch_flux_gs_curved(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipS
             const int64_t n = (int64_t)(G.n[d] + 1 + 2 * O.fofc) * G.N[(d + 1) % 3] * G.N[(d + 2) % 3];
             f.tiles = std::max(f.tiles, (int)nblk_bs(n, bs));
         }
-        k_flux_gs_curved<EOS, REC><<<dim3((unsigned)(f.tiles * f.ndir * G.nq)), bs, 0, s>>>(G, eos, O, f, tags);
+        k_flux_gs<EOS, REC, FLAT><<<dim3((unsigned)(f.tiles * f.ndir * G.nq)), bs, 0, s>>>(G, eos, O, f, tags);
     }
 }
 // The three directions in one launch; one by one where each is timed.
 template <typename EOS, int REC, bool FLAT>
 static void launch_flux(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s, const Opts& O) {
     const DevGrid& G = c->G;
-    const bool uct = c->P.emf != GRMHD_EMF_GS;
     static const char* fam[3] = {"flux_x", "flux_y", "flux_z"};
     f.ring_own = c->ring_copy_now ? c->ring_own : nullptr;
     f.nbr = f.ring_own ? c->ring_nbr : nullptr;
@@ -2227,9 +2210,8 @@ static void launch_flux(grmhd_ctx* c, const EOS& eos, FluxArgs f, hipStream_t s,
         f.tiles = f.tilesr = 0;
         for (int d = f.dir0; d < f.dir0 + f.ndir; ++d) {
             const int t0 = d == 0 ? 1 : 0, t1 = d == 2 ? 1 : 2;
-            const int64_t faces = G.n[d] + 1 + (uct ? 0 : 2 * O.fofc);
-            const int64_t full = uct ? G.n[t0] * G.n[t1] : G.N[t0] * G.N[t1];
-            const int64_t ring = !uct || (f.ring_own && !c->ring_any) ? 0 : 2 * G.ng * (G.n[t0] + G.n[t1]);
+            const int64_t faces = G.n[d] + 1, full = (int64_t)G.n[t0] * G.n[t1];
+            const int64_t ring = f.ring_own && !c->ring_any ? 0 : 2 * G.ng * (G.n[t0] + G.n[t1]);
             f.tiles = std::max(f.tiles, (int)nblk_bs(faces * full, bs));
             f.tilesr = std::max(f.tilesr, (int)nblk_bs(faces * ring, bs));
         }
@@ -2240,17 +2222,15 @@ template <typename EOS, bool FLAT>
 static void flux_rec(grmhd_ctx* c, const EOS& eos, const double* aux, const double* ms, int mnv,
                      const double* const B[3], hipStream_t s, int recon, const Opts& O, uint8_t* const* only) {
     const FluxArgs f = flux_args(c, aux, ms, mnv, B);
-    if constexpr (!FLAT) {
-        if (c->P.emf == GRMHD_EMF_GS) {
-            switch (recon) {
-                case 0: launch_flux_gs_curved<EOS, 0>(c, eos, f, s, O, only); break;
-                case 1: launch_flux_gs_curved<EOS, 1>(c, eos, f, s, O, only); break;
-                case 2: launch_flux_gs_curved<EOS, 2>(c, eos, f, s, O, only); break;
-                default: launch_flux_gs_curved<EOS, 3>(c, eos, f, s, O, only); break;
-            }
-            return;
+    if (c->P.emf == GRMHD_EMF_GS) {
+        switch (recon) {
+            case 0: launch_flux_gs<EOS, 0, FLAT>(c, eos, f, s, O, only); break;
+            case 1: launch_flux_gs<EOS, 1, FLAT>(c, eos, f, s, O, only); break;
+            case 2: launch_flux_gs<EOS, 2, FLAT>(c, eos, f, s, O, only); break;
+            default: launch_flux_gs<EOS, 3, FLAT>(c, eos, f, s, O, only); break;
         }
-    } else if (only) { launch_flux_tagged<EOS>(c, eos, f, s, O, only); return; }
+        return;
+    }
     switch (recon) {
         case 0: launch_flux<EOS, 0, FLAT>(c, eos, f, s, O); break;
         case 1: launch_flux<EOS, 1, FLAT>(c, eos, f, s, O); break;
@@ -2439,11 +2419,13 @@ static void launch_c2p_cells(grmhd_ctx* c, double* st, int snv, const double* ms
             if (c->P.eos_kind == GRMHD_EOS_IDEAL_GAS) { if (flat) C2PL(c->ideal, true, 1); else C2PL(c->ideal, false, 1); }
             else { if (flat) C2PL(c->hybrid, true, 1); else C2PL(c->hybrid, false, 1); }
         } else {
-            const bool x = !flat && c->P.emf == GRMHD_EMF_GS;
+            const bool x = c->P.emf == GRMHD_EMF_GS;
             if (c->P.eos_kind == GRMHD_EOS_IDEAL_GAS) {
-                if (flat) C2PL(c->ideal, true, 0); else if (x) C2PL(c->ideal, false, 0, true); else C2PL(c->ideal, false, 0);
+                if (flat) { if (x) C2PL(c->ideal, true, 0, true); else C2PL(c->ideal, true, 0); }
+                else { if (x) C2PL(c->ideal, false, 0, true); else C2PL(c->ideal, false, 0); }
             } else {
-                if (flat) C2PL(c->hybrid, true, 0); else if (x) C2PL(c->hybrid, false, 0, true); else C2PL(c->hybrid, false, 0);
+                if (flat) { if (x) C2PL(c->hybrid, true, 0, true); else C2PL(c->hybrid, true, 0); }
+                else { if (x) C2PL(c->hybrid, false, 0, true); else C2PL(c->hybrid, false, 0); }
             }
         }
 #undef C2PL

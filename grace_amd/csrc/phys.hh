@@ -203,7 +203,7 @@ struct EosIdeal {
         a2 = gamma * p;
         return p;
     }
-    // the face states' EOS with sound speed, for GS EMFs on a curved metric
+    // the face states' EOS with sound speed, for GS EMFs
     GHD double press_from_temp(double& eps, double& cs2, double& temp, double rho, unsigned& e) const {
         limit_temp(temp, e);
         eps = temp / gm1;
@@ -345,7 +345,7 @@ struct EosHybrid {
         a2 = a2_of(rho_f, rho, eth, eps, p);
         return p;
     }
-    // the face states' EOS with sound speed, for GS EMFs on a curved metric
+    // the face states' EOS with sound speed, for GS EMFs
     GHD double press_from_temp(double& eps, double& cs2, double& temp, double rho, unsigned& e) const {
         chk_rho(rho, e); chk_temp(temp, e);
         double ec; double pc = pcold(ec, rho);
@@ -1048,16 +1048,16 @@ struct C2POut { bool floored, fatal; };
 
 // conservs_to_prims (c2p.cpp:188-414).  cons densitised in, re-densitised out.
 // X: every quotient and root an IEEE operation, the master functions in the
-// general form.  For GS EMFs on a curved metric with the plain solve: they
-// choose a side by the sign of the mass flux, which in a stationary flow (a
-// torus: no poloidal velocity) is rounding at many faces, and one ulp in the
-// primitives was seen to move single faces of the field by 5e-6 of its largest
-// value in one step.  (The Newton finish of the learned and the warm-started
-// guess has another root in the last digits anyway and takes the other form:
-// over tori on grids and forests the field stays within 7e-16 of the one with
-// divisions, the conserved within 6e-15.)  The other form is as accurate
-// (against 128-bit solves of 720 000 states 0.998 +- 0.012 of the error with
-// divisions) and takes 0.7 of the time.
+// general form.  For GS EMFs with the plain solve: they choose a side by the
+// sign of the mass flux, which in a stationary flow (a torus: no poloidal
+// velocity) is rounding at many faces, and one ulp in the primitives was seen
+// to move single faces of the field by 5e-6 of its largest value in one step.
+// (The Newton finish of the learned and the warm-started guess has another
+// root in the last digits anyway and takes the other form: over tori on grids
+// and forests the field stays within 7e-16 of the one with divisions, the
+// conserved within 6e-15.)  The other form is as accurate (against 128-bit
+// solves of 720 000 states 0.998 +- 0.012 of the error with divisions) and
+// takes 0.7 of the time.
 template <bool FL, bool X, typename EOS>
 GHD C2POut c2p(double cons[NCONS], double pr[NPRIM], const Met& m, const EOS& eos, const Atmo& at,
                const ExcPar& ex, const C2PPar& cp, double radius, uint64_t& err, bool dry_run, C2PCount& cnt,
@@ -1251,8 +1251,8 @@ GHD double mc2(double sL, double sR) {
 GHD double minmod(double sL, double sR) {
     return 0.5 * (copysign(1.0, sL) + copysign(1.0, sR)) * fmin(fabs(sL), fabs(sR));
 }
-// The candidates' form of WENO-Z, kept for GS EMFs on a curved metric (see
-// c2p): the same values up to rounding.
+// The candidates' form of WENO-Z, kept for GS EMFs (see gs_face): the same
+// values up to rounding.
 // Per side, the three ratios
 // t5/(b_k+eps) come from one reciprocal of d0 d1 d2 (d_k >= 1e-42, so the
 // product cannot underflow), and the two sides of a face share their
